@@ -264,24 +264,37 @@ inline bool make_geometry(int dtype, size_t n, size_t k, Geometry &g) {
 
 
 /**
- *  Load one 16-byte chunk of which only the first `valid` bytes exist (valid may be <= 0 or >= 16),
- *  with loads no wider than the pointer's known alignment `avec`. Missing bytes read as zero; `xr`
- *  (0 or 0x80808080) is applied to existing bytes only, so zero padding stays zero for u8.
+ *  Load one chunk of BYTES (16, 8 or 2) bytes at any address, of which only the first `valid` bytes exist (valid may be
+ *  <= 0 or >= BYTES). Missing bytes read as zero; `xr` (0 or 0x80808080) is applied to existing bytes only, so zero
+ *  padding stays zero for u8. The aligned dwords that hold the bytes are loaded (each holds one that exists at least, so
+ *  nothing outside the matrix's own dwords is touched) and shifted into place, one v_alignbyte_b32 per dword: byte by byte,
+ *  a chunk at an odd address took 16 loads.
  */
-__device__ __forceinline__ v4i load_chunk_guarded(uint8_t const *p, int valid, int avec, uint32_t xr) {
-    v4i out;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        int const rem = valid - 4 * w;
-        uint32_t x = 0;
-        if (rem >= 4 && avec >= 4) { x = *(uint32_t const *)(p + 4 * w) ^ xr; }
-        else if (rem > 0) {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                if (b < rem) x |= (uint32_t)(uint8_t)(p[4 * w + b] ^ (uint8_t)xr) << (8 * b);
-        }
-        out[w] = (int)x;
+template <int BYTES>
+__device__ __forceinline__ v4i load_chunk_guarded(uint8_t const *p, int valid, uint32_t xr) {
+    typedef int v4i_of_dwords __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int kWords = BYTES / 4 > 0 ? BYTES / 4 : 1;
+    v4i out = {0, 0, 0, 0};
+    if (valid <= 0) return out;
+    uint32_t const shift = (uint32_t)(uintptr_t)p & 3u;
+    uint32_t const *dwords = (uint32_t const *)(p - shift);
+    uint32_t word[kWords + 1];
+    if (BYTES == 16 && valid >= BYTES) {
+        v4i const wide = *(v4i_of_dwords const *)dwords;
+        word[0] = (uint32_t)wide[0], word[1] = (uint32_t)wide[1], word[2] = (uint32_t)wide[2], word[3] = (uint32_t)wide[3];
+        word[kWords] = shift ? dwords[4] : 0u;
     }
+    else {
+#pragma unroll
+        for (int w = 0; w <= kWords; ++w) word[w] = 4 * w < (int)shift + (valid < BYTES ? valid : BYTES) ? dwords[w] : 0u;
+    }
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) {
+        int const left = valid - 4 * w, bytes = left < 0 ? 0 : (left > 4 ? 4 : left);
+        uint32_t const keep = bytes == 4 ? 0xFFFFFFFFu : ((1u << (8 * bytes)) - 1u);
+        out[w] = (int)((__builtin_amdgcn_alignbyte(word[w + 1], word[w], shift) ^ xr) & keep);
+    }
+    if (BYTES < 4) out[0] &= (1 << (8 * (BYTES & 3))) - 1;
     return out;
 }
 
@@ -506,7 +519,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
                 v = __builtin_nontemporal_load((v4i const *)src); // (read once)
                 v[0] ^= (int)xr, v[1] ^= (int)xr, v[2] ^= (int)xr, v[3] ^= (int)xr;
             }
-            else { v = load_chunk_guarded(src, valid, avec, xr); }
+            else { v = load_chunk_guarded<kSrcChunk>(src, valid, xr); }
             if constexpr (WIDEN == 3) {
 #pragma unroll
                 for (int w = 0; w < 4; ++w) v[w] = (int)widen_e2m3x4((uint32_t)v[w]);
@@ -1037,8 +1050,8 @@ __global__ __launch_bounds__(256) void triangle_tiles_kernel(TriangleGrids grids
  *      before the last k-step: one barrier; the first fragments of stage s+1 are read under its MFMAs
  *  The packed image pads K with zeros to an even number of stages; on the A side, the bytes a stage reads
  *  past the end of a row (the next row's, or nothing past the end of the matrix) are masked to zero on their
- *  way into LDS, so ragged depths run through the same loop. Only A that is not even dword-aligned takes a
- *  plain guarded loop instead.
+ *  way into LDS, so ragged depths run through the same loop, and so do rows at any byte address (SHIFTED, below).
+ *  Only such rows of fewer than four stages take a plain guarded loop instead.
  *
  *  A is the MFMA's first operand, so a lane ends up with one column and 16 rows of each 32x32 block and the
  *  epilogue stores dwords that are contiguous across lanes: 128 bytes per row per instruction, any C
@@ -1073,8 +1086,17 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  loads are issued three stages ahead, and one trip of the loop is four stages. For types that reach LDS as they are
  *  in memory, depths of a whole number of trips, the pipelined kernel across tiles, dot products only (the host
  *  checks).
+ *
+ *  SHIFTED: A starts on any byte or its rows are not a multiple of four bytes apart (odd depths). Loads of more than a
+ *  dword need dword addresses, so a thread loads the aligned dwords that hold its chunk, one more than the chunk has, and
+ *  shifts them into place where they are staged, a v_alignbyte_b32 per dword. How far is the same for every chunk that a
+ *  thread stages: its rows are 32 apart, and 32 strides are a multiple of four. Everything behind that (masks, widening,
+ *  sums) sees chunks as if A were aligned. Measured against the guarded loop that such rows used to take (whole calls):
+ *  i8 3 x 162,699 x 4327 1019 -> 155 us, u8 symmetric 6391 x 7163 1625 -> 252 us, f16 symmetric angular 2947 x 3033
+ *  674 -> 113 us; with B packed in the call as well, whose odd rows were read byte by byte: bf16 959 x 74,207 x 4307
+ *  6505 -> 1372 us, i8 45 x 610,671 x 391 433 -> 230 us.
  */
-template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false>
+template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false>
 __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChunked ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
     constexpr int BM = TM * 32;
@@ -1082,6 +1104,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     constexpr int kStageLds = BM * kStageBytes;
     constexpr int kLoads = BM * kStageChunks / NT; // 16-byte LDS chunks per thread per stage = TM
     constexpr int kSrcStage = kStageChunks * T::kSrcChunk; // source bytes of A per row per stage
+    static_assert(!SHIFTED || (ACROSS && !WHOLE && !DIRECT), "shifted loads: only the staged loop has them");
     static_assert(!DIRECT || (ACROSS && !NORMS && !T::kUnsigned && !T::kPrewiden && T::kSrcChunk == 16 && T::kImageChunk == 16),
                   "straight into LDS: only what needs nothing done to it on the way");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[DIRECT ? 16 : 2 * kStageLds];
@@ -1114,7 +1137,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     // Stages the pipelined loop takes: all of them when A is at least dword-aligned, which is all that
     // multi-dword global loads need. (readfirstlane: the value is uniform, and it must stay in a scalar register
     // because the stage offsets of the buffer loads derive from it.)
-    uint32_t const fast = __builtin_amdgcn_readfirstlane(g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) ? stages : 0);
+    uint32_t const fast = __builtin_amdgcn_readfirstlane(SHIFTED || g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) ? stages : 0);
     uint32_t const xr = T::kUnsigned ? 0x80808080u : 0u;
     uint32_t const a_pos = tid & 7;
     // A fragment reads: lane l takes row l % 32 of each 32-row block and chunk 2q + l / 32.
@@ -1128,12 +1151,15 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     // A staging: thread t fetches chunk t % 8 of rows i*32 + t/8 of a tile and stores it at its swizzled
     // position. The offsets are the same for every tile: rows past the end of A are cut off by the size of
     // the tile's buffer descriptor (such loads return zeros, and their outputs are never stored).
+    uint32_t const a_skew = SHIFTED ? (uint32_t)(uintptr_t)g.a & 3u : 0u; // what the descriptors' bases are rounded down by
+    uint32_t const a_shift = SHIFTED ? (a_skew + (tid >> 3) * (uint32_t)g.a_stride + a_pos * T::kSrcChunk) & 3u : 0u;
     uint32_t a_off[kLoads]; // byte offset of the thread's source chunk from the tile's first row
     uint32_t a_lds[kLoads]; // where it goes in an LDS stage
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
         uint32_t const r = i * 32 + (tid >> 3);
         a_off[i] = r * (uint32_t)g.a_stride + a_pos * T::kSrcChunk;
+        if (SHIFTED) a_off[i] = (a_off[i] + a_skew) & ~3u;
         a_lds[i] = r * kStageBytes + ((a_pos ^ ((r >> 1) & 7)) << 4);
     }
     uint32_t const b_lane = lane * T::kImageChunk;
@@ -1157,10 +1183,11 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
         view.row0 = tile_m * BM;
         view.col0 = tile_n * (128 * TN) + wave * (32 * TN);
         uint32_t const rows_here = g.m - view.row0 < (uint32_t)BM ? g.m - view.row0 : (uint32_t)BM;
-        view.a = g.a + (uint64_t)view.row0 * g.a_stride;
+        view.a = g.a + (uint64_t)view.row0 * g.a_stride - a_skew; // (row0 is a multiple of 32: the skew is every tile's)
         // (whole aligned loads: an aligned A never ends in the middle of one that could fault)
-        constexpr uint32_t kLoadAlign = T::kSrcChunk < 4 ? T::kSrcChunk : 4; // (2-byte loads for the 1-bit type)
-        view.a_bytes = (rows_here - 1) * (uint32_t)g.a_stride + (((uint32_t)g.k_src_bytes + kLoadAlign - 1) & ~(kLoadAlign - 1));
+        constexpr uint32_t kLoadAlign = T::kSrcChunk < 4 && !SHIFTED ? T::kSrcChunk : 4; // (2-byte loads for the 1-bit type)
+        view.a_bytes = SHIFTED ? (a_skew + (rows_here - 1) * (uint32_t)g.a_stride + (uint32_t)g.k_src_bytes + 3u) & ~3u
+                               : (rows_here - 1) * (uint32_t)g.a_stride + (((uint32_t)g.k_src_bytes + kLoadAlign - 1) & ~(kLoadAlign - 1));
         uint32_t const tile_bytes = g.k_chunks * kImageTileChunk;
         uint32_t const first = view.col0 / 32 < g.n_tiles ? view.col0 / 32 : g.n_tiles - 1;
         view.b = data + (uint64_t)first * tile_bytes;
@@ -1202,6 +1229,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
         __hip_atomic_fetch_add(&norm_part[set + i * NT + tid], value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     v4i a_reg[2][kLoads];
+    uint32_t a_more[SHIFTED ? 2 : 1][SHIFTED ? kLoads : 1]; // shifted 16-byte chunks: the fifth dword
     v4i b_reg[2][TN][4];
     v4i af[2][TM];
 
@@ -1241,6 +1269,17 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
             v4i v = {0, 0, 0, 0};
             if (T::kSrcChunk == 16) {
                 v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, a_off[i], stage_offset, 0));
+                if constexpr (SHIFTED) a_more[slot][i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, a_off[i] + 16, stage_offset, 0);
+            }
+            else if (SHIFTED && T::kSrcChunk == 8) {
+                typedef unsigned v3u __attribute__((ext_vector_type(3)));
+                v3u const narrow = __builtin_amdgcn_raw_buffer_load_b96(rsrc, a_off[i], stage_offset, 0);
+                v[0] = (int)narrow[0], v[1] = (int)narrow[1], v[2] = (int)narrow[2];
+            }
+            else if (SHIFTED) {
+                typedef unsigned v2u __attribute__((ext_vector_type(2)));
+                v2u const narrow = __builtin_amdgcn_raw_buffer_load_b64(rsrc, a_off[i], stage_offset, 0);
+                v[0] = (int)narrow[0], v[1] = (int)narrow[1];
             }
             else if (T::kSrcChunk == 2) { v[0] = (int)(uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, a_off[i], stage_offset, 0); }
             else {
@@ -1269,6 +1308,18 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
             keep[w] = bytes == 4 ? 0xFFFFFFFFu : ((1u << (8 * bytes)) - 1u);
         }
     };
+    // What a thread loaded for its chunk -> the chunk (SHIFTED; as it is otherwise).
+    auto loaded_chunk = [&](auto slot_tag, int i) {
+        constexpr int slot = decltype(slot_tag)::value;
+        v4i v = a_reg[slot][i];
+        if constexpr (SHIFTED) {
+            uint32_t const last = T::kSrcChunk == 16 ? a_more[slot][i] : 0u;
+#pragma unroll
+            for (int w = 0; w < (T::kSrcChunk + 3) / 4; ++w)
+                v[w] = (int)__builtin_amdgcn_alignbyte(w < 3 ? (uint32_t)v[w < 3 ? w + 1 : 3] : last, (uint32_t)v[w], a_shift);
+        }
+        return v;
+    };
     // Half of the staged chunks of stage `s`, masked and widened where they are (types with kPrewiden): what
     // store_a would do right in front of its LDS writes, done a k-step or two earlier among that k-step's MFMAs.
     auto prewiden = [&](auto slot_tag, uint32_t s, auto half_tag) {
@@ -1279,7 +1330,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             if (i * 2 / kLoads != half_of) continue;
-            v4i v = a_reg[slot][i];
+            v4i v = loaded_chunk(slot_tag, i);
             if (kMaskTail) {
 #pragma unroll
                 for (int w = 0; w < kSrcWords; ++w) v[w] &= (int)keep[w];
@@ -1296,7 +1347,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
         if (!widened && kMaskTail) masks_of(s, keep);
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            v4i v = a_reg[slot][i];
+            v4i v = widened ? a_reg[slot][i] : loaded_chunk(slot_tag, i);
             if (!widened && kMaskTail) {
 #pragma unroll
                 for (int w = 0; w < kSrcWords; ++w) v[w] &= (int)keep[w];
@@ -1369,7 +1420,8 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     // sums; the distance kinds: the squares) and LDS adds (one per sum kept). The k-step that stages asks for them
     // behind its MFMAs, a chunk's worth each; left alone they all land between the last MFMA and the barrier.
     constexpr bool kIntegerSums = __is_same(typename T::acc_t, v16i);
-    constexpr int kStageVector = (T::kUnsigned ? 8 : 0) + (NORMS ? (kIntegerSums ? 5 : 28) : 0);
+    constexpr int kStageVector = (T::kUnsigned ? 8 : 0) + (NORMS ? (kIntegerSums ? 5 : 28) : 0) + (SHIFTED && !T::kPrewiden ? (T::kSrcChunk + 3) / 4 : 0);
+    constexpr int kStageLoads = (kLoads >= 4 ? kLoads / 4 : 1) * (SHIFTED && T::kSrcChunk == 16 ? 2 : 1); // of A, per k-step
     constexpr int kStageDs = 1 + (T::kUnsigned ? 1 : 0) + (NORMS ? 1 : 0);
     // Scheduling hints for one k-step. Masks: 0x008 MFMA, 0x020 VMEM read, 0x100 DS read, 0x200 DS write.
     // Fragment reads go one-to-one with the first TM MFMAs; the global loads of the k-step (TN of B
@@ -1377,7 +1429,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     auto schedule_k_step = [&](auto writes_tag, auto vector_tag) {
         constexpr bool writes = decltype(writes_tag)::value != 0;
         constexpr int vector = decltype(vector_tag)::value; // vector operations to put behind every MFMA (0x002)
-        constexpr int loads = TN + (kLoads >= 4 ? kLoads / 4 : 1);
+        constexpr int loads = TN + kStageLoads;
         constexpr int rest = TM * (TN - 1);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -1418,7 +1470,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
     // The first k-step of a tile of the chunked types: in front of every MFMA the 16 zeros of its block's total;
     // fragment reads and loads as in any k-step without LDS writes.
     auto schedule_fresh_k_step = [&]() {
-        constexpr int loads = TN + (kLoads >= 4 ? kLoads / 4 : 1);
+        constexpr int loads = TN + kStageLoads;
 #pragma unroll
         for (int i = 0; i < TM * TN; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
@@ -1699,7 +1751,7 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
                     int const valid = (int)(left > T::kSrcChunk ? T::kSrcChunk : (left < 0 ? 0 : left));
 #pragma unroll
                     for (int i = 0; i < kLoads; ++i) {
-                        v4i v = load_chunk_guarded(a_tile + (uint64_t)s * kSrcStage + a_slow[i], valid, g.avec, 0u);
+                        v4i v = load_chunk_guarded<T::kSrcChunk>(a_tile + (uint64_t)s * kSrcStage + a_slow[i], valid, 0u);
                         v4i const raw = v;
                         if (T::kUnsigned) {
                             add_row_sum(i, sum_bytes_u8(v), sums_here);
@@ -1914,6 +1966,12 @@ inline size_t triangle_scratch_bytes(uint64_t m, uint64_t n, uint32_t bm, uint32
     return (size_t)(((bands + 1 + 1) & ~1ull) * 4 + live_tiles(m, n, bm, bn, shift) * 8);
 }
 
+/** Rows of A that the pipelined loop reads by shifted loads (see dots_packed_kernel). */
+template <class T>
+inline bool needs_shift(GemmArgs const &g) {
+    return g.avec < (T::kSrcChunk < 4 ? T::kSrcChunk : 4) && g.k_chunks / kStageChunks >= 4;
+}
+
 /** `slots_only`: do not launch, only report how many workgroups of the kernel this call would use are resident on
  *  the device at once. */
 template <class T, int TM, int TN>
@@ -1933,19 +1991,25 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     }
     g.tile_count = (uint32_t)tiles;
     // The tile's A offsets are 32-bit: (rows of a tile) * stride must stay below 4 GiB.
-    if ((uint64_t)BM * g.a_stride > 0xFFFFFFFFull) return hipErrorInvalidValue;
+    if ((uint64_t)BM * g.a_stride + 8 > 0xFFFFFFFFull) return hipErrorInvalidValue;
     // So are the per-lane C offsets: 4 rows plus the tile's width.
     if (4 * (uint64_t)g.c_stride + BN * 4 > 0xFFFFFFFFull) return hipErrorInvalidValue;
     // The offsets into a wavefront's B tiles are 32-bit as well.
     if ((uint64_t)(TN + 1) * g.k_chunks * kTileRows * T::kImageChunk > 0xFFFFFFFFull) return hipErrorInvalidValue;
     // The pipeline runs across tile boundaries when the pipelined loop takes the stages of a tile (A readable
-    // with dword loads) and there are enough of them to prefetch three ahead.
+    // with dword loads, or shifted into place behind them: bf16 959 x 74,207 x 4307 took 5.6 ms in the guarded loop) and
+    // there are enough of them to prefetch three ahead.
     uint32_t const stages = g.k_chunks / kStageChunks;
-    bool const across = g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) && stages >= 4;
+    bool const shifted = needs_shift<T>(g);
+    bool const across = !shifted && stages >= 4;
     bool const norms = g.metric != 0;
     // depths that fill an even number of stages exactly: the pipelined kernel without the tail masks
     bool const whole = across && g.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
     void (*kernel)(GemmArgs) = across ? dots_packed_kernel<T, TM, TN, true, false> : dots_packed_kernel<T, TM, TN, false, false>;
+    if constexpr (TM * TN < 16) {
+        if (shifted) kernel = dots_packed_kernel<T, TM, TN, true, false, false, false, true>;
+    }
+    else if (shifted) return hipErrorInvalidValue; // (launch_typed does not ask for it)
     if constexpr (tail_matters_for<T, false>()) {
         if (whole) kernel = dots_packed_kernel<T, TM, TN, true, false, true>;
     }
@@ -1963,13 +2027,16 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     }
     if constexpr (T::kDistances) {
         if (norms) kernel = across ? dots_packed_kernel<T, TM, TN, true, true> : dots_packed_kernel<T, TM, TN, false, true>;
+        if constexpr (TM * TN < 16) {
+            if (norms && shifted) kernel = dots_packed_kernel<T, TM, TN, true, true, false, false, true>;
+        }
         if (norms && whole) kernel = dots_packed_kernel<T, TM, TN, true, true, true>;
     }
     else if (norms) return hipErrorInvalidValue;
     // Persistent grid: as many workgroups as fit on the device at once (queried once per kernel; threads that
     // ask at the same time store the same number).
-    static std::atomic<int> resident_of[9];
-    std::atomic<int> &slot = resident_of[direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)];
+    static std::atomic<int> resident_of[11];
+    std::atomic<int> &slot = resident_of[shifted ? (norms ? 10 : 9) : direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)];
     int resident = slot.load(std::memory_order_relaxed);
     if (!resident) {
         int per_cu = 0;
@@ -2050,7 +2117,9 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             if (!T::kUnsigned && args.m <= 2048 && best < 2 && tiles_of(args, 2) >= 256) best = 2;
             else if (best < 3 && tiles_of(args, 3) >= 256) best = 3;
         }
-        if (T::kChunked && best == 1) best = 2; // two accumulator sets do not fit the 256 x 256 tile
+        // Two accumulator sets do not fit the 256 x 256 tile, and neither do the fifth dwords of shifted loads (99 registers
+        // of the i8 kernel spill).
+        if ((T::kChunked || needs_shift<T>(args)) && best == 1) best = 2;
         // Shallow products into rows of C that do not start on 128-byte lines: the stores go through the L2 (see the
         // epilogue) and take long enough to matter, and three small workgroups per compute unit overlap one's stores
         // with the others' loops, which one large tile cannot (measured, 64 x 128 against the tile chosen above: i8
@@ -2063,11 +2132,11 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // e2m3 pays 13 vector operations for every dword of A it stages: a 128 x 512 tile (every wavefront 128 x 128)
         // stages half as much A per MFMA as 256 x 256 (8192^3: 0.51 against 0.59 ms; for i8 itself the two are equal)
         // (not the f16 route of very deep rows: its two accumulator sets do not fit that tile)
-        if (T::kDtype == kE2M3 && !T::kChunked && !triangle && args.metric == 0 && first == 1 && tiles_of(args, 5) >= 256) best = 5;
+        if (T::kDtype == kE2M3 && !T::kChunked && !triangle && args.metric == 0 && first == 1 && !needs_shift<T>(args) && tiles_of(args, 5) >= 256) best = 5;
         return best;
     };
     if (chosen_here) config = choose(g, 1);
-    if (T::kChunked && config == 1) config = 2;
+    if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
     // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
     auto grid_of = [](GemmArgs const &args, int c, TriangleScratch const &scratch) {
         uint32_t const bm = kConfigs[c].tm * 32, bn = kConfigs[c].tn * 128;
