@@ -618,7 +618,7 @@ static bool symmetric_window(int dtype, size_t n, size_t k, size_t row_start, si
     if (!make_geometry(dtype, w.columns, k, geo)) return false;
     w.image_bytes = (size_t)((geo.total_bytes + 255) & ~255ull);
     uint32_t const shift = (uint32_t)(row_start - w.col_begin);
-    for (int c = 1; c < kConfigCount; ++c) {
+    for (int c = 1; c < kTriangleConfigs; ++c) {
         size_t const bytes = triangle_scratch_bytes(w.row_end - row_start, w.columns, kConfigs[c].tm * 32,
                                                     kConfigs[c].tn * 128, shift);
         if (bytes > w.scratch_bytes) w.scratch_bytes = bytes;

@@ -1097,7 +1097,7 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  6505 -> 1372 us, i8 45 x 610,671 x 391 433 -> 230 us.
  */
 template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false>
-__global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChunked ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChunked ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
     constexpr int BM = TM * 32;
     constexpr int NT = 256;
@@ -1945,9 +1945,10 @@ __global__ __launch_bounds__(256, (TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChun
 struct TileConfig {
     int tm, tn;
 };
-// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only).
-constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}};
+// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only; 6: full grids only).
+constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}, {1, 1}};
 constexpr int kConfigCount = sizeof(kConfigs) / sizeof(kConfigs[0]);
+constexpr int kTriangleConfigs = 6; // the shapes below this index serve triangular grids
 
 
 /** Tiles of a bm x bn grid over m x n outputs with something on or right of the diagonal col = row + shift. */
@@ -2077,6 +2078,9 @@ hipError_t launch_config(GemmArgs &g, hipStream_t stream, TriangleScratch const 
     case 5:
         if constexpr (T::kDtype != kE2M3) return hipErrorInvalidValue;
         else return launch_one<T, 4, 4>(g, stream, triangle, slots_only);
+    case 6:
+        if (triangle) return hipErrorInvalidValue; // (launch_typed does not ask for it)
+        return launch_one<T, 1, 1>(g, stream, nullptr, slots_only);
     default: return launch_one<T, 2, 1>(g, stream, triangle, slots_only);
     }
 }
@@ -2093,12 +2097,27 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
     auto choose = [&](GemmArgs const &args, int first) {
+        uint32_t const depth_stages = args.k_chunks / kStageChunks;
+        // Few rows: a tile of more rows than A has multiplies what is not there (i8 1 x 1,048,576 x 768 through the 256-row
+        // tile was bound by its matrix instructions), and one that is not full stores through the masked copy of the
+        // epilogue. Measured, whole calls, the tile taken before against this one (us): i8 x 1,048,576 x 768 with 1 row 365
+        // against 156 (32 x 128; 162 with 64 x 128), 32 rows 363 against 199, 64 rows 370 against 223 (64 x 128; 244 with
+        // 32 x 128), 96 rows 391 against 261 (128 x 128); angular, 96 rows 351 against 275; bf16 1 row 361 against 288, 64
+        // rows 399 against 376, 96 rows 442 against 426.
+        if (!triangle && args.m <= 32) return 6;
+        if (!triangle && args.m <= 64) first = 4;
+        else if (!triangle && args.m < 128 && first < 3) first = 3;
         int best = 4;
         for (int c = first; c <= 4; ++c)
             if (tiles_of(args, c) >= 256) {
                 best = c;
                 break;
             }
+        // Fewer tiles of 64 x 128 than CUs: 32 x 128 spreads the epilogues over more of them, which is most of a shallow
+        // product's time (192 x 10,000 x 256, us: i8 angular 25.6 against 23.6, bf16 24.2 against 23.2, bf16 angular 28.1
+        // against 25.2); a deep one gains as long as the smaller tiles fit one round (bf16 1024^3 26.3 against 24.8, angular
+        // 29.3 against 26.1, but 64 x 30,000 x 4096 54 against 62).
+        if (!triangle && tiles_of(args, 4) < 256 && (depth_stages <= 8 || tiles_of(args, 6) <= 256)) return 6;
         // Distances over a shallow depth are bound by the epilogue (a finaliser and a store per output): two
         // workgroups per CU of 128 x 128 tiles overlap it with the other's loop better than one large tile does
         // (measured on 1024 x 1,048,576 x 768: 2.17 against 2.33 ms angular, 1.98 against 2.07 ms euclidean).
@@ -2109,7 +2128,6 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // 1024 128 x 128 (1.42 against 1.55; 0.114 against 0.120); u8 128 x 128 (2.29 against 2.54 and 2.91); bf16
         // angular 1024 x 524,288 x 768 64 x 128 1.58 against 1.72 (128 x 128) and 2.18 (128 x 256), 8192 x 8192 x 1024
         // 0.198 against 0.267 and 0.319, and still 3.39 against 3.77 at depth 2048; f16 and e4m3 likewise.
-        uint32_t const depth_stages = args.k_chunks / kStageChunks;
         if (args.metric != 0 && T::kChunked) {
             if (depth_stages <= 32 && tiles_of(args, 4) >= 256) best = 4;
         }
@@ -2137,6 +2155,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     };
     if (chosen_here) config = choose(g, 1);
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
+    if (triangle && config >= kTriangleConfigs) config = 4;
     // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
     auto grid_of = [](GemmArgs const &args, int c, TriangleScratch const &scratch) {
         uint32_t const bm = kConfigs[c].tm * 32, bn = kConfigs[c].tn * 128;
