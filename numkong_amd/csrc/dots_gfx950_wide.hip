@@ -12,8 +12,8 @@
  *    f64  compensated ("dot2"): two lanes by k mod 2, each a running sum plus the accumulated rounding errors of its
  *         products (by FMA) and of its additions (TwoSum); the four numbers are folded by one more chain of TwoSums.
  *         No matrix form exists for that, so it is a register-tiled kernel on the vector units, which on MI355X run
- *         f64 at the rate of the f64 matrix instructions (78.6 TFLOP/s either way): 256 threads compute a 64 x 64
- *         tile of C, 4 x 4 outputs each, A through LDS transposed (k-major).
+ *         f64 at the rate of the f64 matrix instructions (78.6 TFLOP/s either way): 256 threads compute a tile of 64
+ *         columns of C and 64, 16 or 4 rows (4 x 4, 1 x 4 or 1 x 1 outputs each), A through LDS transposed (k-major).
  *
  *  Either way every output keeps the reference's own accumulators and takes its terms in the reference's own order
  *  along k, so the results are those of its serial kernels bit for bit. B comes from an image that is already k-major
@@ -30,7 +30,7 @@
 
 namespace {
 
-constexpr int kWideTile = 64;  // rows and columns of C per workgroup
+constexpr int kWideTile = 64;  // columns of C per workgroup (and rows at most of the f64 kernel)
 constexpr int kWideDepth = 8;  // k per step through LDS
 
 struct WideArgs {
@@ -166,14 +166,19 @@ __device__ __forceinline__ double fold_compensated(double const (&lane)[4]) {
     return running + error;
 }
 
-template <bool NORMS>
+template <bool NORMS, int ROWS>
 __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
-    __shared__ double a_lds[2][kWideDepth][kWideTile + 1];
+    constexpr int kCols = ROWS >= 16 ? 4 : 1;          // outputs of a thread along a row of C
+    constexpr int kAcross = kWideTile / kCols;         // threads along a row
+    constexpr int kDown = 256 / kAcross;               // and along a column
+    constexpr int kRows = ROWS / kDown;                // outputs of a thread along a column
+    static_assert(kRows * kDown == ROWS, "the threads cover the tile");
+    __shared__ double a_lds[2][kWideDepth][ROWS + 1];
     __shared__ double b_lds[2][kWideDepth][kWideTile];
-    __shared__ double row_parts[NORMS ? kWideTile : 1][4][2]; // distances: four partial sums of squares per row of A
-    __shared__ double row_norms[NORMS ? kWideTile : 1];
-    uint32_t const tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    uint32_t const row0 = blockIdx.y * kWideTile, col0 = blockIdx.x * kWideTile;
+    __shared__ double row_parts[NORMS ? ROWS : 1][4][2]; // distances: four partial sums of squares per row of A
+    __shared__ double row_norms[NORMS ? ROWS : 1];
+    uint32_t const tid = threadIdx.x, tx = tid % kAcross, ty = tid / kAcross;
+    uint32_t const row0 = blockIdx.y * ROWS, col0 = blockIdx.x * kWideTile;
     // symmetric form: a tile wholly left of the diagonal has nothing to store
     if (((row0 + g.tri_shift) & g.tri_mask) > col0 + (kWideTile - 1)) return;
     typedef __attribute__((address_space(1))) double global_f64_t;
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
     PackedHeader const *header = (PackedHeader const *)((uint8_t const *)g.b - sizeof(PackedHeader));
     if (!(header->magic == kMagic && header->version == kVersion && header->dtype == (uint32_t)g.dtype && header->n == g.n &&
           header->k == g.k)) {
-        for (uint32_t at = tid; at < kWideTile * kWideTile; at += 256) {
+        for (uint32_t at = tid; at < ROWS * kWideTile; at += 256) {
             uint32_t const row = row0 + at / kWideTile, col = col0 + at % kWideTile;
             if (row < g.m && col < g.n && ((row + g.tri_shift) & g.tri_mask) <= col)
                 *(global_u64_t *)(g.c + (uint64_t)row * g.c_stride + (uint64_t)col * 8) = ~0ull;
@@ -192,20 +197,20 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
     }
 
     // accumulators: per output, four numbers: (s0, c0, s1, c1)
-    double acc[4][4][4];
+    double acc[kRows][kCols][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kRows; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < kCols; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[i][j][v] = 0;
 
-    // staging: A: thread t brings 2 consecutive k of row t / 4 ... (64 rows x 8 k = 512 values, 2 per thread);
+    // staging: A: thread t brings 2 consecutive k of row t / 4, as far as the tile has rows;
     //          B: thread t brings 2 consecutive columns of depth t / 32 (8 x 64 = 512 values, 2 per thread)
     uint32_t const a_row = tid >> 2, a_k = (tid & 3) * 2;
     uint32_t const b_k = tid >> 5, b_col = (tid & 31) * 2;
-    uint8_t const *a_source = g.a + (uint64_t)(row0 + a_row < g.m ? row0 + a_row : 0) * g.a_stride;
-    bool const a_exists = row0 + a_row < g.m;
+    bool const a_exists = a_row < (uint32_t)ROWS && row0 + a_row < g.m;
+    uint8_t const *a_source = g.a + (uint64_t)(a_exists ? row0 + a_row : 0) * g.a_stride;
     double a_next[2], b_next[2];
     CompensatedSum squares; // distances: of this thread's share of its row of A
     auto fetch = [&](uint32_t k0) {
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
         b_next[0] = b_source[0], b_next[1] = b_source[1];
     };
     auto stash = [&](int buffer) {
-        a_lds[buffer][a_k][a_row] = a_next[0], a_lds[buffer][a_k + 1][a_row] = a_next[1];
+        if (a_row < (uint32_t)ROWS) a_lds[buffer][a_k][a_row] = a_next[0], a_lds[buffer][a_k + 1][a_row] = a_next[1];
         b_lds[buffer][b_k][b_col] = b_next[0], b_lds[buffer][b_k][b_col + 1] = b_next[1];
     };
 
@@ -238,15 +243,15 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
 #pragma unroll
         for (int kk = 0; kk < kWideDepth; ++kk) {
             if (k0 + kk >= depth) break; // (uniform; only the last step can be short)
-            double a_value[4], b_value[4];
+            double a_value[kRows], b_value[kCols];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a_value[i] = a_lds[buffer][kk][ty + 16 * i];
+            for (int i = 0; i < kRows; ++i) a_value[i] = a_lds[buffer][kk][ty + kDown * i];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b_value[j] = b_lds[buffer][kk][tx + 16 * j];
+            for (int j = 0; j < kCols; ++j) b_value[j] = b_lds[buffer][kk][tx + kAcross * j];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < kRows; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < kCols; ++j) {
                     dot2_step(acc[i][j][2 * (kk & 1)], acc[i][j][2 * (kk & 1) + 1], a_value[i], b_value[j]);
                 }
         }
@@ -255,11 +260,11 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
         buffer ^= 1;
     }
 
-    double column_norm[4];
+    double column_norm[kCols];
     if (NORMS) {
-        row_parts[a_row][tid & 3][0] = squares.sum, row_parts[a_row][tid & 3][1] = squares.lost;
+        if (a_row < (uint32_t)ROWS) row_parts[a_row][tid & 3][0] = squares.sum, row_parts[a_row][tid & 3][1] = squares.lost;
         __syncthreads();
-        if (tid < kWideTile) {
+        if (tid < ROWS) {
             CompensatedSum total;
 #pragma unroll
             for (int part = 0; part < 4; ++part) {
@@ -272,17 +277,17 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
         __syncthreads();
         double const *norms = g.b + (uint64_t)g.k_padded * g.n_padded; // behind the matrix, one per padded column
 #pragma unroll
-        for (int j = 0; j < 4; ++j) column_norm[j] = norms[col0 + tx + 16 * j];
+        for (int j = 0; j < kCols; ++j) column_norm[j] = norms[col0 + tx + kAcross * j];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        uint32_t const row = row0 + ty + 16 * i;
+    for (int i = 0; i < kRows; ++i) {
+        uint32_t const row = row0 + ty + kDown * i;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t const col = col0 + tx + 16 * j;
+        for (int j = 0; j < kCols; ++j) {
+            uint32_t const col = col0 + tx + kAcross * j;
             double result = fold_compensated(acc[i][j]);
             if (NORMS) {
-                result = wide_distance(g.metric, result, row_norms[ty + 16 * i], column_norm[j]);
+                result = wide_distance(g.metric, result, row_norms[ty + kDown * i], column_norm[j]);
                 if (g.tri_mask && row + g.tri_shift == col) result = 0; // a vector and itself: exactly 0
             }
             if (row < g.m && col < g.n && ((row + g.tri_shift) & g.tri_mask) <= col)
@@ -291,11 +296,11 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
     }
 }
 
-constexpr int kMatrixRows = 128, kMatrixCols = 64; // rows and columns of C per workgroup of the f32 matrix kernel
+constexpr int kMatrixRows = 128, kMatrixCols = 64; // rows (at most) and columns of C per workgroup of the f32 matrix kernel
 constexpr int kMatrixDepth = 32;                     // k per step: two groups of four MFMA depths for each of the four sums
 // A row of staged A is 128 bytes of f32, eight 16-byte units; unit u of row r sits at position u ^ (r % 8), so that the
 // eight lanes of an LDS cycle, which read the same unit of eight consecutive rows, or write the eight units of one row,
-// spread over all banks without padding. Two stages of A and of B (f64, [k][column]) fill the 64 KiB exactly.
+// spread over all banks without padding. Two stages of A and of B (f64, [k][column]) fill the 64 KiB exactly for 128 rows.
 
 /**
  *  f32 inputs on the f64 matrix cores. `v_mfma_f64_16x16x4_f64` is, per output, a chain of four fused multiply-adds in
@@ -307,33 +312,38 @@ constexpr int kMatrixDepth = 32;                     // k per step: two groups o
  *  reference does, and four instructions (r = 0..3) consume 16 depths. Zero padding past the last depth adds products
  *  of +0, which leave a sum that started at +0 unchanged (such a sum is never -0).
  *
- *  512 threads, 8 wavefronts as 4 x 2, each 32 x 32 outputs = 2 x 2 blocks x 4 sums = 128 accumulator registers, two
- *  wavefronts per SIMD. A is staged as f32, [row][k] so that one 16-byte read gives a lane the four operands
- *  (r = 0..3) of its row and depth group, and widened where it is multiplied; B comes from the k-major f64 image into
- *  [k][column]. A step is 32 depths = 32 MFMAs per wavefront; loads from memory are asked for a whole step before the
- *  stash that takes them, and the stash, the barrier and the reads of LDS sit between groups of MFMAs.
+ *  WR x WC wavefronts, each IB x JB blocks of outputs x 4 sums. The largest tile is 8 wavefronts as 4 x 2, each 32 x 32
+ *  outputs = 128 accumulator registers, two wavefronts per SIMD; f32_tile_rows() says when one of fewer rows is taken.
+ *  A is staged as f32, [row][k] so that one 16-byte read gives a lane the four operands (r = 0..3) of its row and depth
+ *  group, and widened where it is multiplied; B comes from the k-major f64 image into [k][column]. A step is 32 depths =
+ *  8 IB JB MFMAs per wavefront; loads from memory are asked for a whole step before the stash that takes them, and the
+ *  stash, the barrier and the reads of LDS sit between groups of MFMAs.
  */
-template <bool NORMS>
-__global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
+template <bool NORMS, int IB, int JB, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_matrix_kernel(WideArgs g) {
+    constexpr int ROWS = 16 * IB * WR, kThreads = 64 * WR * WC;
+    constexpr int kBLoads = kMatrixDepth * kMatrixCols / 2 / kThreads; // pairs of B's columns per thread and step
+    constexpr int kBApart = kThreads / 32;                             // depths between them
+    static_assert(16 * JB * WC == kMatrixCols && kThreads / 4 >= ROWS, "a tile is 64 columns, and its rows find their threads");
     typedef double __attribute__((ext_vector_type(4))) f64x4_t;
     typedef double __attribute__((ext_vector_type(2))) f64x2_t;
     typedef float __attribute__((ext_vector_type(4))) f32x4_t;
     typedef __attribute__((address_space(1))) double global_f64_t;
     typedef __attribute__((address_space(1))) uint64_t global_u64_t;
-    __shared__ __attribute__((aligned(16))) float a_lds[2][kMatrixRows][kMatrixDepth];
+    __shared__ __attribute__((aligned(16))) float a_lds[2][ROWS][kMatrixDepth];
     __shared__ __attribute__((aligned(16))) double b_lds[2][kMatrixDepth][kMatrixCols];
     // distances: four partial sums of squares per row of A and their total, in the B stages once the loop is over
     double(*row_parts)[4][2] = (double(*)[4][2]) & b_lds[0][0][0];
     double *row_norms = &b_lds[1][0][0];
-    static_assert(sizeof(double) * kMatrixRows * 8 <= sizeof(b_lds) / 2, "the partial sums fit one stage of B");
-    uint32_t const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint32_t const row0 = blockIdx.y * kMatrixRows, col0 = blockIdx.x * kMatrixCols;
+    static_assert(sizeof(double) * ROWS * 8 <= sizeof(b_lds) / 2, "the partial sums fit one stage of B");
+    uint32_t const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t const row0 = blockIdx.y * ROWS, col0 = blockIdx.x * kMatrixCols;
     // symmetric form: a tile wholly left of the diagonal has nothing to store
     if (((row0 + g.tri_shift) & g.tri_mask) > col0 + (kMatrixCols - 1)) return;
     PackedHeader const *header = (PackedHeader const *)((uint8_t const *)g.b - sizeof(PackedHeader));
     if (!(header->magic == kMagic && header->version == kVersion && header->dtype == (uint32_t)g.dtype && header->n == g.n &&
           header->k == g.k)) { // (an image of another type or shape: poison, as the f64 kernel does)
-        for (uint32_t at = tid; at < kMatrixRows * kMatrixCols; at += 512) {
+        for (uint32_t at = tid; at < ROWS * kMatrixCols; at += kThreads) {
             uint32_t const row = row0 + at / kMatrixCols, col = col0 + at % kMatrixCols;
             if (row < g.m && col < g.n && ((row + g.tri_shift) & g.tri_mask) <= col)
                 *(global_u64_t *)(g.c + (uint64_t)row * g.c_stride + (uint64_t)col * 8) = ~0ull;
@@ -341,45 +351,53 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
         return;
     }
 
-    uint32_t const wave_row = (wave >> 1) * 32, wave_col = (wave & 1) * 32;
+    uint32_t const wave_row = wave / WC * (16 * IB), wave_col = wave % WC * (16 * JB);
     uint32_t const in_block = lane & 15, depth_group = lane >> 4;
-    f64x4_t acc[2][2][4]; // [row block][column block][sum r]; element v: row 4 v + lane / 16, column lane % 16
+    f64x4_t acc[IB][JB][4]; // [row block][column block][sum r]; element v: row 4 v + lane / 16, column lane % 16
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < IB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < JB; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = f64x4_t {0, 0, 0, 0};
 
-    // staging: A: thread t brings 8 consecutive k of row t / 4; B: 2 consecutive columns of depths t / 32 and 16 + t / 32
+    // staging: A: thread t brings 8 consecutive k of row t / 4; B: 2 consecutive columns of depth t / 32 and
+    // the depths kBApart from it; a tile of few rows leaves A to its first wavefronts
     uint32_t const a_row = tid >> 2, a_k = (tid & 3) * 8;
     uint32_t const b_k = tid >> 5, b_col = (tid & 31) * 2;
+    bool const brings_a = kThreads / 4 == ROWS || wave < (uint32_t)(ROWS / 16); // (the same in a whole wavefront)
     uint32_t const a_from = row0 + a_row < g.m ? row0 + a_row : g.m - 1; // (rows past the end repeat the last; never stored)
     uint8_t const *a_source = g.a + (uint64_t)a_from * g.a_stride;
     bool const aligned = ((((uint64_t)g.a) | g.a_stride) & 15) == 0;
     f32x4_t a_next[2];
-    f64x2_t b_next[2];
+    f64x2_t b_next[kBLoads];
     CompensatedSum squares; // distances: of this thread's share of its row of A
     // `whole`: the step lies inside the rows of A and they can be read 16 bytes at a time. It is a compile-time choice, one
     // loop for each: where both ways to load sit in one loop, waits for the loads come between them, in front of the MFMAs
     // that are there to cover them.
     auto fetch = [&](uint32_t k0, auto whole) {
+        if (brings_a) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t const at = k0 + a_k + 4 * h;
-            if (whole) a_next[h] = *(f32x4_t const *)(a_source + (uint64_t)at * 4);
-            else {
+            for (int h = 0; h < 2; ++h) {
+                uint32_t const at = k0 + a_k + 4 * h;
+                if (whole) a_next[h] = *(f32x4_t const *)(a_source + (uint64_t)at * 4);
+                else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a_next[h][e] = at + e < g.k ? ((float const *)a_source)[at + e] : 0.f;
+                    for (int e = 0; e < 4; ++e) a_next[h][e] = at + e < g.k ? ((float const *)a_source)[at + e] : 0.f;
+                }
             }
-            b_next[h] = *(f64x2_t const *)(g.b + (uint64_t)(k0 + b_k + 16 * h) * g.n_padded + col0 + b_col); // (inside the padded image)
         }
+#pragma unroll
+        for (int h = 0; h < kBLoads; ++h) // (inside the padded image)
+            b_next[h] = *(f64x2_t const *)(g.b + (uint64_t)(k0 + b_k + kBApart * h) * g.n_padded + col0 + b_col);
     };
     auto stash = [&](int buffer) { // (the first use of what fetch() asked for: the wait for it sits here, behind a group of MFMAs)
 #pragma unroll
+        for (int h = 0; h < kBLoads; ++h) *(f64x2_t *)&b_lds[buffer][b_k + kBApart * h][b_col] = b_next[h];
+        if (!brings_a) return;
+#pragma unroll
         for (int h = 0; h < 2; ++h) {
             *(f32x4_t *)&a_lds[buffer][a_row][4 * ((a_k / 4 + h) ^ (a_row & 7))] = a_next[h];
-            *(f64x2_t *)&b_lds[buffer][b_k + 16 * h][b_col] = b_next[h];
             if (NORMS) { // four exact squares summed with three roundings of their own small sum, then one compensated addition
                 double const x0 = a_next[h][0], x1 = a_next[h][1], x2 = a_next[h][2], x3 = a_next[h][3];
                 squares.add(__builtin_fma(x0, x0, __builtin_fma(x1, x1, __builtin_fma(x2, x2, x3 * x3))));
@@ -387,17 +405,17 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
         }
     };
     struct Operands {
-        f32x4_t a[2];   // [row block]: as staged, widened where it is multiplied: nothing between two groups of MFMAs waits on LDS
-        double b[2][4]; // [column block][sum r]
+        f32x4_t a[IB];   // [row block]: as staged, widened where it is multiplied: nothing between two groups of MFMAs waits on LDS
+        double b[JB][4]; // [column block][sum r]
     };
     auto read_operands = [&](int buffer, int group, Operands &operands) { // 16 depths: 16 group + r + 4 (lane / 16)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < IB; ++i) {
             uint32_t const row = wave_row + 16 * i + in_block;
             operands.a[i] = *(f32x4_t const *)&a_lds[buffer][row][4 * ((4 * group + depth_group) ^ (row & 7))];
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < JB; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 operands.b[j][r] = b_lds[buffer][16 * group + r + 4 * depth_group][wave_col + 16 * j + in_block];
@@ -406,9 +424,9 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
 #pragma unroll
         for (int r = from; r < to; ++r)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < IB; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < JB; ++j)
                     acc[i][j][r] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)operands.a[i][r], operands.b[j][r], acc[i][j][r], 0, 0, 0);
     };
 
@@ -426,9 +444,9 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
     __syncthreads();
     read_operands(0, 0, first);
     int buffer = 0;
-    // One step: 32 MFMAs, and between them, where none of it holds the matrix pipe up: the stash of the step after this one
+    // One step: 8 IB JB MFMAs, and between them, where none of it holds the matrix pipe up: the stash of the step after this one
     // (its stage was last read before the previous barrier), the request for the step after that, the barrier, and the
-    // reads of LDS, each asked for at least 8 MFMAs before its use. The scheduler is held to this order.
+    // reads of LDS, each asked for a quarter of them before its use. The scheduler is held to this order.
     auto step = [&](uint32_t k0, auto whole) { // (a whole step: neither the last nor the one before it)
         bool const more = whole || k0 + kMatrixDepth < depth;
         read_operands(buffer, 1, second);
@@ -455,11 +473,11 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
         for (; k0 + 3 * kMatrixDepth <= g.k; k0 += kMatrixDepth) step(k0, whole);
     for (; k0 < depth; k0 += kMatrixDepth) step(k0, piecewise);
 
-    double column_norm[2];
+    double column_norm[JB];
     if (NORMS) {
-        row_parts[a_row][tid & 3][0] = squares.sum, row_parts[a_row][tid & 3][1] = squares.lost; // (no read of a stage follows the loop's last barrier)
+        if (brings_a) row_parts[a_row][tid & 3][0] = squares.sum, row_parts[a_row][tid & 3][1] = squares.lost; // (no read of a stage follows the loop's last barrier)
         __syncthreads();
-        if (tid < kMatrixRows) {
+        if (tid < ROWS) {
             CompensatedSum total;
 #pragma unroll
             for (int part = 0; part < 4; ++part) {
@@ -472,15 +490,15 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
         __syncthreads();
         double const *norms = g.b + (uint64_t)g.k_padded * g.n_padded; // behind the matrix, one per padded column
 #pragma unroll
-        for (int j = 0; j < 2; ++j) column_norm[j] = norms[col0 + wave_col + 16 * j + in_block];
+        for (int j = 0; j < JB; ++j) column_norm[j] = norms[col0 + wave_col + 16 * j + in_block];
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < IB; ++i)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             uint32_t const in_tile = wave_row + 16 * i + 4 * v + depth_group, row = row0 + in_tile;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < JB; ++j) {
                 uint32_t const col = col0 + wave_col + 16 * j + in_block;
                 double result = ((acc[i][j][0][v] + acc[i][j][1][v]) + acc[i][j][2][v]) + acc[i][j][3][v];
                 if (NORMS) {
@@ -491,6 +509,52 @@ __global__ __launch_bounds__(512) void dots_f32_matrix_kernel(WideArgs g) {
                     __builtin_nontemporal_store(result, (global_f64_t *)(g.c + (uint64_t)row * g.c_stride + (uint64_t)col * 8));
             }
         }
+}
+
+/**
+ *  Rows of a tile, out of those the kernels are built for: the cheapest by rounds of one tile per compute unit times what a
+ *  tile costs a unit, in sixteens of rows through the arithmetic (as measured below; a lower row count wins only if it is
+ *  cheaper). Every output is one thread's chain along k whatever the tile, so the choice changes no bit.
+ */
+struct TileCost {
+    int rows;
+    float cost;
+};
+template <int COUNT>
+int cheapest_tile(WideArgs const &g, TileCost const (&tiles)[COUNT]) {
+    int const units = compute_unit_count() > 0 ? compute_unit_count() : 256;
+    int best = tiles[0].rows;
+    double least = 0;
+    for (int i = 0; i < COUNT; ++i) {
+        uint64_t const rows = (uint64_t)tiles[i].rows;
+        uint64_t const count = g.tri_mask ? live_tiles(g.m, g.n, (uint32_t)rows, kWideTile, g.tri_shift)
+                                          : (g.m + rows - 1) / rows * (g.n_padded / kWideTile);
+        double const cost = (double)((count + units - 1) / units) * tiles[i].cost;
+        if ((g.m + rows - 1) / rows > 65535) continue; // (what the grid's second dimension holds; never the first of the list)
+        if (i == 0 || cost < least) best = tiles[i].rows, least = cost;
+    }
+    return best;
+}
+/** f64: bound by the vector units, so a tile costs its rows, and a little more the fewer outputs a thread has to share what
+ *  it reads from LDS with. Measured, 64 rows against 16 against 4 (us): 1 x 100,000 x 1024 2322, 639, 260 (3.2 TB/s of the
+ *  image); 8 rows 2318, 644, 443; 16 rows 2317, 695, 849; 48 x 50,000 x 1024 1391, 970, 1230; few tiles: 64 x 1024 x 4096
+ *  1649, 613, 354, all pairs of 256 x 1024 436, 176, 112; many: 1000 x 20,001 x 300 2049, 2163, 2603. */
+int f64_tile_rows(WideArgs const &g) {
+    static TileCost const tiles[] = {{64, 4.0f}, {16, 1.03f}, {4, 0.32f}};
+    return cheapest_tile(g, tiles);
+}
+/** f32: bound by the f64 matrix instructions, and below about 48 rows by the image, eight bytes per value. Measured, 128
+ *  rows against 64, 32 and 16 (us): 1 x 100,000 x 1024 501, 267, 184, 170 (4.8 TB/s); 32 rows 502, 269, 186, 328; 48 rows
+ *  506, 271, 336, 478; 150 x 50,000 x 512 278, 203, 204, 369; few tiles: 64 x 1024 x 4096 279, 174, 113, 80; many: 4096 x
+ *  4096 x 1024 589, 592, 594, 655. Shallow products gain by the 64-row tile however many there are, two of which share a
+ *  compute unit, so that one multiplies under the other's epilogue: 1000 x 20,001 x 300 286, 262, 311, 563, angular 333,
+ *  302, 327, 574. All pairs lose by it (3000 x 1000: 249, 261, 225, 348). */
+int f32_tile_rows(WideArgs const &g) {
+    static TileCost const shallow[] = {{128, 8.2f}, {64, 4.05f}, {32, 2.75f}, {16, 2.6f}};
+    static TileCost const deep[] = {{128, 8.2f}, {64, 4.2f}, {32, 2.75f}, {16, 2.6f}};
+    static TileCost const pairs[] = {{128, 8.2f}, {32, 2.3f}, {16, 2.0f}};
+    if (g.tri_mask) return cheapest_tile(g, pairs);
+    return g.k_padded <= 512 ? cheapest_tile(g, shallow) : cheapest_tile(g, deep);
 }
 
 __global__ __launch_bounds__(256) void fill_wide_kernel(uint8_t *c, uint32_t m, uint32_t n, uint64_t c_stride, uint64_t bits,
@@ -577,12 +641,18 @@ hipError_t wide_product(int dtype, void const *a, void const *b_packed, void *c,
         uint64_t const rows = m - first < band ? m - first : band;
         g.a = (uint8_t const *)a + first * a_stride, g.c = (uint8_t *)c + first * c_stride;
         g.m = (uint32_t)rows, g.tri_shift = shift + (uint32_t)first;
-        dim3 const grid(geo.n_padded / kWideTile, (uint32_t)((rows + kWideTile - 1) / kWideTile));
-        dim3 const matrix_grid(geo.n_padded / kMatrixCols, (uint32_t)((rows + kMatrixRows - 1) / kMatrixRows));
-        if (dtype == kF64 && metric) hipLaunchKernelGGL(dots_f64_compensated_kernel<true>, grid, dim3(256), 0, stream, g);
-        else if (dtype == kF64) hipLaunchKernelGGL(dots_f64_compensated_kernel<false>, grid, dim3(256), 0, stream, g);
-        else if (metric) hipLaunchKernelGGL(dots_f32_matrix_kernel<true>, matrix_grid, dim3(512), 0, stream, g);
-        else hipLaunchKernelGGL(dots_f32_matrix_kernel<false>, matrix_grid, dim3(512), 0, stream, g);
+        int const rows_of_tile = dtype == kF64 ? f64_tile_rows(g) : f32_tile_rows(g);
+        dim3 const grid(geo.n_padded / kWideTile, (uint32_t)((rows + rows_of_tile - 1) / rows_of_tile));
+        auto launch = [&](void (*kernel)(WideArgs), int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, g); };
+        if (dtype == kF64) {
+            if (rows_of_tile == 64) launch(metric ? dots_f64_compensated_kernel<true, 64> : dots_f64_compensated_kernel<false, 64>, 256);
+            else if (rows_of_tile == 16) launch(metric ? dots_f64_compensated_kernel<true, 16> : dots_f64_compensated_kernel<false, 16>, 256);
+            else launch(metric ? dots_f64_compensated_kernel<true, 4> : dots_f64_compensated_kernel<false, 4>, 256);
+        }
+        else if (rows_of_tile == 128) launch(metric ? dots_f32_matrix_kernel<true, 2, 2, 4, 2> : dots_f32_matrix_kernel<false, 2, 2, 4, 2>, 512);
+        else if (rows_of_tile == 64) launch(metric ? dots_f32_matrix_kernel<true, 2, 2, 2, 2> : dots_f32_matrix_kernel<false, 2, 2, 2, 2>, 256);
+        else if (rows_of_tile == 32) launch(metric ? dots_f32_matrix_kernel<true, 2, 1, 1, 4> : dots_f32_matrix_kernel<false, 2, 1, 1, 4>, 256);
+        else launch(metric ? dots_f32_matrix_kernel<true, 1, 1, 1, 4> : dots_f32_matrix_kernel<false, 1, 1, 1, 4>, 256);
         hipError_t const status = hipGetLastError();
         if (status != hipSuccess) return status;
     }
