@@ -79,7 +79,7 @@ struct GemmArgs {
     // Store-bound shapes: workgroup b starts b * stagger_ticks / gridDim.x ticks of the 100 MHz clock late, so that the
     // compute phases of some compute units fall into the store phases of others (0: all start together).
     uint32_t stagger_ticks;
-    uint32_t store_policy; // 0: by the alignment of C's rows; 1: past the caches; 2: through them (test hook)
+    uint32_t store_policy; // 0: by the alignment of C's rows; 1: past the caches; 2: through them
     uint32_t tile_count;       // tiles_m * tiles_n, or the length of the list
     uint32_t const *tile_list; // (tile row, tile column) pairs in walking order, or NULL for the full grid
 };
@@ -2061,7 +2061,7 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     }
     int const forced = forced_tile_config();
     if ((forced >> 8) & 0xFFFFF) g.stagger_ticks = (uint32_t)((forced >> 8) & 0xFFFFF) - 1; // (test hook: bits 8..27 = ticks + 1)
-    g.store_policy = (uint32_t)(forced >> 28) & 3;                                          // (test hook: bits 28..29)
+    if ((forced >> 28) & 3) g.store_policy = (uint32_t)(forced >> 28) & 3;                  // (test hook: bits 28..29)
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, g);
     return hipGetLastError();
 }
@@ -2095,6 +2095,11 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         if (triangle) return live_tiles(args.m, args.n, (uint32_t)bm, (uint32_t)bn, args.tri_shift);
         return ((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn);
     };
+    auto unaligned_rows_of_c = [&](GemmArgs const &args) { return !triangle && args.metric == 0 && (((uintptr_t)args.c | args.c_stride) & 127) != 0; };
+    // (strides that the 32-bit offsets of a taller or wider tile could not span stay with the small one)
+    auto roomy = [](GemmArgs const &args) { return args.m >= 128 && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024; };
+    auto large_c = [&](GemmArgs const &args) { return roomy(args) && (uint64_t)args.m * args.n * 4 > 384ull << 20; };
+    auto middling_c = [&](GemmArgs const &args) { return roomy(args) && (uint64_t)args.m * args.n * 4 > 128ull << 20; };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
     auto choose = [&](GemmArgs const &args, int first) {
         uint32_t const depth_stages = args.k_chunks / kStageChunks;
@@ -2143,10 +2148,27 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // with the others' loops, which one large tile cannot (measured, 64 x 128 against the tile chosen above: i8
         // 8192 x 8191 x 1000 0.129 against 0.142 ms, x 512 0.085 against 0.101; f16 8192 x 8191 x 1000 0.239 against
         // 0.280; i8 4096 x 4095 x 1000 0.036 against 0.039; deeper products and aligned rows lose by it).
-        bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0;
-        if (!lines && !triangle && args.metric == 0 && best < 4 && args.k_chunks / kStageChunks <= (T::kChunked ? 16u : 8u) &&
-            tiles_of(args, 4) >= 256)
-            best = 4;
+        // That holds while the last-level cache (256 MiB) takes C in. A larger C is bound by the memory, which the small
+        // tile's many short writes reach as they are: the integers do better through tiles that write longer runs of a row,
+        // the floats, which spend more time multiplying, past the caches. Measured, 64 x 128 against the tile taken (us): i8
+        // 1000 x 500,009 x 304 1226 against 972 (128 x 256), x 1,000,001 x 768 (1024 rows) 2855 against 1879 (256 x 256,
+        // whose rows have to be there: 777 x 200,003 x 900 502 against 360, and 337 with 128 x 256; u8, which does more to
+        // every row it stages, 532 against 427 and 349), 128 x 1,000,001 x 256 247 against 229 (128 x 128); f16 1000 x
+        // 300,009 x 304 862 against 628 (128 x 128), 4096 x 50,001 x 512 665 against 375 (but 3000 x 40,001 x 200, 234 against
+        // 269), 1024 x 500,001 x 768 1889 against 1538 (128 x 256). Deeper products into a C that the cache would lose the
+        // operands to: 128 x 128 past the caches against the largest tile through them, 8192 x 8191 x 2000, i8 211 against
+        // 194, u8 234 against 208, f16 447 against 395; 2000 x 60,001 x 1500, i8 481 (64 x 128) against 309, f16 715 against 634.
+        if (unaligned_rows_of_c(args) && best < 4) {
+            uint32_t const limit = T::kChunked ? 16 : 8;
+            bool const half_empty = args.m < 2048 && ((args.m + 127) / 128) % 2 != 0; // the last 256 rows of A
+            if (depth_stages <= limit && large_c(args) && !(T::kChunked && depth_stages <= 4)) {
+                if (T::kChunked) best = depth_stages <= 8 ? 3 : 2;
+                else if (depth_stages <= 2) best = 3;
+                else if (depth_stages <= 4 || T::kUnsigned || half_empty) best = 2;
+            }
+            else if (depth_stages <= limit) best = tiles_of(args, 4) >= 256 ? 4 : best;
+            else if (depth_stages <= 2 * limit && middling_c(args)) best = 3;
+        }
         // e2m3 pays 13 vector operations for every dword of A it stages: a 128 x 512 tile (every wavefront 128 x 128)
         // stages half as much A per MFMA as 256 x 256 (8192^3: 0.51 against 0.59 ms; for i8 itself the two are equal)
         // (not the f16 route of very deep rows: its two accumulator sets do not fit that tile)
@@ -2154,6 +2176,11 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         return best;
     };
     if (chosen_here) config = choose(g, 1);
+    g.store_policy = 0;
+    if (chosen_here && config == 3 && unaligned_rows_of_c(g)) { // (see choose())
+        uint32_t const depth_stages = g.k_chunks / kStageChunks, limit = T::kChunked ? 16 : 8;
+        if (depth_stages <= limit ? T::kChunked && depth_stages > 4 && depth_stages <= 8 && large_c(g) : depth_stages <= 2 * limit && middling_c(g)) g.store_policy = 1;
+    }
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
     if (triangle && config >= kTriangleConfigs) config = 4;
     // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
