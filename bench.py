@@ -448,6 +448,19 @@ def cpu_baseline(dtype, m, n, k, budget_rows=8192):
                        "(every core the process may use), best and median of 3 after a warm-up run")}
 
 
+def cpu_baselines(dtype, m, n, k, headline):
+    """cpu_baseline of the timed type and, beside the headline, of the metric's other types on a stated share of the rows
+    of A (the kernels are 5-10 times slower). The fallback has no median and names no kernel: what it has is carried."""
+    result = cpu_baseline(dtype, m, n, k)
+    if headline:
+        each = {dtype: dict(result)}
+        for other in METRIC_DTYPES[1:]:
+            each[other] = cpu_baseline(other, m, n, k, budget_rows=2048)
+        kept = ("value", "median", "cores", "kernel_capability", "sample")
+        result["by_dtype"] = {name: {key: one[key] for key in kept if key in one} for name, one in each.items()}
+    return result
+
+
 def main():
     global SPIN_UP_MS
     parser = argparse.ArgumentParser()
@@ -563,12 +576,7 @@ def main():
         "roofline": head["roofline"],
     })
     if not args.no_cpu:
-        line["cpu_baseline"] = cpu_baseline(args.dtype, m, n, k)
-        if headline:  # the metric's other two types, on a stated share of the rows of A (the kernels are 5-10 times slower)
-            line["cpu_baseline"]["by_dtype"] = {"i8": {key: line["cpu_baseline"][key] for key in ("value", "median", "cores", "kernel_capability", "sample")}}
-            for dtype in METRIC_DTYPES[1:]:
-                other = cpu_baseline(dtype, m, n, k, budget_rows=2048)
-                line["cpu_baseline"]["by_dtype"][dtype] = {key: other[key] for key in ("value", "median", "cores", "kernel_capability", "sample") if key in other}
+        line["cpu_baseline"] = cpu_baselines(args.dtype, m, n, k, headline)
     print(json.dumps(line))
 
 
