@@ -2098,10 +2098,14 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     auto unaligned_rows_of_c = [&](GemmArgs const &args) { return !triangle && args.metric == 0 && (((uintptr_t)args.c | args.c_stride) & 127) != 0; };
     // (strides that the 32-bit offsets of a taller or wider tile could not span stay with the small one)
     auto roomy = [](GemmArgs const &args) { return args.m >= 128 && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024; };
-    auto large_c = [&](GemmArgs const &args) { return roomy(args) && (uint64_t)args.m * args.n * 4 > 384ull << 20; };
-    auto middling_c = [&](GemmArgs const &args) { return roomy(args) && (uint64_t)args.m * args.n * 4 > 128ull << 20; };
+    struct Choice {
+        int config;
+        uint32_t store_policy;
+        Choice(int config, uint32_t store_policy = 0) : config(config), store_policy(store_policy) {}
+    };
+    auto past = [](int config) { return Choice(config, 1); };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
-    auto choose = [&](GemmArgs const &args, int first) {
+    auto choose = [&](GemmArgs const &args, int first) -> Choice {
         uint32_t const depth_stages = args.k_chunks / kStageChunks;
         // Few rows: a tile of more rows than A has multiplies what is not there (i8 1 x 1,048,576 x 768 through the 256-row
         // tile was bound by its matrix instructions), and one that is not full stores through the masked copy of the
@@ -2143,44 +2147,69 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // Two accumulator sets do not fit the 256 x 256 tile, and neither do the fifth dwords of shifted loads (99 registers
         // of the i8 kernel spill).
         if ((T::kChunked || needs_shift<T>(args)) && best == 1) best = 2;
-        // Shallow products into rows of C that do not start on 128-byte lines: the stores go through the L2 (see the
+        // e2m3 pays 13 vector operations for every dword of A it stages: a 128 x 512 tile (every wavefront 128 x 128)
+        // stages half as much A per MFMA as 256 x 256 (8192^3: 0.51 against 0.59 ms; for i8 itself the two are equal). Rows of C
+        // off the lines keep it: the rule below is of mixed use there (1000 x 300,009 x 304 579 against 813 us, but 512 x 153,601
+        // x 900 240 against 186).
+        // (not the f16 route of very deep rows: its two accumulator sets do not fit that tile)
+        if (T::kDtype == kE2M3 && !T::kChunked && !triangle && args.metric == 0 && first == 1 && !needs_shift<T>(args) && tiles_of(args, 5) >= 256) return 5;
+        // Products into rows of C that do not start on 128-byte lines. The stores of shallow ones go through the L2 (see the
         // epilogue) and take long enough to matter, and three small workgroups per compute unit overlap one's stores
         // with the others' loops, which one large tile cannot (measured, 64 x 128 against the tile chosen above: i8
         // 8192 x 8191 x 1000 0.129 against 0.142 ms, x 512 0.085 against 0.101; f16 8192 x 8191 x 1000 0.239 against
         // 0.280; i8 4096 x 4095 x 1000 0.036 against 0.039; deeper products and aligned rows lose by it).
-        // That holds while the last-level cache (256 MiB) takes C in. A larger C is bound by the memory, which the small
-        // tile's many short writes reach as they are: the integers do better through tiles that write longer runs of a row,
-        // the floats, which spend more time multiplying, past the caches. Measured, 64 x 128 against the tile taken (us): i8
-        // 1000 x 500,009 x 304 1226 against 972 (128 x 256), x 1,000,001 x 768 (1024 rows) 2855 against 1879 (256 x 256,
-        // whose rows have to be there: 777 x 200,003 x 900 502 against 360, and 337 with 128 x 256; u8, which does more to
-        // every row it stages, 532 against 427 and 349), 128 x 1,000,001 x 256 247 against 229 (128 x 128); f16 1000 x
-        // 300,009 x 304 862 against 628 (128 x 128), 4096 x 50,001 x 512 665 against 375 (but 3000 x 40,001 x 200, 234 against
-        // 269), 1024 x 500,001 x 768 1889 against 1538 (128 x 256). Deeper products into a C that the cache would lose the
-        // operands to: 128 x 128 past the caches against the largest tile through them, 8192 x 8191 x 2000, i8 211 against
-        // 194, u8 234 against 208, f16 447 against 395; 2000 x 60,001 x 1500, i8 481 (64 x 128) against 309, f16 715 against 634.
-        if (unaligned_rows_of_c(args) && best < 4) {
-            uint32_t const limit = T::kChunked ? 16 : 8;
-            bool const half_empty = args.m < 2048 && ((args.m + 127) / 128) % 2 != 0; // the last 256 rows of A
-            if (depth_stages <= limit && large_c(args) && !(T::kChunked && depth_stages <= 4)) {
-                if (T::kChunked) best = depth_stages <= 8 ? 3 : 2;
-                else if (depth_stages <= 2) best = 3;
-                else if (depth_stages <= 4 || T::kUnsigned || half_empty) best = 2;
+        // That holds while the last-level cache (256 MiB) takes most of C in. A larger C is bound by the memory, which the small
+        // tile's many short writes reach as they are, and what is best then depends on the image: as long as the cache can hold
+        // that, C is better written past it. The lines below were drawn through 8700 timed shapes (128 to 8192 rows, C of 130
+        // to 1700 MiB, depths to 2048, rows off the lines by 4 to 64 bytes; 5000 of them at random, every tile at each). The
+        // time of 64 x 128 (of the largest tile for the deeper products) over that of the tile taken, mean and least: floats of 5
+        // to 16 stages 1.22 and 0.79, deeper 1.08 and 0.85; integers of 2 stages 1.09 and 0.80, of 3 and 4 1.22 and 0.96, of 5
+        // to 8 1.32 and 0.90, deeper 1.15 and 0.80 (16 in 1000 of all shapes lose more than 3 per cent); of the best tile at
+        // each, 0.96. Some of them (us): i8 1000 x 500,009 x 304 1226 through 64 x 128 and 972 through
+        // 128 x 256, 1024 x 1,000,001 x 768 2855 and 1879 through 256 x 256 (300 x 524,289 x 768, which leaves a quarter of the
+        // tall tiles empty, 377 through them and 287 through 128 x 256); i8 1024 x 204,801 x 1500 (an image of 300 MiB) 692 past
+        // the caches, 566 through 256 x 256, but 1024 x 107,521 x 1500 (158 MiB) 288 and 306; bf16 2400 x 45,857 x 900 415
+        // through 64 x 128, 337 through 128 x 128 past the caches, 476 through 128 x 256, whose kernel for ragged depths of
+        // 16-bit floats and for shifted rows spills.
+        uint32_t const limit = T::kChunked ? 16 : 8;
+        if (unaligned_rows_of_c(args) && best < 4 && depth_stages <= 2 * limit) {
+            bool const shallow = depth_stages <= limit, bits = T::kDtype == kU1;
+            Choice const small = tiles_of(args, 4) >= 256 ? 4 : best; // 64 x 128 where it gives every CU a tile
+            uint64_t const c_mib = ((uint64_t)args.m * args.n * 4) >> 20;
+            uint64_t const image_mib = ((uint64_t)args.n_tiles * args.k_chunks * kTileRows * T::kImageChunk) >> 20;
+            uintptr_t const rows_at = (uintptr_t)args.c | args.c_stride;
+            bool const halves = (rows_at & 63) == 0 && image_mib < 256; // rows on halves of lines: past the caches they cost no more than whole lines
+            if (!roomy(args) || c_mib < 128) return shallow ? small : Choice(best);
+            if (T::kChunked) {
+                if (depth_stages <= 4) return small;
+                if (image_mib < 256) return c_mib < (!shallow ? (image_mib < 100 ? 256 : 0) : image_mib < 30 ? 384 : image_mib < 100 ? 320 : 200) ? small : past(3);
+                if (shallow && c_mib < 384) return small;
+                if (!(needs_shift<T>(args) || (T::kSrcChunk == 16 && args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) != 0))) return 2;
+                if (shallow) return args.m > 128 && args.m <= 192 ? small : Choice(3); // (three tiles of 64, but four of them in tiles of 128)
+                return args.m > 1000 ? past(3) : Choice(3);
             }
-            else if (depth_stages <= limit) best = tiles_of(args, 4) >= 256 ? 4 : best;
-            else if (depth_stages <= 2 * limit && middling_c(args)) best = 3;
+            if (depth_stages <= 2) return c_mib < 384 ? small : halves && !bits ? past(3) : Choice(3);
+            if (bits) { // (operands of an eighth)
+                if (depth_stages <= 4) return c_mib < 320 ? small : Choice(args.m <= 160 || (args.m < 800 && c_mib > 640) ? 2 : 3);
+                if (shallow) return c_mib < 384 ? small : Choice(args.m < 600 || c_mib > 1200 || (c_mib > 640 && args.m <= 1500) ? 2 : 3);
+                if ((rows_at & 15) == 0) return halves || c_mib >= 300 ? past(3) : Choice(3);
+                return c_mib < 512 ? small : Choice(3);
+            }
+            if (depth_stages <= 4) return c_mib < 320 ? small : halves ? past(3) : Choice(image_mib < 30 || args.m <= 128 ? 3 : 2);
+            if (shallow) {
+                int const wide = args.m <= 400 || T::kUnsigned || (args.m < 1024 && ((args.m + 127) / 128) % 2 != 0) ? 2 : best;
+                if (c_mib < (image_mib < 10 ? 320 : 256)) return small;
+                if (image_mib >= 256) return wide;
+                if (c_mib < 320) return 3;
+                return (rows_at & 7) == 0 ? past(3) : Choice(T::kUnsigned && image_mib < 100 ? 3 : wide);
+            }
+            if (image_mib < 256) return image_mib < 30 && c_mib < 240 ? Choice(3) : past(3);
+            return args.m <= 400 || (T::kUnsigned && c_mib < 640) ? 2 : best;
         }
-        // e2m3 pays 13 vector operations for every dword of A it stages: a 128 x 512 tile (every wavefront 128 x 128)
-        // stages half as much A per MFMA as 256 x 256 (8192^3: 0.51 against 0.59 ms; for i8 itself the two are equal)
-        // (not the f16 route of very deep rows: its two accumulator sets do not fit that tile)
-        if (T::kDtype == kE2M3 && !T::kChunked && !triangle && args.metric == 0 && first == 1 && !needs_shift<T>(args) && tiles_of(args, 5) >= 256) best = 5;
         return best;
     };
-    if (chosen_here) config = choose(g, 1);
-    g.store_policy = 0;
-    if (chosen_here && config == 3 && unaligned_rows_of_c(g)) { // (see choose())
-        uint32_t const depth_stages = g.k_chunks / kStageChunks, limit = T::kChunked ? 16 : 8;
-        if (depth_stages <= limit ? T::kChunked && depth_stages > 4 && depth_stages <= 8 && large_c(g) : depth_stages <= 2 * limit && middling_c(g)) g.store_policy = 1;
-    }
+    Choice const chosen = chosen_here ? choose(g, 1) : Choice(config);
+    config = chosen.config, g.store_policy = chosen.store_policy;
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
     if (triangle && config >= kTriangleConfigs) config = 4;
     // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
@@ -2225,13 +2254,13 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
                 // each launch builds its tile list in its own half of the scratch memory
                 size_t const half = triangle->bytes / 2 / 8 * 8;
                 TriangleScratch const first_half = {triangle->words, half}, second_half = {triangle->words + half / 4, half};
-                int const small = choose(bottom, config + 1);
+                int const narrow = choose(bottom, config + 1).config;
                 TriangleGrids grids;
-                grids.grid[0] = grid_of(top, config, first_half), grids.grid[1] = grid_of(bottom, small, second_half);
+                grids.grid[0] = grid_of(top, config, first_half), grids.grid[1] = grid_of(bottom, narrow, second_half);
                 hipLaunchKernelGGL(triangle_tiles_kernel, dim3(2), dim3(256), 0, stream, grids);
                 if ((e = hipGetLastError()) != hipSuccess) return e;
                 if ((e = launch_config<T>(top, stream, &first_half, config)) != hipSuccess) return e;
-                return launch_config<T>(bottom, stream, &second_half, small);
+                return launch_config<T>(bottom, stream, &second_half, narrow);
             }
         }
     }
