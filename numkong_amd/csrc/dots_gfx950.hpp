@@ -2147,6 +2147,16 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // Two accumulator sets do not fit the 256 x 256 tile, and neither do the fifth dwords of shifted loads (99 registers
         // of the i8 kernel spill).
         if ((T::kChunked || needs_shift<T>(args)) && best == 1) best = 2;
+        // Two stages: the pipeline starts anew with every tile, the large tiles' kernels spill around that (e4m3 and e5m2 80
+        // registers at 128 x 256, 13 before they held a loop for odd rows), and the stores are nearly all of the work. Measured,
+        // the largest tile against 64 x 128 (us), C on whole lines: e4m3 2000 x 262,144 x 128 878 (767 with 13 spilled) against 424,
+        // 1000 x 100,000 x 128 186 against 90, 300 x 60,000 x 128 33 against 18, 8192 x 8192 x 128 62 against 55; bf16 1130, 236, 39
+        // and 67 against 430, 92, 20 and 57; i8 1228, 278, 41 and 71 against 414, 87, 18 and 51; the others likewise. Not the
+        // floats up to 128 MiB of C in rows that are 64 KiB or a multiple apart (512 x 65,536 x 128, e4m3 32.8 against 34.2, bf16 35.6
+        // against 36.2).
+        if (depth_stages <= 2 && args.metric == 0 && args.m >= 128 && !unaligned_rows_of_c(args) &&
+            !(T::kChunked && (args.c_stride & 0xFFFF) == 0 && (uint64_t)args.m * args.n * 4 <= 128ull << 20))
+            return tiles_of(args, 4) >= 256 ? 4 : best;
         // e2m3 pays 13 vector operations for every dword of A it stages: a 128 x 512 tile (every wavefront 128 x 128)
         // stages half as much A per MFMA as 256 x 256 (8192^3: 0.51 against 0.59 ms; for i8 itself the two are equal). Rows of C
         // off the lines keep it: the rule below is of mixed use there (1000 x 300,009 x 304 579 against 813 us, but 512 x 153,601
