@@ -546,15 +546,25 @@ int f64_tile_rows(WideArgs const &g) {
 /** f32: bound by the f64 matrix instructions, and below about 48 rows by the image, eight bytes per value. Measured, 128
  *  rows against 64, 32 and 16 (us): 1 x 100,000 x 1024 501, 267, 184, 170 (4.8 TB/s); 32 rows 502, 269, 186, 328; 48 rows
  *  506, 271, 336, 478; 150 x 50,000 x 512 278, 203, 204, 369; few tiles: 64 x 1024 x 4096 279, 174, 113, 80; many: 4096 x
- *  4096 x 1024 589, 592, 594, 655. Shallow products gain by the 64-row tile however many there are, two of which share a
- *  compute unit, so that one multiplies under the other's epilogue: 1000 x 20,001 x 300 286, 262, 311, 563, angular 333,
- *  302, 327, 574. All pairs lose by it (3000 x 1000: 249, 261, 225, 348). */
+ *  4096 x 1024 589, 592, 594, 655. Up to 512 values the 128-row tile is never the cheaper one: two of 64 rows share a compute
+ *  unit, so that one multiplies under the other's epilogue. 128 against 64, kernels alone, 1000 x 20,001 dots and angular: 256
+ *  values 246 and 214, 283 and 252; 300 values 275 and 249, 322 and 290; 400 values 334 and 315, 385 and 356; 512 values 398
+ *  and 373, 448 and 415; 4096 x 4096 likewise (300 values 204 and 197, 512 values 313 and 299). The gain shrinks with depth
+ *  and does not end at 512 (640 values 480 and 464, 539 and 511; 1024 values, angular, 796 and 762): deeper products keep
+ *  the cost by rounds. Where the 128-row tiles are one round at most and those of 64 rows more than one, few of them share a
+ *  unit, and 128 rows take less (1000 x 2000 x 300 dots 27.3 and 27.9, angular 30.8 and 32.2; 256 x 8000 x 300 28.3 and 29.4,
+ *  31.8 and 33.5), but for dot products up to 256 values (500 x 4090 x 200 23.8 and 21.9). All pairs lose by 64 rows (3000 x
+ *  1000: 249, 261, 225, 348). */
 int f32_tile_rows(WideArgs const &g) {
-    static TileCost const shallow[] = {{128, 8.2f}, {64, 4.05f}, {32, 2.75f}, {16, 2.6f}};
+    static TileCost const shallow[] = {{64, 4.05f}, {32, 2.75f}, {16, 2.6f}};
     static TileCost const deep[] = {{128, 8.2f}, {64, 4.2f}, {32, 2.75f}, {16, 2.6f}};
     static TileCost const pairs[] = {{128, 8.2f}, {32, 2.3f}, {16, 2.0f}};
     if (g.tri_mask) return cheapest_tile(g, pairs);
-    return g.k_padded <= 512 ? cheapest_tile(g, shallow) : cheapest_tile(g, deep);
+    if (g.k_padded > 512) return cheapest_tile(g, deep);
+    int const rows = cheapest_tile(g, shallow);
+    uint64_t const units = compute_unit_count() > 0 ? compute_unit_count() : 256, columns = g.n_padded / kWideTile;
+    bool const one_round_of_tall = (g.m + 127) / 128 * columns <= units && (g.m + 63) / 64 * columns > units;
+    return rows == 64 && one_round_of_tall && (g.metric || g.k_padded > 256) ? 128 : rows;
 }
 
 __global__ __launch_bounds__(256) void fill_wide_kernel(uint8_t *c, uint32_t m, uint32_t n, uint64_t c_stride, uint64_t bits,
