@@ -154,8 +154,8 @@ int nk_hip_symmetric_static_async(int dtype, int metric, void const *vectors, si
 int nk_hip_fill_rows_async(void *c, size_t m, size_t n, size_t c_stride, uint32_t value, void *stream);
 
 /** TEST HOOK, not part of the product interface: forces the tile shape of the calling thread's launches (0 = the
- *  heuristic picks; 1..5 = 256x256, 128x256, 128x128, 64x128, 128x512; bit 7: a forced shape may still split a
- *  triangle; bits 8..27: spread of the workgroups' start times in 10 ns ticks, plus one; bits 28..29: 1 = outputs
+ *  heuristic picks; 1..6 = 256x256, 128x256, 128x128, 64x128, 128x512 (e2m3 only), 32x128 (a triangle takes 64x128 in
+ *  its place); bit 7: a forced shape may still split a triangle; bits 8..27: spread of the workgroups' start times in 10 ns ticks, plus one; bits 28..29: 1 = outputs
  *  stored past the caches, 2 = through them, whatever the alignment of C; bit 30: A is staged through registers also
  *  where it would go straight into LDS). The tests use it to run every shape, both kinds of store and both kinds of
  *  staging over the same cases; thread-local, so it never reaches another thread's calls. */

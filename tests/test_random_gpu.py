@@ -4,7 +4,8 @@ larger arrays (row pitches that are not multiples of 16 or 4 bytes, first elemen
 oracle's restatement of the serial kernels. Integers and the two wide types bit for bit; the other floats through the
 gate of tests/test_dots_gpu.py (mean error against the f64 truth at most twice the serial kernel's, NaN / Inf masks
 identical). The shapes straddle every tile edge and every path through the kernels: the pipelined loop with and
-without tail masks, the guarded loop for rows that are not dword-aligned, depths from 1 to a few stages.
+without tail masks and with shifted loads for rows that are not dword-aligned, the guarded loop for such rows of fewer
+than four stages, depths from 1 to a few stages.
 `NK_RANDOM_CASES` (default 10 per type) and `NK_RANDOM_SEED` (default 7000) widen or move the sample.
 """
 import os

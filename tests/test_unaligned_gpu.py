@@ -29,9 +29,12 @@ def values_of(dtype, rows, cols, rng):
 
 
 def placed(values, pad, offset):
-    """The same values on the GPU, `offset` values into rows that are `pad` values longer."""
+    """The same values on the GPU, `offset` values into rows that are `pad` values longer. What lies around them is NaN in
+    the float types (0x7F is one of both fp8 types): times the zeros that an image's depth is padded with, anything else
+    would vanish, whether or not the kernel masks what it reads past a row's end."""
     rows, cols = values.shape
-    whole = torch.full((rows, cols + pad + offset), 3, dtype=values.dtype).to(DEV)
+    around = float("nan") if values.dtype.is_floating_point else 0x7F
+    whole = torch.full((rows, cols + pad + offset), around, dtype=values.dtype).to(DEV)
     view = whole[:, offset:offset + cols]
     view.copy_(values)
     return view
@@ -67,6 +70,50 @@ def test_unaligned_rows_give_the_aligned_bits(dtype, config):
                 for metric in metrics:
                     got = CALLS[metric](placed(a, pad, offset), packed)
                     assert same(got, expected[metric]), f"{dtype} {metric} {m}x{n}x{cols} pad {pad} offset {offset}"
+        finally:
+            nk.library().nk_hip_set_tile_config(0)
+
+
+# Many tiles for every workgroup (the largest device-resident grid is 1024 workgroups; the fewest tiles here are 2193 of
+# 128 x 256): what a tile's last stages fetch is the next tile's first stages, shifted as its base asks, and the sums that
+# the staging keeps (u8's rows, the distances' squares) change sets with every tile.
+@pytest.mark.parametrize("dtype", NARROWER)
+@pytest.mark.parametrize("config", [0, 2, 3, 4, 6])
+def test_unaligned_rows_across_tiles(dtype, config):
+    rng = np.random.default_rng(33)
+    m, n = 2100, 33_001
+    cols = 125 if dtype == "u1" else 515
+    a, b = values_of(dtype, m, cols, rng), values_of(dtype, 4099, cols, rng)
+    packed = nk.dots_pack(b.to(DEV).repeat(-(-n // 4099), 1)[:n].contiguous(), dtype)
+    for metric in ["dots"] if dtype == "u1" else list(CALLS):
+        nk.library().nk_hip_set_tile_config(config)
+        try:
+            expected = CALLS[metric](aligned(a), packed)
+            for pad, offset in ((0, 0), (1, 1)):
+                got = CALLS[metric](placed(a, pad, offset), packed)
+                assert same(got, expected), f"{dtype} {metric} config {config} pad {pad} offset {offset}"
+        finally:
+            nk.library().nk_hip_set_tile_config(0)
+
+
+# Rows of one or two stages, where the pipeline starts anew with every tile: one byte, under, at and over one stage of 128
+# bytes (16 of the bits), the last odd length before four stages; one tile, and many for every workgroup.
+@pytest.mark.parametrize("dtype", NARROWER)
+@pytest.mark.parametrize("config", [0, 1, 2, 3, 4, 6])
+def test_unaligned_rows_of_two_stages(dtype, config):
+    rng = np.random.default_rng(34)
+    width = api.DTYPES[dtype][1]
+    stage = {"u1": 16, "i4": 64, "u4": 64, "e4m3": 64, "e5m2": 64, "e3m2": 64}.get(dtype, 128 // width)  # values stored in a row of one
+    for m, n, cols in ((1, 1, 1), (33, 70, 5), (67, 130, stage - 1), (130, 257, stage), (257, 300, stage + 1), (2100, 33_001, 2 * stage - 1)):
+        a, b = values_of(dtype, m, cols, rng), values_of(dtype, min(n, 4099), cols, rng)
+        packed = nk.dots_pack(b.to(DEV).repeat(-(-n // 4099), 1)[:n].contiguous(), dtype)
+        nk.library().nk_hip_set_tile_config(config)
+        try:
+            for metric in ["dots"] if dtype == "u1" else list(CALLS):
+                expected = CALLS[metric](aligned(a), packed)
+                for pad, offset in ((0, 0), (0, 1), (2, 1), (1, 3)):
+                    got = CALLS[metric](placed(a, pad, offset), packed)
+                    assert same(got, expected), f"{dtype} {metric} {m}x{n}x{cols} config {config} pad {pad} offset {offset}"
         finally:
             nk.library().nk_hip_set_tile_config(0)
 
