@@ -1134,9 +1134,9 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     uint32_t const *col_norms = col_terms + (uint64_t)g.n_tiles * kTileRows;
 
     uint32_t const stages = g.k_chunks / kStageChunks;
-    // Stages the pipelined loop takes: all of them when A is at least dword-aligned, which is all that
-    // multi-dword global loads need. (readfirstlane: the value is uniform, and it must stay in a scalar register
-    // because the stage offsets of the buffer loads derive from it.)
+    // Stages the pipelined loop takes: all of them when A is at least dword-aligned, which is all that multi-dword
+    // global loads need, or read by shifted loads; none otherwise. (readfirstlane: the value is uniform, and it must
+    // stay in a scalar register because the stage offsets of the buffer loads derive from it.)
     uint32_t const fast = __builtin_amdgcn_readfirstlane(SHIFTED || g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) ? stages : 0);
     uint32_t const xr = T::kUnsigned ? 0x80808080u : 0u;
     uint32_t const a_pos = tid & 7;
@@ -2145,7 +2145,8 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             else if (best < 3 && tiles_of(args, 3) >= 256) best = 3;
         }
         // Two accumulator sets do not fit the 256 x 256 tile, and neither do the fifth dwords of shifted loads (99 registers
-        // of the i8 kernel spill).
+        // of the i8 kernel spill). In the 128 x 256 tile they cost the integers nothing; of the types with two accumulator
+        // sets 37 to 68 registers spill there, where the kernels for aligned ragged rows spill 0 to 58.
         if ((T::kChunked || needs_shift<T>(args)) && best == 1) best = 2;
         // Two stages: the pipeline starts anew with every tile, the large tiles' kernels spill around that (e4m3 and e5m2 80
         // registers at 128 x 256, 13 before they held a loop for odd rows), and the stores are nearly all of the work. Measured,
@@ -2175,11 +2176,12 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // time of 64 x 128 (of the largest tile for the deeper products) over that of the tile taken, mean and least: floats of 5
         // to 16 stages 1.22 and 0.79, deeper 1.08 and 0.85; integers of 2 stages 1.09 and 0.80, of 3 and 4 1.22 and 0.96, of 5
         // to 8 1.32 and 0.90, deeper 1.15 and 0.80 (16 in 1000 of all shapes lose more than 3 per cent); of the best tile at
-        // each, 0.96. Some of them (us): i8 1000 x 500,009 x 304 1226 through 64 x 128 and 972 through
+        // each, 0.96. Those launches wrote the same C over and over; going round three sets of operands and results, 8000 random
+        // shapes, the mean is 1.06 and 23 in 1000 lose more than 3 per cent. Some of them (us): i8 1000 x 500,009 x 304 1226 through 64 x 128 and 972 through
         // 128 x 256, 1024 x 1,000,001 x 768 2855 and 1879 through 256 x 256 (300 x 524,289 x 768, which leaves a quarter of the
         // tall tiles empty, 377 through them and 287 through 128 x 256); i8 1024 x 204,801 x 1500 (an image of 300 MiB) 692 past
-        // the caches, 566 through 256 x 256, but 1024 x 107,521 x 1500 (158 MiB) 288 and 306; bf16 2400 x 45,857 x 900 415
-        // through 64 x 128, 337 through 128 x 128 past the caches, 476 through 128 x 256, whose kernel for ragged depths of
+        // the caches, 566 through 256 x 256, but 1024 x 107,521 x 1500 (158 MiB) 288 and 306; bf16 2400 x 45,857 x 900 433
+        // through 64 x 128, 354 through 128 x 128 past the caches, 533 through 128 x 256, whose kernel for ragged depths of
         // 16-bit floats and for shifted rows spills.
         uint32_t const limit = T::kChunked ? 16 : 8;
         if (unaligned_rows_of_c(args) && best < 4 && depth_stages <= 2 * limit) {
