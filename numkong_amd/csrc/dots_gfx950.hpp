@@ -99,6 +99,7 @@ hipError_t launch_f16(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
 hipError_t launch_e4m3(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
 hipError_t launch_e5m2(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
 hipError_t launch_e2m3(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
+hipError_t launch_e2m3_deep(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
 hipError_t launch_e3m2(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
 hipError_t launch_i4(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
 hipError_t launch_u4(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle);
@@ -598,6 +599,7 @@ constexpr bool kHalfChunked = true;
 #endif
 
 struct I8 {
+    static constexpr bool kDeepOnly = false; // in use for rows of many stages only
     static constexpr bool kChunked = false; // fold the accumulator into a second one every few stages
     static constexpr int kSrcChunk = 16; // source bytes of A behind one 16-byte LDS chunk
     static constexpr int kImageChunk = kChunkBytes; // bytes of one row's chunk in the image
@@ -638,6 +640,7 @@ struct U8 : I8 {
     }
 };
 struct BF16 {
+    static constexpr bool kDeepOnly = false;
     static constexpr bool kChunked = kHalfChunked;
     static constexpr int kSrcChunk = 16; // source bytes of A behind one 16-byte LDS chunk
     static constexpr int kImageChunk = kChunkBytes;
@@ -676,6 +679,7 @@ struct BF16 {
     }
 };
 struct F16 {
+    static constexpr bool kDeepOnly = false;
     static constexpr bool kChunked = kHalfChunked;
     static constexpr int kSrcChunk = 16; // source bytes of A behind one 16-byte LDS chunk
     static constexpr int kImageChunk = kChunkBytes;
@@ -758,6 +762,7 @@ struct E2M3 : I8 {
 /** e2m3 rows too deep for exact i32 sums (see kE2M3IntegerDepth) run widened to f16 like e3m2: every e2m3 value is an
  *  f16 value, the smallest non-zero one 1/8. */
 struct E2M3Deep : F16 {
+    static constexpr bool kDeepOnly = true;
     static constexpr bool kChunked = true;
     static constexpr int kDtype = kE2M3;
     static constexpr int kSrcChunk = 8;
@@ -917,6 +922,8 @@ struct Totals {
 #pragma unroll
         for (int v = 0; v < 16; ++v) value[i][j][v] = 0;
     }
+    /** A block's running sum into its total; the sum is left as it is (the next product starts it from zero). */
+    __device__ __forceinline__ void fold_block(acc_t const (&acc)[TM][TN], int i, int j) { value[i][j] += acc[i][j]; }
     __device__ __forceinline__ auto finish(acc_t const (&acc)[TM][TN], int i, int j, int v) const {
         return acc[i][j][v] + value[i][j][v];
     }
@@ -926,6 +933,7 @@ struct Totals<acc_t, TM, TN, false> {
     __device__ __forceinline__ void clear() {}
     __device__ __forceinline__ void fold(acc_t (&)[TM][TN]) {}
     __device__ __forceinline__ void clear_block(int, int) {}
+    __device__ __forceinline__ void fold_block(acc_t const (&)[TM][TN], int, int) {}
     __device__ __forceinline__ auto finish(acc_t const (&acc)[TM][TN], int i, int j, int v) const { return acc[i][j][v]; }
 };
 
@@ -1095,8 +1103,15 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  i8 3 x 162,699 x 4327 1019 -> 155 us, u8 symmetric 6391 x 7163 1625 -> 252 us, f16 symmetric angular 2947 x 3033
  *  674 -> 113 us; with B packed in the call as well, whose odd rows were read byte by byte: bf16 959 x 74,207 x 4307
  *  6505 -> 1372 us, i8 45 x 610,671 x 391 433 -> 230 us.
+ *
+ *  FOLDS: the two-accumulator types, depths under 32 stages, where sums go into their totals every two stages, after every
+ *  trip of the loop. Then there is no branch around the fold, and no clearing behind it: the next trip's first MFMA of a block
+ *  takes a zero operand and stands right behind the 16 additions that empty the block, so that the matrix pipe works on one
+ *  block while the next is emptied. With the general form a fold of 128 x 256 results was 256 vector operations between
+ *  64 MFMAs. Whole calls, before and now (us): bf16 8192 x 8192 x 1024 184 and 172, 4096 x 4096 x 768 57 and 52, 1000 x 100,000 x
+ *  300 263 and 235; e3m2 the same 224 and 193; all pairs of 8192 x 768 119 and 109; the same bits.
  */
-template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false>
+template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false, bool FOLDS = false>
 __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChunked ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
     constexpr int BM = TM * 32;
@@ -1404,14 +1419,16 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     };
     // The same for the first k-step of a tile: its MFMAs start the sums from a zero operand, so that no accumulator is
     // ever cleared (the totals of the chunked types are, a block's in front of its MFMA).
-    auto multiply_fresh = [&](auto slot_tag, auto q_tag) {
+    auto multiply_fresh = [&](auto slot_tag, auto q_tag, auto fold_tag) {
         constexpr int slot = decltype(slot_tag)::value, q = decltype(q_tag)::value;
+        constexpr bool fold = decltype(fold_tag)::value != 0; // in the middle of a tile: the running sum goes into the total
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             v4i const b = T::operand_b(b_reg[slot][j][q]);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                total.clear_block(i, j);
+                if constexpr (fold) total.fold_block(acc, i, j);
+                else total.clear_block(i, j);
                 T::mma_fresh(acc[i][j], af[q & 1][i], b);
             }
         }
@@ -1487,7 +1504,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     // are constants and which the host guarantees two or three more: see stage_direct).
     auto stage = [&](auto parity_tag, uint32_t s, auto entry_tag, auto inside_tag) __attribute__((always_inline)) {
         constexpr int P = decltype(parity_tag)::value;
-        constexpr int entry = decltype(entry_tag)::value; // 0: in the middle of a sum; 2: the first stage of a tile
+        constexpr int entry = decltype(entry_tag)::value; // 0: in the middle of a sum; 1: a fold in front of it; 2: the first stage of a tile
         constexpr int inside = ACROSS ? decltype(inside_tag)::value : 0; // (without ACROSS a tile may have two stages only)
         // vector operations behind each MFMA of the k-steps that widen in place: their share of half the chunks
         constexpr int kSpread = T::kPrewiden ? (kLoads * 28 + TM * TN - 1) / (TM * TN) : 0;
@@ -1496,11 +1513,11 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         TileView const &a2 = wrap2 ? nxt : cur, &a3 = wrap3 ? nxt : cur, &b2 = a2;
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<P>(), slot_c<1>(), slot_c<1>());
-        if constexpr (entry == 2) multiply_fresh(slot_c<P>(), slot_c<0>());
+        if constexpr (entry != 0) multiply_fresh(slot_c<P>(), slot_c<0>(), slot_c<entry == 1>());
         else multiply(slot_c<P>(), slot_c<0>());
         load_b(b2, s2, slot_c<P>(), slot_c<0>()), load_a(a2, s2, slot_c<P>(), slot_c<2>());
         if constexpr (T::kPrewiden) prewiden(slot_c<P ^ 1>(), s + 1 < fast ? s + 1 : 0u, slot_c<0>());
-        if constexpr (entry == 2 && kChunked) schedule_fresh_k_step();
+        if constexpr (entry != 0 && kChunked) schedule_fresh_k_step();
         else schedule_k_step(slot_c<0>(), slot_c<kSpread>());
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<P>(), slot_c<2>(), slot_c<0>());
@@ -1599,10 +1616,10 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         TileView const &b2 = wrap2 ? nxt : cur, &a3 = wrap3 ? nxt : cur;
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<R>(), slot_c<1>(), slot_c<1>());
-        if constexpr (entry == 2) multiply_fresh(slot_c<P>(), slot_c<0>());
+        if constexpr (entry != 0) multiply_fresh(slot_c<P>(), slot_c<0>(), slot_c<entry == 1>());
         else multiply(slot_c<P>(), slot_c<0>());
         load_b(b2, s2, slot_c<P>(), slot_c<0>()), fetch_a(a3, s3, slot_c<R + 3>(), slot_c<0>());
-        if constexpr (entry == 2 && kChunked) schedule_fresh_k_step();
+        if constexpr (entry != 0 && kChunked) schedule_fresh_k_step();
         else schedule_direct_k_step();
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<R>(), slot_c<2>(), slot_c<0>());
@@ -1717,11 +1734,11 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
                 else {
                     stage(slot_c<0>(), 0u, slot_c<2>(), slot_c<2>()); // (with ACROSS at least four stages: the host checked)
                     stage(slot_c<1>(), 1u, slot_c<0>(), slot_c<1>());
-                    fold_when_due();
+                    if constexpr (!FOLDS) fold_when_due();
                     for (uint32_t s = 2; s < fast; s += 2) {
-                        stage(slot_c<0>(), s, slot_c<0>(), slot_c<0>());
+                        stage(slot_c<0>(), s, slot_c<FOLDS>(), slot_c<0>());
                         stage(slot_c<1>(), s + 1, slot_c<0>(), slot_c<0>());
-                        fold_when_due();
+                        if constexpr (!FOLDS) fold_when_due();
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -2034,10 +2051,19 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
         if (norms && whole) kernel = dots_packed_kernel<T, TM, TN, true, true, true>;
     }
     else if (norms) return hipErrorInvalidValue;
+    // Shallow products of the two-accumulator types fold after every trip of the loop: no branch, and nothing to clear.
+    bool folds = false;
+    if constexpr (T::kChunked && !T::kDeepOnly && TM * TN > 1) {
+        folds = !direct && (across || shifted) && g.chunk_stages == 2;
+        if (folds && !norms) kernel = shifted ? dots_packed_kernel<T, TM, TN, true, false, false, false, true, true>
+                                      : whole ? dots_packed_kernel<T, TM, TN, true, false, true, false, false, true> : dots_packed_kernel<T, TM, TN, true, false, false, false, false, true>;
+        if (folds && norms) kernel = shifted ? dots_packed_kernel<T, TM, TN, true, true, false, false, true, true>
+                                     : whole ? dots_packed_kernel<T, TM, TN, true, true, true, false, false, true> : dots_packed_kernel<T, TM, TN, true, true, false, false, false, true>;
+    }
     // Persistent grid: as many workgroups as fit on the device at once (queried once per kernel; threads that
     // ask at the same time store the same number).
-    static std::atomic<int> resident_of[11];
-    std::atomic<int> &slot = resident_of[shifted ? (norms ? 10 : 9) : direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)];
+    static std::atomic<int> resident_of[22];
+    std::atomic<int> &slot = resident_of[(shifted ? (norms ? 10 : 9) : direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)) + (folds ? 11 : 0)];
     int resident = slot.load(std::memory_order_relaxed);
     if (!resident) {
         int per_cu = 0;
