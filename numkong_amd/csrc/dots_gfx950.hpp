@@ -1111,8 +1111,10 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  64 MFMAs. Whole calls, before and now (us): bf16 8192 x 8192 x 1024 184 and 172, 4096 x 4096 x 768 57 and 52, 1000 x 100,000 x
  *  300 263 and 235; e3m2 the same 224 and 193; all pairs of 8192 x 768 119 and 109; the same bits.
  */
+// (Workgroups per compute unit: 128 x 128 with two accumulator sets needs 232 to 256 registers, so two of them fit; left to one, the
+// compiler takes 300. bf16 angular 1024 x 262,144 x 768 768 us through 64 x 128, the best before, and 684.)
 template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false, bool FOLDS = false>
-__global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 && !T::kChunked ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
     constexpr int BM = TM * 32;
     constexpr int NT = 256;
@@ -2130,6 +2132,43 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         Choice(int config, uint32_t store_policy = 0) : config(config), store_policy(store_policy) {}
     };
     auto past = [](int config) { return Choice(config, 1); };
+    // Where storing C is most of the work, what counts is how much of it there is, against the 256 MiB of the last-level
+    // cache above all, and whether its rows start on lines. Drawn through 980 random shapes (33 to 8192 rows, depths of 1 to 64
+    // stages, C of 4 to 2200 MiB, half of them with rows off the lines; whole calls that go round three sets of operands and
+    // results), every tile at each. Some of them (us, before and now): bf16 208 x 60,160 x 485 71 and 43 (64 x 128), e5m2 150 x
+    // 136,704 x 320 84 and 63 (64 x 128), i8 angular 371 x 34,739 x 1600 154 and 58 (64 x 128), bf16 3439 x 38,656 x 826 382 and
+    // 316 (128 x 128: two workgroups of it fit a compute unit, and the kernels for depths of no whole stage spill at 128 x 256).
+    // 0: nothing here applies.
+    auto by_bytes_of_c = [&](GemmArgs const &args) -> int {
+        uint32_t const stages = args.k_chunks / kStageChunks;
+        uint64_t const mib = ((uint64_t)args.m * args.n * 4) >> 20;
+        bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0, norms = args.metric != 0;
+        bool const whole = args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
+        if (args.m <= 64) return 0;
+        if (!lines) {
+            if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : 3;
+            if (norms) return stages > 16 && mib >= 96 ? 3 : 0;
+            if (T::kChunked) return (stages > 4 && mib >= 32 && mib < 96) || (stages > 16 && mib >= 32 && mib < 256) ? 3 : 0;
+            return stages <= 16 && mib < 96 ? 4 : 0;
+        }
+        if (T::kChunked && norms) {
+            return stages > 16 && stages < 32 && mib >= 64 ? 3 : 0;
+        }
+        if (T::kChunked) {
+            if (mib < 96) return stages > 2 && (stages <= 16 || (stages < 32 && !whole)) ? 4 : 0;
+            if (stages <= 4) return stages > 2 ? 4 : 0;
+            return stages <= 16 || (stages < 32 && !whole) ? 3 : 0;
+        }
+        if (!norms) {
+            if (stages > 16) return 0;
+            if (mib < 96) return stages <= 8 || mib >= 32 ? 4 : 0; // (i8 2048^3 28.0 us through 128 x 128, 28.8 through 64 x 128)
+            if (stages <= 4) return stages > 2 ? 4 : 0;
+            return stages <= 8 && mib < 512 ? 3 : 0;
+        }
+        if (stages > 16) return stages < 32 && mib < 96 ? 4 : 0;
+        if (mib < 256) return stages <= 8 || mib < 96 ? 4 : 3;
+        return stages <= 4 ? 4 : 0;
+    };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
     auto choose = [&](GemmArgs const &args, int first) -> Choice {
         uint32_t const depth_stages = args.k_chunks / kStageChunks;
@@ -2153,6 +2192,8 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // against 25.2); a deep one gains as long as the smaller tiles fit one round (bf16 1024^3 26.3 against 24.8, angular
         // 29.3 against 26.1, but 64 x 30,000 x 4096 54 against 62).
         if (!triangle && tiles_of(args, 4) < 256 && (depth_stages <= 8 || tiles_of(args, 6) <= 256)) return 6;
+        if (!triangle && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024)
+            if (int const config = by_bytes_of_c(args); config && tiles_of(args, config) >= 256) return config;
         // Distances over a shallow depth are bound by the epilogue (a finaliser and a store per output): two
         // workgroups per CU of 128 x 128 tiles overlap it with the other's loop better than one large tile does
         // (measured on 1024 x 1,048,576 x 768: 2.17 against 2.33 ms angular, 1.98 against 2.07 ms euclidean).
