@@ -82,6 +82,7 @@ struct GemmArgs {
     uint32_t store_policy; // 0: by the alignment of C's rows; 1: past the caches; 2: through them
     uint32_t tile_count;       // tiles_m * tiles_n, or the length of the list
     uint32_t const *tile_list; // (tile row, tile column) pairs in walking order, or NULL for the full grid
+    uint32_t strip_tiles;      // dots_strips_kernel: tiles that a workgroup walks along a strip (tiles_n counts strips)
 };
 
 /** Scratch memory of a triangular grid: the first tile of every band, then the list itself. */
@@ -1961,11 +1962,359 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     }
 }
 
+/**
+ *  Shallow products, strip by strip. A workgroup of 8 wavefronts keeps the (32*TM) rows of its part of A in LDS, whole depth,
+ *  and walks along the columns of C, 256 at a time (a 32-column tile of the image per wavefront). What a tile costs in
+ *  dots_packed_kernel besides its own columns (A fetched, masked, widened, its squares and bytes summed, a barrier every
+ *  stage) is done once per strip; the loop is B from the image into registers, A fragments from LDS and MFMAs, and the
+ *  wavefronts meet only to store.
+ *
+ *  B is fetched two stages ahead, across tiles, so that what a tile waits for was asked for before the tile before it was
+ *  stored (loads and stores of a wavefront complete in order).
+ *
+ *  Stores are whole 128-byte lines wherever the rows of C start. A partial line costs the memory a read and a write, and
+ *  a row's tile ends in the middle of one unless C is aligned to lines: 1000 x 500,009 results written as the accumulators
+ *  hold them, 128 bytes per row and instruction, take 1190 us past the caches and 600 through them, as whole lines 400 (the
+ *  same as rows on lines). Because a workgroup walks along its rows, what a tile lacks of its first line is what the tile
+ *  before it had left over of its last. A row's tile starts `skew` columns past a line; in LDS it starts at the same
+ *  position of a row of 256, and its last `skew` columns go around to the row's start. There the first line's missing columns
+ *  are filled in from `carried`, and the ones that went around wait there for the next tile.
+ */
+constexpr int kStripWaves = 8, kStripColumns = 32 * kStripWaves;
+template <class T, int TM, int METRIC, int BATCH>
+__global__ __launch_bounds__(64 * kStripWaves, 2) void dots_strips_kernel(GemmArgs g) {
+    typedef typename T::acc_t acc_t;
+    typedef typename T::norm_t norm_t;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) uint8_t global_u8_t;
+    typedef __attribute__((address_space(1))) uint32_t global_u32_t;
+    constexpr int BM = TM * 32, NT = 64 * kStripWaves;
+    constexpr int kStageLds = BM * kStageBytes;
+    constexpr int kSrcStage = kStageChunks * T::kSrcChunk;
+    constexpr int kImageTileChunk = kTileRows * T::kImageChunk;
+    constexpr bool kChunked = T::kChunked;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t strip_lds[];
+    uint32_t const stages = g.k_chunks / kStageChunks;
+    uint32_t *const stage_rows = (uint32_t *)(strip_lds + stages * kStageLds);    // BATCH rows of 256 results
+    uint32_t *const carried = stage_rows + BATCH * kStripColumns;                 // per row what its next line starts with
+    uint32_t *const row_terms = carried + BM * 32;                                 // as in dots_packed_kernel
+    uint32_t *const row_norms = row_terms + BM;
+    float *const row_factors = (float *)(row_norms + BM);
+
+    uint32_t const tid = threadIdx.x, lane = tid & 63;
+    uint32_t const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t const half = lane >> 5, col_in_tile = lane & 31;
+
+    PackedHeader const *header = (PackedHeader const *)g.bp;
+    bool const image_ok = header->magic == kMagic && header->version == kVersion &&
+                          header->dtype == (uint32_t)T::kDtype && header->n == g.n && header->k == g.k &&
+                          header->k_chunks == g.k_chunks && header->n_tiles == g.n_tiles;
+    uint8_t const *data = g.bp + sizeof(PackedHeader);
+    uint32_t const *col_terms = (uint32_t const *)(data + (uint64_t)g.n_tiles * g.k_chunks * kImageTileChunk);
+    uint32_t const *col_norms = col_terms + (uint64_t)g.n_tiles * kTileRows;
+    uint32_t const strip_columns = g.strip_tiles * kStripColumns;
+    if (!image_ok) { // the image was not packed for this call: the reference's error convention, all bits set
+        for (uint32_t unit = blockIdx.x; unit < g.tile_count; unit += gridDim.x) {
+            uint32_t tile_m, strip;
+            tile_of_block(unit, g, tile_m, strip);
+            for (uint32_t row = tile_m * BM; row < tile_m * BM + BM && row < g.m; ++row)
+                for (uint32_t at = tid; at < strip_columns; at += NT)
+                    if (strip * strip_columns + at < g.n) *(global_u32_t *)((global_u8_t *)g.c + (uint64_t)row * g.c_stride + (uint64_t)(strip * strip_columns + at) * 4) = 0xFFFFFFFFu;
+        }
+        return;
+    }
+
+    uint32_t a_frag[4]; // (lane l takes row l % 32 of each 32-row block and chunk 2q + l / 32)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t const r = lane & 31, c = 2 * q + (lane >> 5);
+        a_frag[q] = r * kStageBytes + ((c ^ ((r >> 1) & 7)) << 4);
+    }
+    uint32_t const tile_bytes = g.k_chunks * kImageTileChunk;
+    struct ImageView {
+        uint8_t const *b;
+        uint32_t bytes;
+    };
+    auto view_of = [&](uint32_t col0) { // (columns past the last tile: that tile once more, never stored)
+        uint32_t const tile = col0 / 32 < g.n_tiles ? col0 / 32 : g.n_tiles - 1;
+        uint64_t const left = (uint64_t)(g.n_tiles - tile) * tile_bytes;
+        return ImageView {data + (uint64_t)tile * tile_bytes, left < 0xFFFFFFFFull ? (uint32_t)left : 0xFFFFFFFFu};
+    };
+    v4i b_reg[2][4];
+    v4i af[2][TM];
+    acc_t acc[TM][1];
+    Totals<acc_t, TM, 1, kChunked> total;
+    auto load_b = [&](ImageView const &view, uint32_t s, auto slot_tag, auto q_tag) __attribute__((always_inline)) {
+        constexpr int slot = decltype(slot_tag)::value, q = decltype(q_tag)::value;
+        __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)view.b, 0, (int)view.bytes, 0x00020000);
+        uint32_t const offset = __builtin_amdgcn_readfirstlane(s * (kStageChunks * kImageTileChunk));
+        if constexpr (T::kImageChunk == 2)
+            b_reg[slot][q][0] = (int)(uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, lane * 2 + q * 2 * kImageTileChunk, offset, 0);
+        else
+            b_reg[slot][q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane * 16 + q * 2 * kImageTileChunk, offset, 0));
+    };
+    auto read_frags = [&](uint32_t stage_at, auto q_tag, auto parity_tag) __attribute__((always_inline)) {
+        constexpr int q = decltype(q_tag)::value, parity = decltype(parity_tag)::value;
+        uint8_t const *src = strip_lds + stage_at + a_frag[q];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) af[parity][i] = *(v4i const *)(src + i * 32 * kStageBytes);
+    };
+    auto multiply = [&](auto slot_tag, auto q_tag, auto entry_tag) __attribute__((always_inline)) {
+        constexpr int slot = decltype(slot_tag)::value, q = decltype(q_tag)::value, entry = decltype(entry_tag)::value;
+        v4i const b = T::operand_b(b_reg[slot][q]);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if constexpr (entry == 0) T::mma(acc[i][0], af[q & 1][i], b);
+            else {
+                if constexpr (entry == 1) total.fold_block(acc, i, 0);
+                else total.clear_block(i, 0);
+                T::mma_fresh(acc[i][0], af[q & 1][i], b);
+            }
+        }
+    };
+    auto schedule_k_step = [&](auto vector_tag) __attribute__((always_inline)) {
+        constexpr int vector = decltype(vector_tag)::value;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if constexpr (vector > 0) __builtin_amdgcn_sched_group_barrier(0x002, vector, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto meet = [&]() __attribute__((always_inline)) { // (orders LDS only: prefetched loads and stores stay in flight)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+
+    // Where in the LDS rows a lane's results go, in bytes, two to a register: 16 rows of each 32-row block, the same in all
+    // of them (32 rows further on a row's start has moved by whole lines).
+    uint32_t places[4][2];
+#pragma unroll
+    for (int quad = 0; quad < 4; ++quad)
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+            uint32_t const words = (uint32_t)((uint64_t)g.c >> 2) + (8 * quad + 4 * half + e) * (uint32_t)(g.c_stride >> 2);
+            uint32_t const even = ((words & 31) + 32 * wave + col_in_tile) & (kStripColumns - 1);
+            uint32_t const odd = (((words + (uint32_t)(g.c_stride >> 2)) & 31) + 32 * wave + col_in_tile) & (kStripColumns - 1);
+            places[quad][e / 2] = (even * 4 + half * (4 * 4 * kStripColumns)) | (odd * 4 + half * (4 * 4 * kStripColumns)) << 16;
+        }
+
+    for (uint32_t unit = blockIdx.x; unit < g.tile_count; unit += gridDim.x) {
+        uint32_t tile_m, strip;
+        tile_of_block(unit, g, tile_m, strip);
+        uint32_t const row0 = tile_m * BM, strip_col = strip * strip_columns;
+        if (strip_col >= g.n) continue;
+        // The part of A. Thread t takes chunk t % 8 of every stage of rows t / 8, t / 8 + 64, ...: the partial sums of a row
+        // are those of dots_packed_kernel, in the same order.
+        meet(); // (the strip before is done with the LDS)
+        {
+            uint32_t *const part_sums = stage_rows;           // (BM x 8 words)
+            norm_t *const part_norms = (norm_t *)carried;     // (BM x 8, at most 16 KiB: `carried` is as large)
+            uint32_t const a_pos = tid & 7;
+            for (uint32_t r = tid >> 3; r < (uint32_t)BM; r += NT / 8) {
+                bool const exists = row0 + r < g.m;
+                uint8_t const *source = g.a + (uint64_t)(exists ? row0 + r : g.m - 1) * g.a_stride + a_pos * T::kSrcChunk;
+                uint32_t sum = 0;
+                norm_t squares = 0;
+#pragma unroll 4
+                for (uint32_t s = 0; s < stages; ++s) {
+                    int64_t const left = (int64_t)g.k_src_bytes - (int64_t)s * kSrcStage - (int64_t)a_pos * T::kSrcChunk;
+                    int const valid = (int)(left > T::kSrcChunk ? T::kSrcChunk : (left < 0 ? 0 : left));
+                    v4i v = load_chunk_guarded<T::kSrcChunk>(source + (uint64_t)s * kSrcStage, valid, 0u);
+                    v4i const raw = v;
+                    if (T::kUnsigned) {
+                        sum += sum_bytes_u8(v);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) { // flip only bytes that exist: the zero padding stays zero
+                            int const rem = valid - 4 * w;
+                            v[w] ^= (int)(rem >= 4 ? 0x80808080u : (rem <= 0 ? 0u : (0x80808080u >> (8 * (4 - rem)))));
+                        }
+                    }
+                    v4i const wide = T::widen(v);
+                    if (METRIC != 0) squares += T::sumsq(raw, wide);
+                    *(v4i *)(strip_lds + s * kStageLds + r * kStageBytes + ((a_pos ^ ((r >> 1) & 7)) << 4)) = wide;
+                }
+                if (T::kUnsigned) part_sums[r * 8 + a_pos] = sum;
+                if (METRIC != 0) part_norms[r * 8 + a_pos] = squares;
+            }
+            meet();
+            if ((T::kUnsigned || METRIC != 0) && tid < BM) {
+                if (T::kUnsigned) {
+                    uint32_t sum = 0;
+#pragma unroll
+                    for (int part = 0; part < 8; ++part) sum += part_sums[tid * 8 + part];
+                    row_terms[tid] = sum * 128u;
+                }
+                if (METRIC != 0) {
+                    norm_t sum = 0;
+#pragma unroll
+                    for (int part = 0; part < 8; ++part) sum += part_norms[tid * 8 + part];
+                    uint32_t bits;
+                    if constexpr (sizeof(norm_t) == 8) bits = __builtin_bit_cast(uint32_t, (float)sum);
+                    else bits = (uint32_t)sum;
+                    row_norms[tid] = __builtin_bit_cast(uint32_t, norm_as_f32<T>(bits));
+                    row_factors[tid] = refined_rsqrt(norm_as_f32<T>(bits));
+                }
+            }
+            meet();
+        }
+
+        ImageView cur = view_of(strip_col + 32 * wave);
+        auto load_stage = [&](auto slot_tag) __attribute__((always_inline)) {
+            constexpr int slot = decltype(slot_tag)::value;
+            load_b(cur, slot, slot_tag, slot_c<0>()), load_b(cur, slot, slot_tag, slot_c<1>());
+            load_b(cur, slot, slot_tag, slot_c<2>()), load_b(cur, slot, slot_tag, slot_c<3>());
+        };
+        load_stage(slot_c<0>()), load_stage(slot_c<1>());
+        auto column_at = [&](uint32_t col0) { return (col0 / 32 < g.n_tiles ? col0 / 32 : g.n_tiles - 1) * kTileRows + col_in_tile; };
+        uint32_t col_term = 0, col_norm = 0;
+        if (T::kUnsigned) col_term = col_terms[column_at(strip_col + 32 * wave)];
+        if (METRIC != 0) col_norm = col_norms[column_at(strip_col + 32 * wave)];
+        read_frags(0, slot_c<0>(), slot_c<0>());
+
+        for (uint32_t tile = 0; tile < g.strip_tiles; ++tile) {
+            uint32_t const tile_col = strip_col + tile * kStripColumns;
+            if (tile_col >= g.n + 32) break; // (nothing left, not even of a last line; uniform)
+            uint32_t const next_col = tile_col + kStripColumns + 32 * wave;
+            ImageView const nxt = view_of(next_col);
+            auto stage = [&](auto slot_tag, uint32_t s, auto entry_tag) __attribute__((always_inline)) {
+                constexpr int entry = decltype(entry_tag)::value;
+                bool const wrap = s + 2 >= stages;
+                uint32_t const ahead = wrap ? s + 2 - stages : s + 2;
+                ImageView const &from = wrap ? nxt : cur;
+                uint32_t const here = s * kStageLds, after = s + 1 < stages ? here + kStageLds : 0;
+                __builtin_amdgcn_sched_barrier(0);
+                read_frags(here, slot_c<1>(), slot_c<1>());
+                multiply(slot_tag, slot_c<0>(), entry_tag);
+                load_b(from, ahead, slot_tag, slot_c<0>());
+                schedule_k_step(slot_c<kChunked && entry != 0 ? 16 : 0>());
+                read_frags(here, slot_c<2>(), slot_c<0>());
+                multiply(slot_tag, slot_c<1>(), slot_c<0>());
+                load_b(from, ahead, slot_tag, slot_c<1>());
+                schedule_k_step(slot_c<0>());
+                read_frags(here, slot_c<3>(), slot_c<1>());
+                multiply(slot_tag, slot_c<2>(), slot_c<0>());
+                load_b(from, ahead, slot_tag, slot_c<2>());
+                schedule_k_step(slot_c<0>());
+                read_frags(after, slot_c<0>(), slot_c<0>());
+                multiply(slot_tag, slot_c<3>(), slot_c<0>());
+                load_b(from, ahead, slot_tag, slot_c<3>());
+                schedule_k_step(slot_c<0>());
+            };
+            stage(slot_c<0>(), 0u, slot_c<2>());
+            stage(slot_c<1>(), 1u, slot_c<0>());
+            for (uint32_t s = 2; s < stages; s += 2) { // (two-accumulator types: the sums go into the totals every two stages)
+                stage(slot_c<0>(), s, slot_c<kChunked ? 1 : 0>());
+                stage(slot_c<1>(), s + 1, slot_c<0>());
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
+            uint32_t const my_term = col_term, my_norm = col_norm;
+            if (T::kUnsigned) col_term = col_terms[column_at(next_col)]; // (asked for in front of the stores)
+            if (METRIC != 0) col_norm = col_norms[column_at(next_col)];
+
+            // Buffer stores: rows past the last one lie behind the descriptor's end, and so does the offset of a column that is
+            // not to be stored. (All of the offset is the lane's: the range check takes a scalar offset off the
+            // descriptor's size, which rows past the end would make negative.)
+            typedef __attribute__((address_space(4))) GemmArgs const late_args_t;
+            late_args_t *late = (late_args_t *)__builtin_amdgcn_kernarg_segment_ptr();
+            asm volatile("" : "+s"(late));
+            constexpr int kRowLanes = NT / BATCH; // threads that store a row
+            float const col_value = METRIC != 0 ? norm_as_f32<T>(my_norm) : 0.0f;
+            float const col_factor = METRIC == 1 ? refined_rsqrt(col_value) : 0.0f;
+            uint32_t const row_step = (uint32_t)late->c_stride, n = late->n;
+            uint32_t const words = (uint32_t)((uint64_t)late->c >> 2), step = row_step >> 2;
+            constexpr uint32_t kNowhere = 0x80000000u; // (the host checks that a tile's rows end below it)
+            uint8_t *const c_tile = late->c + (uint64_t)row0 * late->c_stride + (uint64_t)tile_col * 4 - 128;
+            uint64_t const left = (uint64_t)(late->m - row0 - 1) * late->c_stride + (uint64_t)n * 4 - (uint64_t)tile_col * 4 + 128;
+            __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)c_tile, 0, (int)(left < kNowhere ? (uint32_t)left : kNowhere), 0x00020000);
+            bool const inner = tile != 0 && tile_col + kStripColumns <= n;
+            bool const last = tile + 1 == g.strip_tiles;
+#pragma unroll
+            for (int batch = 0; batch < BM / BATCH; ++batch) {
+                int const i = batch * BATCH / 32;
+#pragma unroll
+                for (int quad = 0; quad < BATCH / 8; ++quad) {
+                    int const row_quad = (batch * BATCH % 32) / 8 + quad; // run of four rows per lane, of the 32 of block i
+                    int const rows_at = i * 32 + 8 * row_quad + 4 * half;
+                    v4i row_term4 = {0, 0, 0, 0}, row_norm4 = {0, 0, 0, 0};
+                    v4f row_factor4 = {0, 0, 0, 0};
+                    if (T::kUnsigned) row_term4 = *(v4i const *)&row_terms[rows_at];
+                    if (METRIC == 1) row_factor4 = *(v4f const *)&row_factors[rows_at];
+                    if (METRIC == 2) row_norm4 = *(v4i const *)&row_norms[rows_at];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        auto const element = total.finish(acc, i, 0, 4 * row_quad + e);
+                        uint32_t bits = finished_dot<T>(__builtin_bit_cast(uint32_t, element));
+                        if (T::kUnsigned) bits += (uint32_t)row_term4[e] + my_term;
+                        if (METRIC == 1) {
+                            bool cheap;
+                            float const quick = angular_from_factors<T>(bits, row_factor4[e], col_factor, &cheap);
+                            uint32_t result = __builtin_bit_cast(uint32_t, quick);
+                            if (__builtin_amdgcn_ballot_w64(!cheap) != 0) {
+                                int const row_bits = *(int const *)&row_norms[rows_at + e];
+                                uint32_t const full = distance_from_dot<T, 1>(bits, __builtin_bit_cast(float, row_bits), col_value);
+                                result = cheap ? result : full;
+                            }
+                            bits = result;
+                        }
+                        else if (METRIC == 2) {
+                            int const row_bits = row_norm4[e];
+                            bits = distance_from_dot<T, 2>(bits, __builtin_bit_cast(float, row_bits), col_value);
+                        }
+                        uint32_t const pair = places[row_quad][e / 2], place = e % 2 ? pair >> 16 : pair & 0xFFFFu;
+                        *(uint32_t *)((uint8_t *)(stage_rows + (8 * quad + e) * kStripColumns) + place) = bits;
+                    }
+                }
+                meet();
+                uint32_t const row_in_batch = tid / kRowLanes, row = batch * BATCH + row_in_batch;
+                uint32_t const skew = (words + row * step) & 31;
+                uint32_t const row_at = row * row_step;
+#pragma unroll
+                for (int part = 0; part < kStripColumns / 4 / kRowLanes; ++part) {
+                    uint32_t const chunk = part * kRowLanes + tid % kRowLanes; // sixteen bytes of the row's lines
+                    v4u const fresh = *(v4u const *)&stage_rows[row_in_batch * kStripColumns + 4 * chunk];
+                    v4u values = fresh;
+                    uint32_t const target = row_at + (32 - skew + 4 * chunk) * 4;
+                    int const column = (int)(tile_col - skew + 4 * chunk);
+                    if (part == 0 && chunk < 8) {
+                        v4u *const waiting = (v4u *)&carried[row * 32 + 4 * chunk];
+                        v4u const before = *waiting;
+                        *waiting = fresh;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) values[e] = 4 * chunk + e < skew ? before[e] : fresh[e];
+                        if (last) { // the end of the strip: what the last line of every row still lacks
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                bool const mine = 4 * chunk + e < skew && column + kStripColumns + e < (int)n;
+                                __builtin_amdgcn_raw_buffer_store_b32(fresh[e], rsrc, mine ? target + 4 * kStripColumns + 4 * e : kNowhere, 0, 0);
+                            }
+                        }
+                    }
+                    if (inner) __builtin_amdgcn_raw_buffer_store_b128(values, rsrc, target, 0, 2); // (2: `nt`)
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            bool const mine = column + e >= (int)strip_col && column + e < (int)n;
+                            __builtin_amdgcn_raw_buffer_store_b32(values[e], rsrc, mine ? target + 4 * e : kNowhere, 0, 0);
+                        }
+                    }
+                }
+                meet();
+            }
+        }
+    }
+}
+
 struct TileConfig {
     int tm, tn;
 };
-// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only; 6: full grids only).
-constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}, {1, 1}};
+// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only; 6: full grids only; 7: strips, dots_strips_kernel).
+constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}, {1, 1}, {4, 2}};
 constexpr int kConfigCount = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kTriangleConfigs = 6; // the shapes below this index serve triangular grids
 
@@ -2094,6 +2443,53 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     return hipGetLastError();
 }
 
+/** LDS of dots_strips_kernel. */
+constexpr size_t strips_lds_bytes(int bm, int batch, uint32_t stages) {
+    return (size_t)stages * bm * kStageBytes + (size_t)batch * kStripColumns * 4 + (size_t)bm * (32 + 3) * 4;
+}
+constexpr size_t kStripsLds = 160 << 10;
+template <class T>
+inline bool strips_possible(GemmArgs const &g) {
+    uint32_t const stages = g.k_chunks / kStageChunks;
+    return stages >= 2 && strips_lds_bytes(64, 16, stages) <= kStripsLds && (!T::kChunked || g.chunk_stages == 2) && g.n >= 128 &&
+           g.c_stride >= 4 * (uint64_t)g.n && g.c_stride < (1u << 24) - 1024;
+}
+template <class T, int TM, int BATCH>
+hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream) {
+    constexpr int BM = TM * 32;
+    void (*kernel)(GemmArgs) = dots_strips_kernel<T, TM, 0, BATCH>;
+    if constexpr (T::kDistances) {
+        if (g.metric == 1) kernel = dots_strips_kernel<T, TM, 1, BATCH>;
+        if (g.metric == 2) kernel = dots_strips_kernel<T, TM, 2, BATCH>;
+    }
+    else if (g.metric != 0) return hipErrorInvalidValue;
+    uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256; // (one workgroup's registers fill a compute unit)
+    // Strips per row of tiles: the number whose rounds of resident workgroups walk the fewest tiles, a tile's worth for
+    // starting and ending each strip included.
+    g.tiles_m = (g.m + BM - 1) / BM;
+    uint64_t const tiles = ((uint64_t)g.n + kStripColumns - 1) / kStripColumns;
+    uint64_t best = ~0ull, strips = 1;
+    uint64_t const from = resident / g.tiles_m ? resident / g.tiles_m : 1;
+    for (uint64_t s = from; s <= 4 * from + 4; ++s) {
+        uint64_t const length = (tiles + s - 1) / s, rounds = (g.tiles_m * s + resident - 1) / resident;
+        if (rounds * (length + 1) < best) best = rounds * (length + 1), strips = s;
+    }
+    g.strip_tiles = (uint32_t)((tiles + strips - 1) / strips);
+    g.tiles_n = (uint32_t)((tiles + g.strip_tiles - 1) / g.strip_tiles);
+    uint64_t const units = (uint64_t)g.tiles_m * g.tiles_n;
+    if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    g.tile_count = (uint32_t)units, g.tile_list = nullptr;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)(units < resident ? units : resident)), dim3(64 * kStripWaves),
+                       strips_lds_bytes(BM, BATCH, g.k_chunks / kStageChunks), stream, g);
+    return hipGetLastError();
+}
+template <class T>
+hipError_t launch_strips(GemmArgs &g, hipStream_t stream) {
+    uint32_t const stages = g.k_chunks / kStageChunks;
+    if (g.m > 64 && strips_lds_bytes(128, 32, stages) <= kStripsLds) return launch_strips_as<T, 4, 32>(g, stream); // (up to six stages)
+    return launch_strips_as<T, 2, 16>(g, stream);
+}
+
 template <class T>
 hipError_t launch_config(GemmArgs &g, hipStream_t stream, TriangleScratch const *triangle, int config,
                          int *slots_only = nullptr) {
@@ -2135,15 +2531,23 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // Where storing C is most of the work, what counts is how much of it there is, against the 256 MiB of the last-level
     // cache above all, and whether its rows start on lines. Drawn through 980 random shapes (33 to 8192 rows, depths of 1 to 64
     // stages, C of 4 to 2200 MiB, half of them with rows off the lines; whole calls that go round three sets of operands and
-    // results), every tile at each. Some of them (us, before and now): bf16 208 x 60,160 x 485 71 and 43 (64 x 128), e5m2 150 x
-    // 136,704 x 320 84 and 63 (64 x 128), i8 angular 371 x 34,739 x 1600 154 and 58 (64 x 128), bf16 3439 x 38,656 x 826 382 and
-    // 316 (128 x 128: two workgroups of it fit a compute unit, and the kernels for depths of no whole stage spill at 128 x 256).
+    // results), every tile and the strips at each: 1.19 of the rules below in the mean; of the best at each shape 0.99; 27
+    // lose more than 3 per cent (0.90 at the least). Some of them (us, before and now): u8 euclidean 1000 x 500,009 x 301
+    // 1165 and 610 (strips), i8 1024 x 204,801 x 220 298 and 151 (strips), f16 8192 x 8191 x 1000 289 and 230 (strips); with rows on
+    // lines bf16 208 x 60,160 x 485 71 and 43 (64 x 128), e5m2 150 x 136,704 x 320 84 and 63 (64 x 128), i8 angular 371 x
+    // 34,739 x 1600 154 and 58 (64 x 128), bf16 527 x 400,384 x 192 384 and 259 (strips), bf16 3439 x 38,656 x 826 382 and 316
+    // (128 x 128: two workgroups of it fit a compute unit, and the kernels for depths of no whole stage spill at 128 x 256).
     // 0: nothing here applies.
     auto by_bytes_of_c = [&](GemmArgs const &args) -> int {
         uint32_t const stages = args.k_chunks / kStageChunks;
         uint64_t const mib = ((uint64_t)args.m * args.n * 4) >> 20;
         bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0, norms = args.metric != 0;
         bool const whole = args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
+        bool strips = false;
+        if constexpr (!T::kDeepOnly) strips = strips_possible<T>(args) && stages <= 16;
+        // A strip has a start and an end to pay for: enough of C for many tiles to a strip, and what it saves (partial lines,
+        // the part of A staged with every tile) has to be a large part.
+        if (!lines && strips && mib >= (stages <= 2 ? 64 : 96)) return 7;
         if (args.m <= 64) return 0;
         if (!lines) {
             if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : 3;
@@ -2152,21 +2556,24 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             return stages <= 16 && mib < 96 ? 4 : 0;
         }
         if (T::kChunked && norms) {
+            if (strips && mib >= 256 && args.n >= 32768) return 7;
             return stages > 16 && stages < 32 && mib >= 64 ? 3 : 0;
         }
         if (T::kChunked) {
             if (mib < 96) return stages > 2 && (stages <= 16 || (stages < 32 && !whole)) ? 4 : 0;
+            if (strips && mib >= 256 && stages <= 8) return 7;
             if (stages <= 4) return stages > 2 ? 4 : 0;
             return stages <= 16 || (stages < 32 && !whole) ? 3 : 0;
         }
         if (!norms) {
             if (stages > 16) return 0;
             if (mib < 96) return stages <= 8 || mib >= 32 ? 4 : 0; // (i8 2048^3 28.0 us through 128 x 128, 28.8 through 64 x 128)
-            if (stages <= 4) return stages > 2 ? 4 : 0;
+            if (stages <= 4) return strips && mib >= 256 ? 7 : stages > 2 ? 4 : 0;
             return stages <= 8 && mib < 512 ? 3 : 0;
         }
         if (stages > 16) return stages < 32 && mib < 96 ? 4 : 0;
         if (mib < 256) return stages <= 8 || mib < 96 ? 4 : 3;
+        if (strips && (stages <= 2 || stages > 8 || (stages <= 4 && mib >= 512))) return 7;
         return stages <= 4 ? 4 : 0;
     };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
@@ -2193,7 +2600,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // 29.3 against 26.1, but 64 x 30,000 x 4096 54 against 62).
         if (!triangle && tiles_of(args, 4) < 256 && (depth_stages <= 8 || tiles_of(args, 6) <= 256)) return 6;
         if (!triangle && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024)
-            if (int const config = by_bytes_of_c(args); config && tiles_of(args, config) >= 256) return config;
+            if (int const config = by_bytes_of_c(args); config == 7 || (config && tiles_of(args, config) >= 256)) return config;
         // Distances over a shallow depth are bound by the epilogue (a finaliser and a store per output): two
         // workgroups per CU of 128 x 128 tiles overlap it with the other's loop better than one large tile does
         // (measured on 1024 x 1,048,576 x 768: 2.17 against 2.33 ms angular, 1.98 against 2.07 ms euclidean).
@@ -2289,6 +2696,11 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     };
     Choice const chosen = chosen_here ? choose(g, 1) : Choice(config);
     config = chosen.config, g.store_policy = chosen.store_policy;
+    if (config == 7) {
+        if constexpr (!T::kDeepOnly)
+            if (!triangle && strips_possible<T>(g)) return launch_strips<T>(g, stream);
+        config = 4;
+    }
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
     if (triangle && config >= kTriangleConfigs) config = 4;
     // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
