@@ -446,9 +446,10 @@ size_t nk_hip_dots_packed_size(int dtype, size_t n, size_t k) {
     return (size_t)g.total_bytes;
 }
 
-/** `terms`: also the per-column terms after the tiles (only the u8 product and the distances read them). */
+/** `terms`: also the per-column terms after the tiles (only the u8 product and the distances read them; 2: see pack_kernel).
+ *  `lists`: tile lists to be written by the same launch. */
 static int pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_stride, void *b_packed, void *stream_,
-                      bool terms) {
+                      int terms, TriangleGrids lists = {}) {
     hipStream_t stream = (hipStream_t)stream_;
     Geometry g;
     bool const wide = dtype == kF32 || dtype == kF64;
@@ -483,7 +484,7 @@ static int pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_str
         uint32_t const xr = dtype == kU8 ? 0x80808080u : 0u;
         // by how the source is widened and by what the image then holds (see pack_kernel)
         typedef void (*pack_fn)(uint8_t const *, uint64_t, uint32_t, uint64_t, uint32_t, uint32_t, uint8_t *, uint32_t *,
-                                uint32_t *, int, uint32_t, int, PackedHeader);
+                                uint32_t *, int, uint32_t, int, PackedHeader, TriangleGrids);
         pack_fn kernel = nullptr;
         switch (widen_kind_of(dtype, k)) {
         case 0: kernel = dtype == kI8 ? pack_kernel<0, 0> : (dtype == kU8 ? pack_kernel<0, 1> : (dtype == kBF16 ? pack_kernel<0, 2> : pack_kernel<0, 3>)); break;
@@ -496,8 +497,9 @@ static int pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_str
         case 7: kernel = pack_kernel<7, 4>; break;
         default: kernel = pack_kernel<8, 3>; break;
         }
-        hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(kPackThreads), 0, stream, (uint8_t const *)b, (uint64_t)b_stride, g.n,
-                           g.k_src_bytes, g.k_chunks, g.k, data, sums, norms, widest_load(b, b_stride), xr, terms ? 1 : 0, h);
+        lists.pack_blocks = g.n_tiles;
+        hipLaunchKernelGGL(kernel, dim3(g.n_tiles + lists.grid[0].bands + lists.grid[1].bands), dim3(kPackThreads), 0, stream, (uint8_t const *)b, (uint64_t)b_stride, g.n,
+                           g.k_src_bytes, g.k_chunks, g.k, data, sums, norms, widest_load(b, b_stride), xr, terms, h, lists);
         e = hipGetLastError();
         if (e != hipSuccess) return fail(e, "pack_kernel");
     }
@@ -512,7 +514,7 @@ static int pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_str
 
 int nk_hip_dots_pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_stride, void *b_packed,
                            void *stream) {
-    return pack_async(dtype, b, n, k, b_stride, b_packed, stream, true);
+    return pack_async(dtype, b, n, k, b_stride, b_packed, stream, 1);
 }
 
 int nk_hip_fill_rows_async(void *c, size_t m, size_t n, size_t c_stride, uint32_t value, void *stream) {
@@ -648,13 +650,20 @@ int nk_hip_symmetric_async(int dtype, int metric, void const *vectors, size_t n,
     if (k && !vectors) return fail_msg("nk_hip_symmetric: vectors is NULL");
     // The columns of the window, packed as the B of an ordinary product; the rows of the window are its A.
     uint8_t const *rows = (uint8_t const *)vectors;
-    int status = pack_async(dtype, rows + w.col_begin * stride, w.columns, k, stride, workspace, stream,
-                            metric != 0 || dtype == kU8);
-    if (status) return status;
-    TriangleScratch const scratch = {(uint32_t *)((uint8_t *)workspace + w.image_bytes), w.scratch_bytes};
+    // First what the product will read besides the image (its tile lists), then one launch that writes both, then the product.
+    TriangleGrids lists = {};
+    TriangleScratch scratch = {(uint32_t *)((uint8_t *)workspace + w.image_bytes), w.scratch_bytes, &lists, row_start == w.col_begin};
     uint8_t *c = (uint8_t *)result + row_start * result_stride + w.col_begin * out_bytes;
-    return product_async(dtype, metric, rows + row_start * stride, workspace, c, w.row_end - row_start, w.columns, k, stride,
-                         result_stride, stream, &scratch, (uint32_t)(row_start - w.col_begin));
+    bool const wide = dtype == kF32 || dtype == kF64; // (no lists)
+    auto product = [&]() {
+        return product_async(dtype, metric, rows + row_start * stride, workspace, c, w.row_end - row_start, w.columns, k, stride,
+                             result_stride, stream, &scratch, (uint32_t)(row_start - w.col_begin));
+    };
+    int status = wide || !k ? 0 : product();
+    if (status) return status;
+    scratch.plan = nullptr;
+    status = pack_async(dtype, rows + w.col_begin * stride, w.columns, k, stride, workspace, stream, metric != 0 ? 2 : dtype == kU8 ? 1 : 0, lists);
+    return status ? status : product();
 }
 
 /**

@@ -85,10 +85,23 @@ struct GemmArgs {
     uint32_t strip_tiles;      // dots_strips_kernel: tiles that a workgroup walks along a strip (tiles_n counts strips)
 };
 
-/** Scratch memory of a triangular grid: the first tile of every band, then the list itself. */
+/** A triangular grid's tile list (see write_tile_list): up to two launches, `bands` of 8 tile rows each. */
+struct TriangleGrid {
+    uint32_t tiles_m, tiles_n, bm_log2, bn_log2, shift, bands;
+    uint32_t *list;
+};
+struct TriangleGrids {
+    uint32_t pack_blocks; // workgroups of the launch that pack
+    TriangleGrid grid[2];
+};
+
+/** Scratch memory of a triangular grid, where its tile lists go. `plan`: nothing is launched, the lists that the launch will
+ *  read are described there instead. `self`: A is the image's own vectors, from its first on. */
 struct TriangleScratch {
     uint32_t *words;
     size_t bytes;
+    TriangleGrids *plan;
+    bool self;
 };
 
 /** The product (or its triangular form) for one element type: picks the tile shape and launches. Defined in
@@ -448,6 +461,51 @@ inline int widen_kind_of(int dtype, size_t k) {
     }
 }
 
+#pragma region Tile lists
+
+/** First tile column of tile row `t` that holds an element on or right of the diagonal col = row + shift; tiles
+ *  are 2^bm_log2 rows by 2^bn_log2 columns. */
+__host__ __device__ inline uint32_t first_live_tile(uint32_t t, uint32_t bm_log2, uint32_t bn_log2, uint32_t shift) {
+    return ((t << bm_log2) + shift) >> bn_log2;
+}
+
+/**
+ *  The tile list of a triangular grid, in the order of `tile_of_block`: bands of kTileBand tile rows, column
+ *  by column within a band, top to bottom within a column, and only tiles with something on or right of the
+ *  diagonal. A workgroup writes a band, all of its threads a column at a time. A band's first columns form a staircase (row t
+ *  joins at column first_live_tile(t)); the cells left of column c number the sum over its rows of max(0, c -
+ *  first_live_tile(t)). Every tile row has a live tile, and a band's rows span whole tiles of columns (kTileBand times
+ *  64 rows at least, 512 columns at most), so the bands before this one are an arithmetic series.
+ *  The lists are written by the launch that packs the vectors, by workgroups behind its own (a launch of one workgroup in front
+ *  of the product took 8 to 11 us of all pairs of 8192, 768 values).
+ */
+__device__ inline void write_tile_list(TriangleGrids const &grids, uint32_t band) {
+    bool const second = band >= grids.grid[0].bands;
+    TriangleGrid const &mine = grids.grid[second ? 1 : 0];
+    if (second) band -= grids.grid[0].bands;
+    uint32_t const tiles_n = mine.tiles_n, first = band * kTileBand, last = first + kTileBand < mine.tiles_m ? first + kTileBand : mine.tiles_m;
+    uint32_t joins[kTileBand]; // where each row of the band joins (past the grid for rows that do not exist)
+    uint64_t start = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kTileBand; ++i) {
+        joins[i] = first + i < last ? first_live_tile(first + i, mine.bm_log2, mine.bn_log2, mine.shift) : 0xFFFFFFFFu;
+        // (row i of the bands before: `band` of them, each `span` columns of tiles further right than the one above)
+        uint32_t const span = (kTileBand << mine.bm_log2) >> mine.bn_log2;
+        start += (uint64_t)band * (tiles_n - first_live_tile(i, mine.bm_log2, mine.bn_log2, mine.shift)) - (uint64_t)span * ((uint64_t)band * (band - 1) / 2);
+    }
+    if (band == 0) start = 0;
+    for (uint32_t column = joins[0] + threadIdx.x; column < tiles_n; column += blockDim.x) {
+        uint64_t at = start;
+#pragma unroll
+        for (uint32_t i = 0; i < kTileBand; ++i) at += column > joins[i] ? column - joins[i] : 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kTileBand; ++i)
+            if (joins[i] <= column) mine.list[2 * at] = first + i, mine.list[2 * at + 1] = column, ++at;
+    }
+}
+
+#pragma endregion Tile lists
+
 #pragma region Packing
 
 /** Sum of the squares of the 8 values of a 16-byte chunk of bf16 (f32 = bits << 16) or f16, in f64. */
@@ -486,8 +544,15 @@ __device__ __forceinline__ double chunk_sumsq_f64(v4i v) {
  *  1-bit type as they are, otherwise the kind of widen_chunk (8 source bytes per chunk).
  *  KIND, by what the image holds: 0 signed bytes (i8, the widened 4-bit types, e2m3 as 8 x its values), 1 u8 stored
  *  with its offset, 2 bf16, 3 f16 (and what is widened to it), 4 bits (no terms: zeros).
- *  `terms` == 0: the tiles only (callers that will never read the terms).
+ *  `terms` == 0: the tiles only (callers that will never read the terms). 2: where the byte sums of u8 go, the float types
+ *  leave the rows' sums of squares as the loop of the product takes them from A (eight values at a time, in f32): what the
+ *  symmetric kinds, which have the image only, need for the bits of the packed ones. (The loop adds the chunks of a stage's
+ *  position one after the other; here four threads share them. f64 holds such sums exactly unless the squares span more
+ *  than 2^29.)
+ *  Workgroups past the tiles write the tile lists of a triangular grid (`lists`), a band each.
  */
+template <int WIDEN, bool BF16_VALUES>
+__device__ __forceinline__ double chunk_sumsq_as_staged(v4i v);
 constexpr int kPackThreads = 1024;
 constexpr int kPackChunks = kPackThreads / kTileRows; // chunks of every row per step of a workgroup
 template <int WIDEN, int KIND>
@@ -495,7 +560,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
                                                             uint64_t k_src_bytes, uint32_t k_chunks, uint32_t k,
                                                             uint8_t *__restrict__ data, uint32_t *__restrict__ sums,
                                                             uint32_t *__restrict__ norms, int avec, uint32_t xr, int terms,
-                                                            PackedHeader header) {
+                                                            PackedHeader header, TriangleGrids lists) {
+    if (blockIdx.x >= lists.pack_blocks) return write_tile_list(lists, blockIdx.x - lists.pack_blocks);
     constexpr int kSrcChunk = WIDEN == 0 || WIDEN == 3 ? 16 : (WIDEN == 7 ? 2 : 8);
     constexpr int kImageChunk = WIDEN == 7 ? 2 : kChunkBytes;
     __shared__ int part_sum[kPackChunks][kTileRows];
@@ -510,7 +576,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
     uint8_t *target = data + ((uint64_t)tile * k_chunks * kTileRows + r) * kImageChunk;
     int sum = 0;
     uint32_t squares = 0;
-    double squares_f64 = 0;
+    double squares_f64 = 0, staged_f64 = 0;
     auto take = [&](uint32_t c) {
         int64_t const left = (int64_t)k_src_bytes - (int64_t)c * kSrcChunk;
         int const valid = row < n ? (int)(left > kSrcChunk ? kSrcChunk : (left < 0 ? 0 : left)) : 0;
@@ -542,7 +608,10 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
                 squares = (uint32_t)__builtin_amdgcn_sdot4(v[w], v[w], (int)squares, false);
             }
         }
-        else if (KIND == 2 || KIND == 3) { squares_f64 += chunk_sumsq_f64<KIND == 2>(v); }
+        else if (KIND == 2 || KIND == 3) {
+            squares_f64 += chunk_sumsq_f64<KIND == 2>(v);
+            if (terms == 2) staged_f64 += chunk_sumsq_as_staged<WIDEN, KIND == 2>(v);
+        }
     };
 #pragma unroll 4
     for (uint32_t c = part; c < k_chunks; c += kPackChunks) take(c);
@@ -558,6 +627,22 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
         if (KIND == 1) squares += 256u * (uint32_t)sum + 16384u * k;
         sums[(uint64_t)tile * kTileRows + mine] = (uint32_t)sum * 128u;
         norms[(uint64_t)tile * kTileRows + mine] = KIND < 2 ? squares : (KIND == 4 ? 0u : __builtin_bit_cast(uint32_t, (float)squares_f64));
+    }
+    if ((KIND == 2 || KIND == 3) && terms == 2) {
+        __syncthreads();
+        part_f64[part][r] = staged_f64;
+        __syncthreads();
+        if (threadIdx.x < kTileRows) {
+            double staged = 0;
+#pragma unroll
+            for (int position = 0; position < 8; ++position) { // (chunk `position` of every stage, then the positions in turn)
+                double one = 0;
+#pragma unroll
+                for (int p = position; p < kPackChunks; p += 8) one += part_f64[p][threadIdx.x];
+                staged += one;
+            }
+            sums[(uint64_t)tile * kTileRows + threadIdx.x] = __builtin_bit_cast(uint32_t, (float)staged);
+        }
     }
 }
 
@@ -804,6 +889,14 @@ struct U4 : I8 {
     static __device__ __forceinline__ norm_t sumsq(v4i, v4i wide) { return I8::sumsq(wide, wide); }
 };
 
+/** Sum of the squares of a chunk as the product's loop takes it (`sumsq` of the type that is stored this way). */
+template <int WIDEN, bool BF16_VALUES>
+__device__ __forceinline__ double chunk_sumsq_as_staged(v4i v) {
+    if constexpr (BF16_VALUES) return BF16::sumsq(v, v);
+    else if constexpr (WIDEN == 1 || WIDEN == 4 || WIDEN == 8) return F16::sumsq_of_normals(v);
+    else return F16::sumsq(v, v);
+}
+
 /**
  *  Distances from a dot product and two sums of squares, as the reference's scalar finalisers compute them
  *  (spatial/serial.h:257-344): integer inputs are converted to f32 first (the i8 kernels read both norms as
@@ -967,77 +1060,6 @@ __device__ __forceinline__ void tile_of_block(uint32_t pid, GemmArgs const &g, u
     tn = in_band / rows;
 }
 
-/** First tile column of tile row `t` that holds an element on or right of the diagonal col = row + shift; tiles
- *  are 2^bm_log2 rows by 2^bn_log2 columns. */
-__host__ __device__ inline uint32_t first_live_tile(uint32_t t, uint32_t bm_log2, uint32_t bn_log2, uint32_t shift) {
-    return ((t << bm_log2) + shift) >> bn_log2;
-}
-
-/**
- *  The tile list of a triangular grid, in the order of `tile_of_block`: bands of kTileBand tile rows, column
- *  by column within a band, top to bottom within a column, and only tiles with something on or right of the
- *  diagonal. One workgroup per list: the bands' sizes are scanned 256 at a time, then every band is filled by all
- *  threads, a column each. A band's first columns form a staircase (row t joins at column first_live_tile(t)); the cells
- *  left of column c number the sum over its rows of max(0, c - first_live_tile(t)).
- */
-struct TriangleGrid {
-    uint32_t tiles_m, tiles_n, bm_log2, bn_log2, shift;
-    uint32_t *band_start, *list;
-};
-struct TriangleGrids {
-    TriangleGrid grid[2];
-};
-__global__ __launch_bounds__(256) void triangle_tiles_kernel(TriangleGrids grids) {
-    TriangleGrid const &mine = grids.grid[blockIdx.x]; // one workgroup per list
-    uint32_t const tiles_m = mine.tiles_m, tiles_n = mine.tiles_n, bm_log2 = mine.bm_log2, bn_log2 = mine.bn_log2,
-                   shift = mine.shift;
-    uint32_t *band_start = mine.band_start, *list = mine.list;
-    __shared__ uint32_t scan[256];
-    __shared__ uint32_t base;
-    uint32_t const tid = threadIdx.x;
-    uint32_t const bands = (tiles_m + kTileBand - 1) / kTileBand;
-    if (tid == 0) base = 0, band_start[0] = 0;
-    __syncthreads();
-    for (uint32_t chunk = 0; chunk < bands; chunk += 256) {
-        uint32_t const band = chunk + tid;
-        uint32_t count = 0;
-        if (band < bands) {
-            uint32_t const first = band * kTileBand, last = first + kTileBand < tiles_m ? first + kTileBand : tiles_m;
-            for (uint32_t t = first; t < last; ++t) {
-                uint32_t const from = first_live_tile(t, bm_log2, bn_log2, shift);
-                count += from < tiles_n ? tiles_n - from : 0;
-            }
-        }
-        scan[tid] = count;
-        __syncthreads();
-        for (uint32_t step = 1; step < 256; step *= 2) {
-            uint32_t const below = tid >= step ? scan[tid - step] : 0;
-            __syncthreads();
-            scan[tid] += below;
-            __syncthreads();
-        }
-        if (band < bands) band_start[band + 1] = base + scan[tid];
-        __syncthreads();
-        if (tid == 255) base += scan[255];
-        __syncthreads();
-    }
-    for (uint32_t band = 0; band < bands; ++band) {
-        uint32_t const first = band * kTileBand, last = first + kTileBand < tiles_m ? first + kTileBand : tiles_m;
-        uint32_t joins[kTileBand]; // where each row of the band joins (past the grid for rows that do not exist)
-#pragma unroll
-        for (uint32_t i = 0; i < kTileBand; ++i) joins[i] = first + i < last ? first_live_tile(first + i, bm_log2, bn_log2, shift) : 0xFFFFFFFFu;
-        uint32_t const start = band_start[band];
-        for (uint32_t column = joins[0] + tid; column < tiles_n; column += 256) {
-            uint32_t at = start;
-#pragma unroll
-            for (uint32_t i = 0; i < kTileBand; ++i) at += column > joins[i] ? column - joins[i] : 0;
-#pragma unroll
-            for (uint32_t i = 0; i < kTileBand; ++i)
-                if (joins[i] <= column) list[2 * (uint64_t)at] = first + i, list[2 * (uint64_t)at + 1] = column, ++at;
-        }
-    }
-}
-
 /**
  *  A persistent workgroup of 4 wavefronts (one per SIMD) walks over (32*TM) x (128*TN) tiles of C. Every
  *  wavefront owns all 32*TM rows of the tile and its own 32*TN columns: B fragments are loaded by exactly
@@ -1096,6 +1118,12 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  in memory, depths of a whole number of trips, the pipelined kernel across tiles, dot products only (the host
  *  checks).
  *
+ *  SELF: all pairs of one set of vectors (windows that start on a tile of the image): A is read out of the packed image as well.
+ *  There it lies in the order of the operands, widened, with zeros behind the rows' ends and its sums taken, so that
+ *  staging is a load and an LDS write of 16 bytes whatever the type, the depth and the alignment of the vectors. Whole calls, before
+ *  and now (us), with the tile lists written by the launch that packs: bf16 8192 x 768 angular 134 and 98, 8192 x 4096 417 and 337,
+ *  i8 8192 x 768 angular 91 and 75, f16 4096 x 300 dots 53 and 43, e2m3 5000 x 600 euclidean 60 and 48.
+ *
  *  SHIFTED: A starts on any byte or its rows are not a multiple of four bytes apart (odd depths). Loads of more than a
  *  dword need dword addresses, so a thread loads the aligned dwords that hold its chunk, one more than the chunk has, and
  *  shifts them into place where they are staged, a v_alignbyte_b32 per dword. How far is the same for every chunk that a
@@ -1114,7 +1142,7 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  */
 // (Workgroups per compute unit: 128 x 128 with two accumulator sets needs 232 to 256 registers, so two of them fit; left to one, the
 // compiler takes 300. bf16 angular 1024 x 262,144 x 768 768 us through 64 x 128, the best before, and 684.)
-template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false, bool FOLDS = false>
+template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false, bool FOLDS = false, bool SELF = false>
 __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
     constexpr int BM = TM * 32;
@@ -1122,6 +1150,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     constexpr int kStageLds = BM * kStageBytes;
     constexpr int kLoads = BM * kStageChunks / NT; // 16-byte LDS chunks per thread per stage = TM
     constexpr int kSrcStage = kStageChunks * T::kSrcChunk; // source bytes of A per row per stage
+    static_assert(!SELF || (ACROSS && !WHOLE && !DIRECT && !SHIFTED), "A out of the image: only the staged loop has it");
     static_assert(!SHIFTED || (ACROSS && !WHOLE && !DIRECT), "shifted loads: only the staged loop has them");
     static_assert(!DIRECT || (ACROSS && !NORMS && !T::kUnsigned && !T::kPrewiden && T::kSrcChunk == 16 && T::kImageChunk == 16),
                   "straight into LDS: only what needs nothing done to it on the way");
@@ -1131,11 +1160,11 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     __shared__ __attribute__((aligned(1024))) uint8_t ring2[DIRECT ? kStageLds : 16];
     __shared__ __attribute__((aligned(1024))) uint8_t ring3[DIRECT ? kStageLds : 16];
     __shared__ __attribute__((aligned(16))) uint32_t row_terms[T::kUnsigned ? BM : 4]; // u8 only: 128 * (sum of the bytes of each A row of the tile)
-    __shared__ uint32_t row_part[T::kUnsigned ? 2 * BM * kStageChunks : 1]; // u8 only: the partial sums behind them
+    __shared__ uint32_t row_part[T::kUnsigned && !SELF ? 2 * BM * kStageChunks : 1]; // u8 only: the partial sums behind them
     typedef typename T::norm_t norm_t;
     __shared__ __attribute__((aligned(16))) uint32_t row_norms[NORMS ? BM : 4]; // distances only: sum of squares of each A row
     __shared__ __attribute__((aligned(16))) float row_factors[NORMS ? BM : 4];  // ... and its refined reciprocal square root
-    __shared__ norm_t norm_part[NORMS ? 2 * BM * kStageChunks : 1];              // ... and the partial sums behind them
+    __shared__ norm_t norm_part[NORMS && !SELF ? 2 * BM * kStageChunks : 1];              // ... and the partial sums behind them
 
     uint32_t const tid = threadIdx.x, lane = tid & 63;
     // The wavefront index is the same in all lanes; telling the compiler keeps B addressing in scalar registers.
@@ -1155,7 +1184,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     // Stages the pipelined loop takes: all of them when A is at least dword-aligned, which is all that multi-dword
     // global loads need, or read by shifted loads; none otherwise. (readfirstlane: the value is uniform, and it must
     // stay in a scalar register because the stage offsets of the buffer loads derive from it.)
-    uint32_t const fast = __builtin_amdgcn_readfirstlane(SHIFTED || g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) ? stages : 0);
+    uint32_t const fast = __builtin_amdgcn_readfirstlane(SHIFTED || SELF || g.avec >= (T::kSrcChunk < 4 ? T::kSrcChunk : 4) ? stages : 0);
     uint32_t const xr = T::kUnsigned ? 0x80808080u : 0u;
     uint32_t const a_pos = tid & 7;
     // A fragment reads: lane l takes row l % 32 of each 32-row block and chunk 2q + l / 32.
@@ -1163,7 +1192,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         uint32_t const r = lane & 31, c = 2 * q + (lane >> 5);
-        a_frag[q] = r * kStageBytes + ((c ^ ((r >> 1) & 7)) << 4);
+        a_frag[q] = SELF ? (uint32_t)q * 1024 + lane * 16 : r * kStageBytes + ((c ^ ((r >> 1) & 7)) << 4);
     }
 
     // A staging: thread t fetches chunk t % 8 of rows i*32 + t/8 of a tile and stores it at its swizzled
@@ -1179,6 +1208,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         a_off[i] = r * (uint32_t)g.a_stride + a_pos * T::kSrcChunk;
         if (SHIFTED) a_off[i] = (a_off[i] + a_skew) & ~3u;
         a_lds[i] = r * kStageBytes + ((a_pos ^ ((r >> 1) & 7)) << 4);
+        if (SELF) a_off[i] = i * (g.k_chunks * kImageTileChunk) + tid * T::kImageChunk, a_lds[i] = i * (32 * kStageBytes) + tid * 16;
     }
     uint32_t const b_lane = lane * T::kImageChunk;
 
@@ -1207,6 +1237,11 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         view.a_bytes = SHIFTED ? (a_skew + (rows_here - 1) * (uint32_t)g.a_stride + (uint32_t)g.k_src_bytes + 3u) & ~3u
                                : (rows_here - 1) * (uint32_t)g.a_stride + (((uint32_t)g.k_src_bytes + kLoadAlign - 1) & ~(kLoadAlign - 1));
         uint32_t const tile_bytes = g.k_chunks * kImageTileChunk;
+        if constexpr (SELF) { // (rows past the last tile: past the descriptor's end, zeros)
+            uint32_t const first_a = (view.row0 + g.tri_shift) / 32;
+            uint64_t const left_a = (uint64_t)(g.n_tiles - first_a) * tile_bytes;
+            view.a = data + (uint64_t)first_a * tile_bytes, view.a_bytes = left_a < 0xFFFFFFFFull ? (uint32_t)left_a : 0xFFFFFFFFu;
+        }
         uint32_t const first = view.col0 / 32 < g.n_tiles ? view.col0 / 32 : g.n_tiles - 1;
         view.b = data + (uint64_t)first * tile_bytes;
         uint64_t const left = (uint64_t)(g.n_tiles - first) * tile_bytes;
@@ -1231,7 +1266,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     // i * 256 + tid: fire-and-forget LDS adds instead of 2 x kLoads registers held through the loop). Two sets:
     // what is staged ahead for the next tile goes to the other one, and the sets swap roles with every tile.
     uint32_t sums_here = 0; // offset of the set of the tile being computed
-    if (T::kUnsigned) {
+    if (T::kUnsigned && !SELF) {
 #pragma unroll
         for (int i = 0; i < 2 * kLoads; ++i) row_part[i * NT + tid] = 0;
     }
@@ -1239,7 +1274,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         __hip_atomic_fetch_add(&row_part[set + i * NT + tid], value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     // Distances: the same bookkeeping for the sums of squares of the rows (u32, or f64 for the float types).
-    if (NORMS) {
+    if (NORMS && !SELF) {
 #pragma unroll
         for (int i = 0; i < 2 * kLoads; ++i) norm_part[i * NT + tid] = 0;
     }
@@ -1280,12 +1315,16 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     auto load_a = [&](TileView const &view, uint32_t s, auto slot_tag, auto part_tag) {
         constexpr int slot = decltype(slot_tag)::value, part = decltype(part_tag)::value;
         __amdgpu_buffer_rsrc_t const rsrc = a_rsrc_of(view);
-        uint32_t const stage_offset = __builtin_amdgcn_readfirstlane(s * kSrcStage); // (the same in all lanes: see load_b)
+        uint32_t const stage_offset = __builtin_amdgcn_readfirstlane(s * (SELF ? kStageChunks * kImageTileChunk : kSrcStage)); // (the same in all lanes: see load_b)
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             if (i * 4 / kLoads != part) continue;
             v4i v = {0, 0, 0, 0};
-            if (T::kSrcChunk == 16) {
+            if constexpr (SELF) {
+                if constexpr (T::kImageChunk == 2) v[0] = (int)(uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, a_off[i], stage_offset, 0);
+                else v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, a_off[i], stage_offset, 0));
+            }
+            else if (T::kSrcChunk == 16) {
                 v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, a_off[i], stage_offset, 0));
                 if constexpr (SHIFTED) a_more[slot][i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, a_off[i] + 16, stage_offset, 0);
             }
@@ -1317,7 +1356,8 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     // `s` is the stage the registers hold: the bytes of its chunk that lie past the end of the row are cleared
     // (for whole stages the masks come out as all ones; no branch either way).
     int const a_tail = (int)(uint32_t)g.k_src_bytes - (int)(a_pos * T::kSrcChunk); // bytes of the row from this thread's chunk on, stage 0
-    constexpr bool kMaskTail = !WHOLE && tail_matters_for<T, NORMS>();
+    constexpr bool kMaskTail = !WHOLE && !SELF && tail_matters_for<T, NORMS>();
+    constexpr bool kPrewiden = T::kPrewiden && !SELF;
     auto masks_of = [&](uint32_t s, uint32_t (&keep)[(T::kSrcChunk + 3) / 4]) {
         int const left = a_tail - (int)(s * kSrcStage);
 #pragma unroll
@@ -1373,13 +1413,13 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
             // (without a next tile to stage for, what is staged past the end is dropped)
             uint32_t const set = across && !mine ? sums_here ^ (uint32_t)(kLoads * NT) : sums_here;
             v4i const raw = v;
-            if (T::kUnsigned) {
+            if (T::kUnsigned && !SELF) {
                 uint32_t const sum = sum_bytes_u8(v);
                 add_row_sum(i, across ? sum : sum * mine, set);
                 v[0] ^= (int)xr, v[1] ^= (int)xr, v[2] ^= (int)xr, v[3] ^= (int)xr;
             }
-            v4i const wide = widened ? v : T::widen(v);
-            if (NORMS) {
+            v4i const wide = widened || (SELF && T::kImageChunk == 16) ? v : T::widen(v);
+            if (NORMS && !SELF) {
                 norm_t const squares = T::sumsq(raw, wide);
                 add_row_norm(i, across || mine ? squares : (norm_t)0, set);
             }
@@ -1440,9 +1480,9 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     // sums; the distance kinds: the squares) and LDS adds (one per sum kept). The k-step that stages asks for them
     // behind its MFMAs, a chunk's worth each; left alone they all land between the last MFMA and the barrier.
     constexpr bool kIntegerSums = __is_same(typename T::acc_t, v16i);
-    constexpr int kStageVector = (T::kUnsigned ? 8 : 0) + (NORMS ? (kIntegerSums ? 5 : 28) : 0) + (SHIFTED && !T::kPrewiden ? (T::kSrcChunk + 3) / 4 : 0);
+    constexpr int kStageVector = SELF ? 0 : (T::kUnsigned ? 8 : 0) + (NORMS ? (kIntegerSums ? 5 : 28) : 0) + (SHIFTED && !T::kPrewiden ? (T::kSrcChunk + 3) / 4 : 0);
     constexpr int kStageLoads = (kLoads >= 4 ? kLoads / 4 : 1) * (SHIFTED && T::kSrcChunk == 16 ? 2 : 1); // of A, per k-step
-    constexpr int kStageDs = 1 + (T::kUnsigned ? 1 : 0) + (NORMS ? 1 : 0);
+    constexpr int kStageDs = SELF ? 1 : 1 + (T::kUnsigned ? 1 : 0) + (NORMS ? 1 : 0);
     // Scheduling hints for one k-step. Masks: 0x008 MFMA, 0x020 VMEM read, 0x100 DS read, 0x200 DS write.
     // Fragment reads go one-to-one with the first TM MFMAs; the global loads of the k-step (TN of B
     // and a quarter of A) are spread over the remaining MFMAs; k-step 2 also carries the LDS writes.
@@ -1510,7 +1550,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         constexpr int entry = decltype(entry_tag)::value; // 0: in the middle of a sum; 1: a fold in front of it; 2: the first stage of a tile
         constexpr int inside = ACROSS ? decltype(inside_tag)::value : 0; // (without ACROSS a tile may have two stages only)
         // vector operations behind each MFMA of the k-steps that widen in place: their share of half the chunks
-        constexpr int kSpread = T::kPrewiden ? (kLoads * 28 + TM * TN - 1) / (TM * TN) : 0;
+        constexpr int kSpread = kPrewiden ? (kLoads * 28 + TM * TN - 1) / (TM * TN) : 0;
         bool const wrap2 = inside < 1 && s + 2 >= fast, wrap3 = inside < 2 && s + 3 >= fast;
         uint32_t const s2 = wrap2 ? s + 2 - fast : s + 2, s3 = wrap3 ? s + 3 - fast : s + 3;
         TileView const &a2 = wrap2 ? nxt : cur, &a3 = wrap3 ? nxt : cur, &b2 = a2;
@@ -1519,14 +1559,14 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         if constexpr (entry != 0) multiply_fresh(slot_c<P>(), slot_c<0>(), slot_c<entry == 1>());
         else multiply(slot_c<P>(), slot_c<0>());
         load_b(b2, s2, slot_c<P>(), slot_c<0>()), load_a(a2, s2, slot_c<P>(), slot_c<2>());
-        if constexpr (T::kPrewiden) prewiden(slot_c<P ^ 1>(), s + 1 < fast ? s + 1 : 0u, slot_c<0>());
+        if constexpr (kPrewiden) prewiden(slot_c<P ^ 1>(), s + 1 < fast ? s + 1 : 0u, slot_c<0>());
         if constexpr (entry != 0 && kChunked) schedule_fresh_k_step();
         else schedule_k_step(slot_c<0>(), slot_c<kSpread>());
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<P>(), slot_c<2>(), slot_c<0>());
         multiply(slot_c<P>(), slot_c<1>());
         load_b(b2, s2, slot_c<P>(), slot_c<1>()), load_a(a2, s2, slot_c<P>(), slot_c<3>());
-        if constexpr (T::kPrewiden) prewiden(slot_c<P ^ 1>(), s + 1 < fast ? s + 1 : 0u, slot_c<1>());
+        if constexpr (kPrewiden) prewiden(slot_c<P ^ 1>(), s + 1 < fast ? s + 1 : 0u, slot_c<1>());
         schedule_k_step(slot_c<0>(), slot_c<kSpread>());
         __builtin_amdgcn_sched_barrier(0);
         read_frags(slot_c<P>(), slot_c<3>(), slot_c<1>());
@@ -1535,7 +1575,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         // A(s+1), loaded over the last two stages, goes to the other buffer (every wavefront left it
         // at the previous barrier); then its registers start being refilled with A(s+3).
         bool const mine = s + 1 < fast;
-        store_a(slot_c<P ^ 1>(), slot_c<P ^ 1>(), mine ? s + 1 : 0u, mine ? 1u : 0u, slot_c<T::kPrewiden ? 1 : 0>());
+        store_a(slot_c<P ^ 1>(), slot_c<P ^ 1>(), mine ? s + 1 : 0u, mine ? 1u : 0u, slot_c<kPrewiden ? 1 : 0>());
         if constexpr (kStageDs > 1) load_b(b2, s2, slot_c<P>(), slot_c<2>()); // (see schedule_k_step)
         load_a(a3, s3, slot_c<P ^ 1>(), slot_c<0>());
         schedule_k_step(slot_c<1>(), slot_c<kStageVector>());
@@ -1685,6 +1725,14 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         // u8: the column terms of this tile are fetched now and used in the epilogue, so that nothing has to
         // wait for them (a wait for a load is a wait for every store issued before it).
         uint32_t col_term[TN], col_norm[TN];
+        // Vectors with themselves: a row's terms are its column's, but for the sums of squares of the floats, which the pack
+        // kernel has left where u8 keeps its byte sums (added up as the loop of a product of two matrices does it).
+        uint32_t self_term = 0, self_norm = 0;
+        if constexpr (SELF && (T::kUnsigned || NORMS)) {
+            uint32_t const row = row0 + g.tri_shift + tid, last = g.n_tiles * kTileRows - 1;
+            if (T::kUnsigned) self_term = col_terms[row < last ? row : last] + 16384u * g.k;
+            if (NORMS) self_norm = (kIntegerSums ? col_norms : col_terms)[row < last ? row : last];
+        }
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             col_term[j] = 0, col_norm[j] = 0;
@@ -1811,8 +1859,17 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         uint32_t const half = lane >> 5, col_in_tile = lane & 31;
         if (T::kUnsigned || NORMS) {
             __syncthreads();
+            if constexpr (SELF) {
+                if (tid < BM) {
+                    if (T::kUnsigned) row_terms[tid] = self_term;
+                    if (NORMS) {
+                        row_norms[tid] = __builtin_bit_cast(uint32_t, norm_as_f32<T>(self_norm));
+                        row_factors[tid] = refined_rsqrt(norm_as_f32<T>(self_norm));
+                    }
+                }
+            }
             // The 8 threads that staged a row left its partial sums in 8 adjacent slots.
-            if (tid < BM) {
+            else if (tid < BM) {
                 if (T::kUnsigned) {
                     uint32_t const *parts = &row_part[sums_here + tid * 8];
                     uint32_t sum = 0;
@@ -1834,7 +1891,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
             }
             __syncthreads();
 #pragma unroll
-            for (int i = 0; i < kLoads; ++i) { // own slots: ready for the tile after next
+            for (int i = 0; i < (SELF ? 0 : kLoads); ++i) { // own slots: ready for the tile after next
                 if (T::kUnsigned) row_part[sums_here + i * NT + tid] = 0;
                 if (NORMS) norm_part[sums_here + i * NT + tid] = 0;
             }
@@ -2331,8 +2388,7 @@ inline uint64_t live_tiles(uint64_t m, uint64_t n, uint32_t bm, uint32_t bn, uin
     return count;
 }
 inline size_t triangle_scratch_bytes(uint64_t m, uint64_t n, uint32_t bm, uint32_t bn, uint32_t shift) {
-    uint64_t const bands = ((m + bm - 1) / bm + kTileBand - 1) / kTileBand;
-    return (size_t)(((bands + 1 + 1) & ~1ull) * 4 + live_tiles(m, n, bm, bn, shift) * 8);
+    return (size_t)live_tiles(m, n, bm, bn, shift) * 8;
 }
 
 /** Rows of A that the pipelined loop reads by shifted loads (see dots_packed_kernel). */
@@ -2355,8 +2411,7 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
         tiles = live_tiles(g.m, g.n, BM, BN, g.tri_shift);
         if (!tiles) return hipSuccess;
         if (triangle_scratch_bytes(g.m, g.n, BM, BN, g.tri_shift) > triangle->bytes) return hipErrorInvalidValue;
-        uint32_t const bands = (g.tiles_m + kTileBand - 1) / kTileBand;
-        g.tile_list = triangle->words + ((bands + 1 + 1) & ~1u); // (written by the caller's triangle_tiles_kernel)
+        g.tile_list = triangle->words;
     }
     g.tile_count = (uint32_t)tiles;
     // The tile's A offsets are 32-bit: (rows of a tile) * stride must stay below 4 GiB.
@@ -2369,7 +2424,8 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     // with dword loads, or shifted into place behind them: bf16 959 x 74,207 x 4307 took 5.6 ms in the guarded loop) and
     // there are enough of them to prefetch three ahead.
     uint32_t const stages = g.k_chunks / kStageChunks;
-    bool const shifted = needs_shift<T>(g);
+    bool const self = triangle && triangle->self && stages >= 4 && (uint64_t)TM * g.k_chunks * kTileRows * T::kImageChunk <= 0xFFFFFFFFull;
+    bool const shifted = !self && needs_shift<T>(g);
     bool const across = !shifted && stages >= 4;
     bool const norms = g.metric != 0;
     // depths that fill an even number of stages exactly: the pipelined kernel without the tail masks
@@ -2405,16 +2461,28 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     // Shallow products of the two-accumulator types fold after every trip of the loop: no branch, and nothing to clear.
     bool folds = false;
     if constexpr (T::kChunked && !T::kDeepOnly && TM * TN > 1) {
-        folds = !direct && (across || shifted) && g.chunk_stages == 2;
+        folds = !direct && !self && (across || shifted) && g.chunk_stages == 2;
         if (folds && !norms) kernel = shifted ? dots_packed_kernel<T, TM, TN, true, false, false, false, true, true>
                                       : whole ? dots_packed_kernel<T, TM, TN, true, false, true, false, false, true> : dots_packed_kernel<T, TM, TN, true, false, false, false, false, true>;
         if (folds && norms) kernel = shifted ? dots_packed_kernel<T, TM, TN, true, true, false, false, true, true>
                                      : whole ? dots_packed_kernel<T, TM, TN, true, true, true, false, false, true> : dots_packed_kernel<T, TM, TN, true, true, false, false, false, true>;
     }
+    // All pairs: A from the image, where it lies as the MFMA wants it (widened, its rows' ends zero, its sums taken).
+    if constexpr (TM * TN > 1 && TM * TN < 16 || (TM == 8 && TN == 2)) {
+        constexpr bool kFolds = T::kChunked && !T::kDeepOnly;
+        if (self) {
+            direct = false;
+            folds = kFolds && g.chunk_stages == 2;
+            kernel = folds ? dots_packed_kernel<T, TM, TN, true, false, false, false, false, kFolds, true> : dots_packed_kernel<T, TM, TN, true, false, false, false, false, false, true>;
+            if constexpr (T::kDistances) {
+                if (norms) kernel = folds ? dots_packed_kernel<T, TM, TN, true, true, false, false, false, kFolds, true> : dots_packed_kernel<T, TM, TN, true, true, false, false, false, false, true>;
+            }
+        }
+    }
     // Persistent grid: as many workgroups as fit on the device at once (queried once per kernel; threads that
     // ask at the same time store the same number).
-    static std::atomic<int> resident_of[22];
-    std::atomic<int> &slot = resident_of[(shifted ? (norms ? 10 : 9) : direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)) + (folds ? 11 : 0)];
+    static std::atomic<int> resident_of[26];
+    std::atomic<int> &slot = resident_of[self ? 22 + (norms ? 1 : 0) + (folds ? 2 : 0) : (shifted ? (norms ? 10 : 9) : direct ? 8 : (across ? 1 : 0) + (norms ? 2 : 0) + (whole ? 4 : 0)) + (folds ? 11 : 0)];
     int resident = slot.load(std::memory_order_relaxed);
     if (!resident) {
         int per_cu = 0;
@@ -2576,6 +2644,24 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         if (strips && (stages <= 2 || stages > 8 || (stages <= 4 && mib >= 512))) return 7;
         return stages <= 4 ? 4 : 0;
     };
+    // All pairs, once A comes out of the image: drawn through 110 random shapes (256 to 16,384 vectors of 64 to 8192 values),
+    // every tile at each. Some of them (us, the largest tile that fills the device and the one taken): dots i8 8192 x 768 81 and 63
+    // (128 x 128), u8 11,269 x 320 188 and 122 (128 x 128), f16 4096 x 300 43 and 34 (64 x 128), e4m3 8192 x 1024 113 and 101 (128 x
+    // 128); euclidean u4 13,649 x 1449 382 and 233 (128 x 128), e5m2 15,409 x 1216 447 and 365 (128 x 128); angular i8 8192 x 768 76
+    // and 69 (64 x 128). 0: nothing here applies.
+    auto by_tiles_of_triangle = [&](GemmArgs const &args) -> int {
+        uint32_t const stages = args.k_chunks / kStageChunks;
+        uint64_t const tiles = tiles_of(args, 3);
+        bool const norms = args.metric != 0;
+        if (T::kChunked && norms) return stages >= 12 && tiles >= 1500 ? 3 : 0;
+        if (T::kChunked) {
+            if (stages <= 2) return 0;
+            if (stages < 32) return tiles >= 1024 ? 3 : tiles >= 256 ? 4 : 0;
+            return tiles >= 512 && tiles < 1024 ? 3 : 0;
+        }
+        if (norms) return tiles < 600 ? 0 : stages <= 8 ? 4 : 3;
+        return stages > 2 && tiles >= 1500 && (stages <= 16 || (T::kDtype == kU1 && stages <= 32)) ? 3 : 0;
+    };
     // Largest tile that still gives every one of the 256 CUs at least one workgroup.
     auto choose = [&](GemmArgs const &args, int first) -> Choice {
         uint32_t const depth_stages = args.k_chunks / kStageChunks;
@@ -2599,6 +2685,8 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // against 25.2); a deep one gains as long as the smaller tiles fit one round (bf16 1024^3 26.3 against 24.8, angular
         // 29.3 against 26.1, but 64 x 30,000 x 4096 54 against 62).
         if (!triangle && tiles_of(args, 4) < 256 && (depth_stages <= 8 || tiles_of(args, 6) <= 256)) return 6;
+        if (triangle && triangle->self && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024)
+            if (int const config = by_tiles_of_triangle(args); config >= first) return config;
         if (!triangle && args.a_stride < (1u << 24) - 1 && args.c_stride < (1u << 30) - 1024)
             if (int const config = by_bytes_of_c(args); config == 7 || (config && tiles_of(args, config) >= 256)) return config;
         // Distances over a shallow depth are bound by the epilogue (a finaliser and a store per output): two
@@ -2703,22 +2791,21 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     }
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
     if (triangle && config >= kTriangleConfigs) config = 4;
-    // Where the tile list of a launch goes (the same arithmetic as launch_one's) and what it holds.
     auto grid_of = [](GemmArgs const &args, int c, TriangleScratch const &scratch) {
         uint32_t const bm = kConfigs[c].tm * 32, bn = kConfigs[c].tn * 128;
         TriangleGrid grid;
         grid.tiles_m = (args.m + bm - 1) / bm, grid.tiles_n = (args.n + bn - 1) / bn;
         grid.bm_log2 = log2_of(bm), grid.bn_log2 = log2_of(bn), grid.shift = args.tri_shift;
-        uint32_t const bands = (grid.tiles_m + kTileBand - 1) / kTileBand;
-        grid.band_start = scratch.words, grid.list = scratch.words + ((bands + 1 + 1) & ~1u);
+        grid.bands = (grid.tiles_m + kTileBand - 1) / kTileBand, grid.list = scratch.words;
         return grid;
     };
 
     // A triangular grid rarely fills a whole number of rounds of the persistent workgroups, and a last round that
     // is mostly empty costs as much as a full one. When that last round would be less than half full, the tile rows
     // from the top that fill whole rounds go to this tile shape and the rows below them, the narrow end of the
-    // triangle, to a second launch with small tiles that spreads them over the whole device.
-    if (triangle && (chosen_here || (forced & 0x80)) && config < 4) {
+    // triangle, to a second launch with small tiles that spreads them over the whole device. (Not 128 x 128 with A out of the
+    // image, two workgroups per compute unit: i8 8192 x 768 68 us in two launches, 63 in one; bf16 96 and 91.)
+    if (triangle && (chosen_here || (forced & 0x80)) && config < 4 && !(config == 3 && triangle->self && chosen_here)) {
         int slots = 0;
         GemmArgs probe = g;
         hipError_t e = launch_config<T>(probe, stream, triangle, config, &slots);
@@ -2744,23 +2831,20 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
                 bottom.tri_shift = g.tri_shift + top.m;
                 // each launch builds its tile list in its own half of the scratch memory
                 size_t const half = triangle->bytes / 2 / 8 * 8;
-                TriangleScratch const first_half = {triangle->words, half}, second_half = {triangle->words + half / 4, half};
+                TriangleScratch const first_half = {triangle->words, half, nullptr, triangle->self}, second_half = {triangle->words + half / 4, half, nullptr, triangle->self};
                 int const narrow = choose(bottom, config + 1).config;
-                TriangleGrids grids;
-                grids.grid[0] = grid_of(top, config, first_half), grids.grid[1] = grid_of(bottom, narrow, second_half);
-                hipLaunchKernelGGL(triangle_tiles_kernel, dim3(2), dim3(256), 0, stream, grids);
-                if ((e = hipGetLastError()) != hipSuccess) return e;
+                if (triangle->plan) {
+                    triangle->plan->grid[0] = grid_of(top, config, first_half), triangle->plan->grid[1] = grid_of(bottom, narrow, second_half);
+                    return hipSuccess;
+                }
                 if ((e = launch_config<T>(top, stream, &first_half, config)) != hipSuccess) return e;
                 return launch_config<T>(bottom, stream, &second_half, narrow);
             }
         }
     }
-    if (triangle && tiles_of(g, config) > 0) {
-        TriangleGrids grids;
-        grids.grid[0] = grids.grid[1] = grid_of(g, config, *triangle);
-        hipLaunchKernelGGL(triangle_tiles_kernel, dim3(1), dim3(256), 0, stream, grids);
-        hipError_t const e = hipGetLastError();
-        if (e != hipSuccess) return e;
+    if (triangle && triangle->plan) {
+        triangle->plan->grid[0] = grid_of(g, config, *triangle), triangle->plan->grid[1] = TriangleGrid {};
+        return hipSuccess;
     }
     return launch_config<T>(g, stream, triangle, config);
 }
