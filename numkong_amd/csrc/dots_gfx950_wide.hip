@@ -372,15 +372,21 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
     f32x4_t a_next[2];
     f64x2_t b_next[kBLoads];
     CompensatedSum squares; // distances: of this thread's share of its row of A
-    // `whole`: the step lies inside the rows of A and they can be read 16 bytes at a time. It is a compile-time choice, one
-    // loop for each: where both ways to load sit in one loop, waits for the loads come between them, in front of the MFMAs
+    // `way` 1: the step lies inside the rows of A and they can be read 16 bytes at a time; 2: they can, and their length is a
+    // multiple of 16 bytes; 0: neither. It is a compile-time choice, one loop for each: where both ways to load sit in one loop, waits for the loads come between them, in front of the MFMAs
     // that are there to cover them.
-    auto fetch = [&](uint32_t k0, auto whole) {
+    auto fetch = [&](uint32_t k0, auto way) {
         if (brings_a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 uint32_t const at = k0 + a_k + 4 * h;
-                if (whole) a_next[h] = *(f32x4_t const *)(a_source + (uint64_t)at * 4);
+                if constexpr (decltype(way)::value == 1) a_next[h] = *(f32x4_t const *)(a_source + (uint64_t)at * 4);
+                else if constexpr (decltype(way)::value == 2) { // (past the row: its first values, made zeros; no branch)
+                    bool const inside = at < g.k;
+                    f32x4_t const loaded = *(f32x4_t const *)(a_source + (uint64_t)(inside ? at : 0u) * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a_next[h][e] = inside ? loaded[e] : 0.f;
+                }
                 else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) a_next[h][e] = at + e < g.k ? ((float const *)a_source)[at + e] : 0.f;
@@ -436,27 +442,35 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
     // and no wave waits on LDS with the matrix pipe idle.
     static_assert(kMatrixDepth == 32, "two groups of 16 depths per step");
     Operands first, second;
-    std::false_type const piecewise;
-    std::true_type const whole;
-    fetch(0, piecewise);
+    std::integral_constant<int, 0> const piecewise;
+    std::integral_constant<int, 1> const whole;
+    std::integral_constant<int, 2> const quads;
+    bool const in_quads = aligned && g.k % 4 == 0 && g.k > 0;
+    if (in_quads) fetch(0, quads);
+    else fetch(0, piecewise);
     stash(0);
-    if (kMatrixDepth < depth) fetch(kMatrixDepth, piecewise);
+    if (kMatrixDepth < depth) {
+        if (in_quads) fetch(kMatrixDepth, quads);
+        else fetch(kMatrixDepth, piecewise);
+    }
     __syncthreads();
     read_operands(0, 0, first);
     int buffer = 0;
     // One step: 8 IB JB MFMAs, and between them, where none of it holds the matrix pipe up: the stash of the step after this one
     // (its stage was last read before the previous barrier), the request for the step after that, the barrier, and the
     // reads of LDS, each asked for a quarter of them before its use. The scheduler is held to this order.
-    auto step = [&](uint32_t k0, auto whole) { // (a whole step: neither the last nor the one before it)
-        bool const more = whole || k0 + kMatrixDepth < depth;
+    // The second group of the last step is left out where the rows end before it (its products are zeros, which change no sum).
+    auto step = [&](uint32_t k0, auto way) { // (a whole step: neither the last nor the one before it)
+        constexpr bool inside = decltype(way)::value == 1;
+        bool const more = inside || k0 + kMatrixDepth < depth, both = inside || k0 + kMatrixDepth / 2 < g.k;
         read_operands(buffer, 1, second);
         __builtin_amdgcn_sched_barrier(0);
         multiply(first, 0, 4);
         __builtin_amdgcn_sched_barrier(0);
         if (more) stash(buffer ^ 1);
-        if (whole || k0 + 2 * kMatrixDepth < depth) fetch(k0 + 2 * kMatrixDepth, whole); // a whole step ahead of its stash()
+        if (inside || k0 + 2 * kMatrixDepth < depth) fetch(k0 + 2 * kMatrixDepth, way); // a whole step ahead of its stash()
         __builtin_amdgcn_sched_barrier(0);
-        multiply(second, 0, 2);
+        if (both) multiply(second, 0, 2);
         __builtin_amdgcn_sched_barrier(0);
         // a barrier that orders LDS only: __syncthreads() would also wait for the loads just asked for
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -464,13 +478,15 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         if (more) read_operands(buffer ^ 1, 0, first);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(second, 2, 4);
+        if (both) multiply(second, 2, 4);
         __builtin_amdgcn_sched_barrier(0);
         buffer ^= 1;
     };
     uint32_t k0 = 0;
     if (aligned)
         for (; k0 + 3 * kMatrixDepth <= g.k; k0 += kMatrixDepth) step(k0, whole);
+    if (in_quads)
+        for (; k0 < depth; k0 += kMatrixDepth) step(k0, quads);
     for (; k0 < depth; k0 += kMatrixDepth) step(k0, piecewise);
 
     double column_norm[JB];

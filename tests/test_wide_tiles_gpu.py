@@ -119,3 +119,23 @@ def test_few_tiles_of_all_pairs(dtype):
         own = (row >= start) & (row < start + rows) & (column >= row)
         expected[own] = serial[own]
         assert np.array_equal(out.cpu().numpy().view(np.uint64), expected.view(np.uint64)), (count, depth, start)
+
+
+# Rows of a multiple of four values at 16-byte addresses (read whole, to the last step of 32 values) against the same values at
+# other addresses (read one by one); depths around the groups of 16 and the steps of 32, which the last step's second group may
+# lie behind. NaN behind every row.
+@pytest.mark.parametrize("metric", ["dots", "angular", "euclidean"])
+def test_f32_rows_of_whole_quads(metric):
+    call = {"dots": nk.dots_packed, "angular": nk.angulars_packed, "euclidean": nk.euclideans_packed}[metric]
+    rng = np.random.default_rng(57)
+    for depth in (4, 12, 16, 20, 32, 36, 48, 52, 64, 80, 100, 112, 300):
+        packed = nk.dots_pack(torch.from_numpy(rng.standard_normal((97, depth)).astype(np.float32)).to("cuda:0"), "f32")
+        for rows in (3, 40, 130):
+            values = torch.from_numpy(rng.standard_normal((rows, depth)).astype(np.float32)).to("cuda:0")
+            results = []
+            for pad, offset in ((4, 0), (4, 1)):
+                whole = torch.full((rows, depth + pad), float("nan"), device="cuda:0")
+                view = whole[:, offset:offset + depth]
+                view.copy_(values)
+                results.append(call(view, packed))
+            assert torch.equal(results[0].view(torch.int64), results[1].view(torch.int64)), f"{metric} {rows} rows of {depth}"
