@@ -82,6 +82,30 @@ __device__ __forceinline__ double wide_distance(int metric, double dot, double q
     return squared > 0 ? squared * wide_rsqrt(squared) : 0.0;
 }
 
+/** The same distances from the hardware's reciprocal square root (good to half of f64's digits) and two Newton steps with fused
+ *  residuals: half of the operations of the bit trick's four, and no further from the root. For arguments well inside the
+ *  range of f64; where a lane's is not (zero, infinite or NaN sums of squares among them), the wavefront takes the form above as
+ *  well. Measured (us): angular 1000 x 20,001 x 300 284 and 278, 100 x 100,000 x 132
+ *  128 and 121; the error against longer arithmetic is that of the form above or a little less (2-norms 5.22e-17 and 5.24e-17). */
+__device__ __forceinline__ double quick_rsqrt(double number) {
+    double y = __builtin_amdgcn_rsq(number);
+    y = __builtin_fma(0.5 * y, __builtin_fma(-(number * y), y, 1.0), y);
+    return __builtin_fma(0.5 * y, __builtin_fma(-(number * y), y, 1.0), y);
+}
+__device__ __forceinline__ double quick_distance(int metric, double dot, double query, double target) {
+#pragma clang fp contract(off)
+    double const argument = metric == 1 ? query * target : query + target - 2.0 * dot;
+    bool const ordinary = argument > 1e-280 && argument < 1e280;
+    double const root = quick_rsqrt(argument);
+    double const angular = 1.0 - dot * root;
+    double result = metric == 1 ? (angular > 0 ? angular : 0) : argument * root;
+    if (__builtin_amdgcn_ballot_w64(!ordinary) != 0) {
+        double const full = wide_distance(metric, dot, query, target);
+        result = ordinary ? result : full;
+    }
+    return result;
+}
+
 /** Sum of squares of every row of B (f32 or f64, row-major) in f64, behind the image's matrix: one wavefront per
  *  row, a compensated sum per lane over every 64th element, the lanes folded the same way. The reference sums the
  *  rounded squares one after the other with a compensation (reduce/serial.h:50-92); this is the same quantity to
@@ -518,7 +542,7 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
                 uint32_t const col = col0 + wave_col + 16 * j + in_block;
                 double result = ((acc[i][j][0][v] + acc[i][j][1][v]) + acc[i][j][2][v]) + acc[i][j][3][v];
                 if (NORMS) {
-                    result = wide_distance(g.metric, result, row_norms[in_tile], column_norm[j]);
+                    result = quick_distance(g.metric, result, row_norms[in_tile], column_norm[j]);
                     if (g.tri_mask && row + g.tri_shift == col) result = 0; // a vector and itself: exactly 0
                 }
                 if (row < g.m && col < g.n && ((row + g.tri_shift) & g.tri_mask) <= col)

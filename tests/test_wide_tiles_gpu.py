@@ -139,3 +139,21 @@ def test_f32_rows_of_whole_quads(metric):
                 view.copy_(values)
                 results.append(call(view, packed))
             assert torch.equal(results[0].view(torch.int64), results[1].view(torch.int64)), f"{metric} {rows} rows of {depth}"
+
+
+# The quicker root of the f32 distances gives way where a sum of squares is zero, infinite, NaN or near the ends of f64's range: the
+# f64 kernel, which always takes the reference's form, has the expected values (the products of these vectors are exact).
+@pytest.mark.parametrize("metric", ["angular", "euclidean"])
+def test_f32_distances_of_extreme_vectors(metric):
+    call = {"angular": nk.angulars_packed, "euclidean": nk.euclideans_packed}[metric]
+    inf, nan = float("inf"), float("nan")
+    rows = [[0, 0, 0, 0], [1e-45, 0, 0, 0], [1e-42, -1e-42, 0, 0], [3e38, 0, 0, 0], [3e38, -3e38, 3e38, 3e38], [inf, 0, 0, 0], [-inf, 1, 0, 0],
+            [nan, 1, 2, 3], [1, 2, 3, 4], [-4, 3, 0.5, -1], [1e-20, 0, 1e-20, 0], [0, 1e19, 0, 0]]
+    values = torch.tensor(rows * 6, dtype=torch.float32, device="cuda:0")
+    got = call(values, nk.dots_pack(values, "f32"))
+    expected = call(values.double(), nk.dots_pack(values.double(), "f64"))
+    assert torch.equal(got.isnan(), expected.isnan()) and torch.equal(got.isinf(), expected.isinf())
+    finite = expected.isfinite()
+    # (roundings of a few units of 2^-53: of one for the angular distance, of the result for the other)
+    scale = torch.ones_like(expected) if metric == "angular" else expected.abs()
+    assert bool(((got - expected).abs()[finite] <= 16 * 2.0**-53 * scale[finite]).all())
