@@ -43,11 +43,6 @@ int nk_hip_memcpy2d_h2d(void *dst, size_t dst_pitch, void const *src, size_t src
 int nk_hip_memcpy2d_d2h(void *dst, size_t dst_pitch, void const *src, size_t src_pitch, size_t width_bytes,
                         size_t rows, void *stream);
 int nk_hip_stream_synchronize(void *stream);
-/** The same wait for work that is expected to take less than 300 us and leaves its results in device memory, on a stream of the
- *  calling thread's (nk_hip_thread_stream): a small kernel behind it writes a word of pinned memory that the host looks at. An
- *  empty kernel takes 8.3 us from launch to return that way, 10.9 with the runtime's wait (medians of 400); i8 1 x 10,000 x 256
- *  through Python 16.9 and 13.3. After 300 us it becomes the runtime's wait. */
-int nk_hip_stream_wait(void *stream);
 
 /**
  *  Per-thread state of the synchronous entry points, so that host threads calling at the same time (the reference's

@@ -81,8 +81,6 @@ struct ThreadContext {
     hipStream_t stream[kThreadStreams] = {};
     hipEvent_t event[kThreadEvents] = {};
     CachedBuffer device[kThreadSlots], pinned[kThreadSlots];
-    uint32_t *flag = nullptr; // pinned: what the last signal_kernel of this thread has written (nk_hip_stream_wait)
-    uint32_t signals = 0;
     void release(bool everything) {
         for (int slot = 0; slot < kThreadSlots; ++slot) {
             if (device[slot].ptr) (void)hipFree(device[slot].ptr);
@@ -90,11 +88,6 @@ struct ThreadContext {
             device[slot] = CachedBuffer(), pinned[slot] = CachedBuffer();
         }
         if (!everything) return;
-        if (flag) {
-            for (hipStream_t s : stream)
-                if (s) (void)hipStreamSynchronize(s);
-            (void)hipHostFree(flag), flag = nullptr;
-        }
         for (hipEvent_t &e : event)
             if (e) (void)hipEventDestroy(e), e = nullptr;
         for (hipStream_t &s : stream)
@@ -280,39 +273,6 @@ int nk_hip_memcpy2d_d2h(void *dst, size_t dst_pitch, void const *src, size_t src
 int nk_hip_stream_synchronize(void *stream) {
     hipError_t e = hipStreamSynchronize((hipStream_t)stream);
     return e == hipSuccess ? 0 : fail(e, "hipStreamSynchronize");
-}
-
-/** A kernel behind the work of a stream: what came before it is complete, and visible to every later kernel, when it runs. */
-__global__ __launch_bounds__(64) void signal_kernel(uint32_t *flag, uint32_t value) {
-    if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-int nk_hip_stream_wait(void *stream) {
-    ThreadContext *context = thread_context();
-    if (!context) return nk_hip_stream_synchronize(stream);
-    if (!context->flag) {
-        if (hipHostMalloc((void **)&context->flag, 64, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            context->flag = nullptr;
-            return nk_hip_stream_synchronize(stream);
-        }
-        __atomic_store_n(context->flag, 0u, __ATOMIC_RELAXED);
-    }
-    uint32_t const signal = ++context->signals;
-    hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, context->flag, signal);
-    if (hipError_t const e = hipGetLastError(); e != hipSuccess) return fail(e, "signal_kernel");
-    struct timespec now, until;
-    clock_gettime(CLOCK_MONOTONIC, &until);
-    until.tv_nsec += 300000;
-    if (until.tv_nsec >= 1000000000) until.tv_sec += 1, until.tv_nsec -= 1000000000;
-    do {
-        for (int look = 0; look < 64; ++look) {
-            if (__atomic_load_n(context->flag, __ATOMIC_ACQUIRE) == signal) return 0;
-            __builtin_ia32_pause();
-        }
-        clock_gettime(CLOCK_MONOTONIC, &now);
-    } while (now.tv_sec < until.tv_sec || (now.tv_sec == until.tv_sec && now.tv_nsec < until.tv_nsec));
-    return nk_hip_stream_synchronize(stream); // (longer than it looked, or failed: that call says so)
 }
 
 /**

@@ -363,7 +363,7 @@ static void nk_amd_pack_(nk_dtype_t dtype, void const *b, nk_size_t n, nk_size_t
     }
     if (!status) status = nk_hip_dots_pack_async((int)dtype, device_b, n, k, device_b_stride, device_p, stream);
     if (!status && staged_p) status = nk_amd_download_flat_(b_packed, staged_p, total, stream);
-    if (!status) status = p_kind == 1 && !staged_b && (double)n * (double)k < 2e7 ? nk_hip_stream_wait(stream) : nk_hip_stream_synchronize(stream);
+    if (!status) status = nk_hip_stream_synchronize(stream);
     if (status) nk_amd_set_error_("nk_dots_pack");
     if (staged_p) {
         /* the host image is what the caller multiplies with next: its device copy is kept for those calls */
@@ -374,15 +374,6 @@ static void nk_amd_pack_(nk_dtype_t dtype, void const *b, nk_size_t n, nk_size_t
 }
 
 /** `metric`: 0 dot products, 1 angular distances, 2 euclidean distances; outputs are 4 bytes wide, 8 for f32 and f64 inputs. */
-/** Does a product of this size take well under the 300 microseconds that nk_hip_stream_wait looks at memory? By its operations, its
- *  results and its table, each at a rate that the slowest type of its kind reaches: 1.1e15, 4e12 bytes of results and of table. */
-static int nk_amd_short_(nk_dtype_t dtype, nk_size_t m, nk_size_t n, nk_size_t k) {
-    double const products = (double)m * (double)n * (double)k, outputs = (double)m * (double)n, values = (double)n * (double)k;
-    if (dtype == nk_f64_k) return products < 4e8 && outputs < 4e7 && values < 3e7;
-    if (dtype == nk_f32_k) return products < 4e9 && outputs < 4e7 && values < 3e7;
-    return products < 8e10 && outputs < 8e7 && values < 2.5e8;
-}
-
 static void nk_amd_packed_(nk_dtype_t dtype, int metric, void const *a, void const *b_packed, void *c, nk_size_t m,
                            nk_size_t n, nk_size_t k, nk_size_t a_stride, nk_size_t c_stride) {
     nk_amd_error_[0] = 0;
@@ -409,7 +400,7 @@ static void nk_amd_packed_(nk_dtype_t dtype, int metric, void const *a, void con
          * staged, so there is nothing else to wait for or to tidy up. */
         int status = metric == 0 ? nk_hip_dots_packed_async((int)dtype, a, b_packed, c, m, n, k, a_stride, c_stride, stream)
                                  : nk_hip_spatials_packed_async((int)dtype, metric, a, b_packed, c, m, n, k, a_stride, c_stride, stream);
-        if (!status) status = c_kind == 1 && nk_amd_short_(dtype, m, n, k) ? nk_hip_stream_wait(stream) : nk_hip_stream_synchronize(stream);
+        if (!status) status = nk_hip_stream_synchronize(stream);
         if (status) {
             nk_amd_set_error_("nk_dots_packed");
             (void)nk_hip_stream_synchronize(stream);
@@ -584,14 +575,7 @@ static void nk_amd_symmetric_(nk_dtype_t dtype, int metric, void const *vectors,
     if (!status && staged_r)
         status = nk_amd_download_(host_window, result_stride, staged_r, device_r_stride, (n - first) * out_bytes,
                                   row_end - row_start, stream);
-    int const in_place = !staged_v && !staged_r;
-    if (!status)
-        status = in_place && r_kind == 1 && nk_amd_short_(dtype, row_end - row_start, n, k) ? nk_hip_stream_wait(stream)
-                                                                                            : nk_hip_stream_synchronize(stream);
-    if (!status && in_place) { /* (nothing else in flight) */
-        nk_hip_thread_trim(nk_amd_keep_slot_k, nk_amd_keep_cached_k);
-        return;
-    }
+    if (!status) status = nk_hip_stream_synchronize(stream);
     if (status) {
         nk_amd_set_error_("nk_dots_symmetric");
         nk_amd_settle_();
