@@ -485,18 +485,22 @@ static int pack_async(int dtype, void const *b, size_t n, size_t k, size_t b_str
         // by how the source is widened and by what the image then holds (see pack_kernel)
         typedef void (*pack_fn)(uint8_t const *, uint64_t, uint32_t, uint64_t, uint32_t, uint32_t, uint8_t *, uint32_t *,
                                 uint32_t *, int, uint32_t, int, PackedHeader, TriangleGrids);
-        pack_fn kernel = nullptr;
-        switch (widen_kind_of(dtype, k)) {
-        case 0: kernel = dtype == kI8 ? pack_kernel<0, 0> : (dtype == kU8 ? pack_kernel<0, 1> : (dtype == kBF16 ? pack_kernel<0, 2> : pack_kernel<0, 3>)); break;
-        case 1: kernel = kE4M3ViaBF16 ? pack_kernel<1, 2> : pack_kernel<1, 3>; break;
-        case 2: kernel = pack_kernel<2, 3>; break;
-        case 3: kernel = pack_kernel<3, 0>; break;
-        case 4: kernel = pack_kernel<4, 3>; break;
-        case 5: kernel = pack_kernel<5, 0>; break;
-        case 6: kernel = pack_kernel<6, 0>; break;
-        case 7: kernel = pack_kernel<7, 4>; break;
-        default: kernel = pack_kernel<8, 3>; break;
-        }
+        auto const kernel_of = [&](auto pairs_) -> pack_fn {
+            constexpr bool pairs = decltype(pairs_)::value;
+            switch (widen_kind_of(dtype, k)) {
+            case 0: return dtype == kI8 ? pack_kernel<0, 0, pairs> : (dtype == kU8 ? pack_kernel<0, 1, pairs> : (dtype == kBF16 ? pack_kernel<0, 2, pairs> : pack_kernel<0, 3, pairs>));
+            case 1: return kE4M3ViaBF16 ? pack_kernel<1, 2, pairs> : pack_kernel<1, 3, pairs>;
+            case 2: return pack_kernel<2, 3, pairs>;
+            case 3: return pack_kernel<3, 0, pairs>;
+            case 4: return pack_kernel<4, 3, pairs>;
+            case 5: return pack_kernel<5, 0, pairs>;
+            case 6: return pack_kernel<6, 0, pairs>;
+            case 7: return pack_kernel<7, 4, pairs>;
+            default: return pack_kernel<8, 3, pairs>;
+            }
+        };
+        bool const for_pairs = terms == 2 || lists.grid[0].bands + lists.grid[1].bands != 0;
+        pack_fn const kernel = for_pairs ? kernel_of(std::true_type()) : kernel_of(std::false_type());
         lists.pack_blocks = g.n_tiles;
         hipLaunchKernelGGL(kernel, dim3(g.n_tiles + lists.grid[0].bands + lists.grid[1].bands), dim3(kPackThreads), 0, stream, (uint8_t const *)b, (uint64_t)b_stride, g.n,
                            g.k_src_bytes, g.k_chunks, g.k, data, sums, norms, widest_load(b, b_stride), xr, terms, h, lists);

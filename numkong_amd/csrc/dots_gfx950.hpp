@@ -549,19 +549,20 @@ __device__ __forceinline__ double chunk_sumsq_f64(v4i v) {
  *  symmetric kinds, which have the image only, need for the bits of the packed ones. (The loop adds the chunks of a stage's
  *  position one after the other; here four threads share them. f64 holds such sums exactly unless the squares span more
  *  than 2^29.)
- *  Workgroups past the tiles write the tile lists of a triangular grid (`lists`), a band each.
+ *  PAIRS, the symmetric kinds' launch: workgroups past the tiles write the tile lists of a triangular grid (`lists`), a band
+ *  each, and `terms` may be 2. A kernel of its own: every workgroup of an ordinary pack would wait for `lists` to be read.
  */
 template <int WIDEN, bool BF16_VALUES>
 __device__ __forceinline__ double chunk_sumsq_as_staged(v4i v);
 constexpr int kPackThreads = 1024;
 constexpr int kPackChunks = kPackThreads / kTileRows; // chunks of every row per step of a workgroup
-template <int WIDEN, int KIND>
+template <int WIDEN, int KIND, bool PAIRS>
 __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__restrict__ b, uint64_t b_stride, uint32_t n,
                                                             uint64_t k_src_bytes, uint32_t k_chunks, uint32_t k,
                                                             uint8_t *__restrict__ data, uint32_t *__restrict__ sums,
                                                             uint32_t *__restrict__ norms, int avec, uint32_t xr, int terms,
                                                             PackedHeader header, TriangleGrids lists) {
-    if (blockIdx.x >= lists.pack_blocks) return write_tile_list(lists, blockIdx.x - lists.pack_blocks);
+    if (PAIRS && blockIdx.x >= lists.pack_blocks) return write_tile_list(lists, blockIdx.x - lists.pack_blocks);
     constexpr int kSrcChunk = WIDEN == 0 || WIDEN == 3 ? 16 : (WIDEN == 7 ? 2 : 8);
     constexpr int kImageChunk = WIDEN == 7 ? 2 : kChunkBytes;
     __shared__ int part_sum[kPackChunks][kTileRows];
@@ -610,7 +611,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
         }
         else if (KIND == 2 || KIND == 3) {
             squares_f64 += chunk_sumsq_f64<KIND == 2>(v);
-            if (terms == 2) staged_f64 += chunk_sumsq_as_staged<WIDEN, KIND == 2>(v);
+            if (PAIRS && terms == 2) staged_f64 += chunk_sumsq_as_staged<WIDEN, KIND == 2>(v);
         }
     };
 #pragma unroll 4
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(uint8_t const *__res
         sums[(uint64_t)tile * kTileRows + mine] = (uint32_t)sum * 128u;
         norms[(uint64_t)tile * kTileRows + mine] = KIND < 2 ? squares : (KIND == 4 ? 0u : __builtin_bit_cast(uint32_t, (float)squares_f64));
     }
-    if ((KIND == 2 || KIND == 3) && terms == 2) {
+    if (PAIRS && (KIND == 2 || KIND == 3) && terms == 2) {
         __syncthreads();
         part_f64[part][r] = staged_f64;
         __syncthreads();
