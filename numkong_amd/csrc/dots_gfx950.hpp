@@ -78,12 +78,18 @@ struct GemmArgs {
     uint32_t tri_shift, tri_mask;
     // Store-bound shapes: workgroup b starts b * stagger_ticks / gridDim.x ticks of the 100 MHz clock late, so that the
     // compute phases of some compute units fall into the store phases of others (0: all start together).
-    uint32_t stagger_ticks;
+    union {
+        uint32_t stagger_ticks;
+        uint32_t strip_tiles; // dots_strips_kernel, which starts its workgroups together: tiles that one walks along a strip (tiles_n counts strips)
+    };
     uint32_t store_policy; // 0: by the alignment of C's rows; 1: past the caches; 2: through them
     uint32_t tile_count;       // tiles_m * tiles_n, or the length of the list
     uint32_t const *tile_list; // (tile row, tile column) pairs in walking order, or NULL for the full grid
-    uint32_t strip_tiles;      // dots_strips_kernel: tiles that a workgroup walks along a strip (tiles_n counts strips)
 };
+// One more word makes the kernels' argument segments 384 bytes (376 with what the runtime adds), and every launch of every product
+// slower, measured with the same code in all else (us): i8 1 x 10,000 x 256 3.67 and 3.84, 2048^3 12.3 and 12.65, 13.05 where
+// launches go round three sets of operands.
+static_assert(sizeof(GemmArgs) <= 120, "kernel arguments: see above");
 
 /** A triangular grid's tile list (see write_tile_list): up to two launches, `bands` of 8 tile rows each. */
 struct TriangleGrid {
