@@ -119,6 +119,8 @@ def library() -> ctypes.CDLL:
     lib.nk_hip_last_error.restype = ctypes.c_char_p
     lib.nk_hip_set_tile_config.argtypes = [i32]
     lib.nk_hip_set_tile_config.restype = None
+    lib.nk_hip_planned_tile.argtypes = [i32, i32, sz, sz, sz, vp, sz, vp, sz, ctypes.POINTER(ctypes.c_uint32)]
+    lib.nk_hip_planned_tile.restype = i32
     lib.nk_hip_device_count.restype = i32
     lib.nk_capabilities.restype = ctypes.c_uint64
     lib.nk_configure_thread.argtypes = [ctypes.c_uint64]

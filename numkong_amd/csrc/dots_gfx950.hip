@@ -21,6 +21,8 @@ namespace nk_gfx950 {
 
 static thread_local int t_forced_config = 0;
 int forced_tile_config() { return t_forced_config; }
+static thread_local PlannedTile t_planned = {};
+PlannedTile *planned_tile() { return &t_planned; }
 
 uint64_t next_image_nonce() {
     static std::atomic<uint64_t> counter {0};
@@ -721,7 +723,18 @@ int nk_hip_symmetric_static_async(int dtype, int metric, void const *vectors, si
 }
 
 void nk_hip_set_tile_config(int config) {
-    t_forced_config = config; // (bits 0..6 the shape; bit 7: a forced shape may still hand the narrow end of a triangle to small tiles; bits 8..27: start spread in 10 ns ticks + 1; bits 28..29: kind of store; bit 30: no staging straight into LDS)
+    t_forced_config = config & 0x7FFFFFFF; // (bits 0..6 the shape; bit 7: a forced shape may still hand the narrow end of a triangle to small tiles; bits 8..27: start spread in 10 ns ticks + 1; bits 28..29: kind of store; bit 30: no staging straight into LDS)
+}
+
+int nk_hip_planned_tile(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                        uint32_t planned[4]) {
+    if (!m || !n || !k || dtype == kF32 || dtype == kF64) return fail_msg("nk_hip_planned_tile: no tile to choose");
+    int const forced = t_forced_config;
+    t_forced_config = (int)((uint32_t)forced | 0x80000000u), t_planned = {};
+    int const status = product_async(dtype, metric, a, (void const *)256, c, m, n, k, a_stride, c_stride, nullptr); // (launches nothing, reads nothing)
+    t_forced_config = forced;
+    planned[0] = t_planned.shape, planned[1] = t_planned.store_policy, planned[2] = t_planned.units, planned[3] = t_planned.strip_tiles;
+    return status;
 }
 
 char const *nk_hip_last_error(void) { return g_last_error; }

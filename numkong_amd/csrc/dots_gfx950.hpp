@@ -141,6 +141,12 @@ hipError_t wide_product(int dtype, void const *a, void const *b_packed, void *c,
 uint64_t next_image_nonce();
 /** Tile shape forced by nk_hip_set_tile_config for the calling thread (0: the heuristic picks). */
 int forced_tile_config();
+/** What a call would run as (test hook nk_hip_planned_tile): with the sign bit of forced_tile_config() set, calls are written down
+ *  here and not launched. */
+struct PlannedTile {
+    uint32_t shape, store_policy, units, strip_tiles;
+};
+PlannedTile *planned_tile();
 /** Compute units of the current device, asked once per process. */
 int compute_unit_count();
 
@@ -2529,8 +2535,29 @@ inline bool strips_possible(GemmArgs const &g) {
     return stages >= 2 && strips_lds_bytes(64, 16, stages) <= kStripsLds && (!T::kChunked || g.chunk_stages == 2) && g.n >= 128 &&
            g.c_stride >= 4 * (uint64_t)g.n && g.c_stride < (1u << 24) - 1024;
 }
+/** How many strips each row of tiles is cut into: of the numbers that fill whole rounds of resident workgroups, the one whose rounds
+ *  walk the fewest tiles, a tile's worth for starting and ending each strip included. Eight candidates, each the most strips that
+ *  fit the rounds they need (fewer walk as far); trying every number up to several hundred took 2.8 us of a call with few rows. */
+struct StripPlan {
+    uint32_t tiles_m, strips, strip_tiles;
+};
+inline StripPlan strip_plan(uint32_t m, uint32_t n, uint32_t bm) {
+    uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256; // (one workgroup's registers fill a compute unit)
+    uint64_t const tiles_m = (m + (uint64_t)bm - 1) / bm, tiles = ((uint64_t)n + kStripColumns - 1) / kStripColumns;
+    uint64_t best = ~0ull, length = tiles;
+    uint64_t strips = 1;
+    for (int candidate = 0; candidate < 8; ++candidate) {
+        uint64_t const rounds = (tiles_m * strips + resident - 1) / resident;
+        strips = rounds * resident / tiles_m;
+        uint64_t const here = strips < tiles ? (tiles + strips - 1) / strips : 1;
+        if (rounds * (here + 1) < best) best = rounds * (here + 1), length = here;
+        if (here == 1) break;
+        ++strips;
+    }
+    return {(uint32_t)tiles_m, (uint32_t)((tiles + length - 1) / length), (uint32_t)length};
+}
 template <class T, int TM, int BATCH>
-hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream) {
+hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream, PlannedTile *planned) {
     constexpr int BM = TM * 32;
     void (*kernel)(GemmArgs) = dots_strips_kernel<T, TM, 0, BATCH>;
     if constexpr (T::kDistances) {
@@ -2538,31 +2565,25 @@ hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream) {
         if (g.metric == 2) kernel = dots_strips_kernel<T, TM, 2, BATCH>;
     }
     else if (g.metric != 0) return hipErrorInvalidValue;
-    uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256; // (one workgroup's registers fill a compute unit)
-    // Strips per row of tiles: the number whose rounds of resident workgroups walk the fewest tiles, a tile's worth for
-    // starting and ending each strip included.
-    g.tiles_m = (g.m + BM - 1) / BM;
-    uint64_t const tiles = ((uint64_t)g.n + kStripColumns - 1) / kStripColumns;
-    uint64_t best = ~0ull, strips = 1;
-    uint64_t const from = resident / g.tiles_m ? resident / g.tiles_m : 1;
-    for (uint64_t s = from; s <= 4 * from + 4; ++s) {
-        uint64_t const length = (tiles + s - 1) / s, rounds = (g.tiles_m * s + resident - 1) / resident;
-        if (rounds * (length + 1) < best) best = rounds * (length + 1), strips = s;
-    }
-    g.strip_tiles = (uint32_t)((tiles + strips - 1) / strips);
-    g.tiles_n = (uint32_t)((tiles + g.strip_tiles - 1) / g.strip_tiles);
+    StripPlan const plan = strip_plan(g.m, g.n, BM);
+    g.tiles_m = plan.tiles_m, g.tiles_n = plan.strips, g.strip_tiles = plan.strip_tiles;
     uint64_t const units = (uint64_t)g.tiles_m * g.tiles_n;
     if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    if (planned) {
+        *planned = {7, 0, (uint32_t)units, g.strip_tiles};
+        return hipSuccess;
+    }
     g.tile_count = (uint32_t)units, g.tile_list = nullptr;
+    uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256;
     hipLaunchKernelGGL(kernel, dim3((uint32_t)(units < resident ? units : resident)), dim3(64 * kStripWaves),
                        strips_lds_bytes(BM, BATCH, g.k_chunks / kStageChunks), stream, g);
     return hipGetLastError();
 }
 template <class T>
-hipError_t launch_strips(GemmArgs &g, hipStream_t stream) {
+hipError_t launch_strips(GemmArgs &g, hipStream_t stream, PlannedTile *planned) {
     uint32_t const stages = g.k_chunks / kStageChunks;
-    if (g.m > 64 && strips_lds_bytes(128, 32, stages) <= kStripsLds) return launch_strips_as<T, 4, 32>(g, stream); // (up to six stages)
-    return launch_strips_as<T, 2, 16>(g, stream);
+    if (g.m > 64 && strips_lds_bytes(128, 32, stages) <= kStripsLds) return launch_strips_as<T, 4, 32>(g, stream, planned); // (up to six stages)
+    return launch_strips_as<T, 2, 16>(g, stream, planned);
 }
 
 template <class T>
@@ -2589,6 +2610,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     int const forced = forced_tile_config();
     int config = forced & 0x7F;
     bool const chosen_here = config <= 0 || config >= kConfigCount;
+    PlannedTile *const planned = forced < 0 ? planned_tile() : nullptr;
     auto tiles_of = [&](GemmArgs const &args, int c) {
         uint64_t const bm = kConfigs[c].tm * 32, bn = (uint64_t)kConfigs[c].tn * 128;
         if (triangle) return live_tiles(args.m, args.n, (uint32_t)bm, (uint32_t)bn, args.tri_shift);
@@ -2793,7 +2815,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     config = chosen.config, g.store_policy = chosen.store_policy;
     if (config == 7) {
         if constexpr (!T::kDeepOnly)
-            if (!triangle && strips_possible<T>(g)) return launch_strips<T>(g, stream);
+            if (!triangle && strips_possible<T>(g)) return launch_strips<T>(g, stream, planned);
         config = 4;
     }
     if ((T::kChunked || needs_shift<T>(g)) && (config == 1 || config == 5)) config = 2;
@@ -2851,6 +2873,10 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     }
     if (triangle && triangle->plan) {
         triangle->plan->grid[0] = grid_of(g, config, *triangle), triangle->plan->grid[1] = TriangleGrid {};
+        return hipSuccess;
+    }
+    if (planned) {
+        *planned = {(uint32_t)config, g.store_policy, (uint32_t)tiles_of(g, config), 0};
         return hipSuccess;
     }
     return launch_config<T>(g, stream, triangle, config);

@@ -335,3 +335,31 @@ def random_matrix(oracle: Oracle, dtype: str, rows: int, cols: int, rng: np.rand
         if kind == "fp8":
             full[rng.random(shape) < 0.01] = 0
     return full[:, :cols] if pad else full
+
+
+class Route:
+    """What a packed product would run as (nk_hip_planned_tile): the shape's number, the kind of store, pieces of work and, of strips,
+    the tiles in one."""
+
+    def __init__(self, shape, store_policy, units, strip_tiles):
+        self.shape, self.store_policy, self.units, self.strip_tiles = shape, store_policy, units, strip_tiles
+
+
+STRIPS = 7  # the number of the strips among the tile shapes
+
+
+def route_of(dtype: str, metric: str, m: int, n: int, k: int, config: int = 0, row_bytes: int = 0, a_row_bytes: int = 0) -> Route:
+    """`row_bytes`, `a_row_bytes`: from one row of C and of A to the next, if not packed rows; both start on lines."""
+    import numkong_amd as nk
+
+    planned = (ctypes.c_uint32 * 4)()
+    per = DIMENSIONS_PER_VALUE.get(dtype, 1)
+    a_row = a_row_bytes or -(-k // per) * np.dtype(STORAGE[dtype]).itemsize
+    nk.library().nk_hip_set_tile_config(config)
+    try:
+        status = nk.library().nk_hip_planned_tile(CODES[dtype], {"dots": 0, **METRICS}[metric], m, n, k, 1 << 30, a_row, 1 << 40,
+                                                  row_bytes or 4 * n, planned)
+    finally:
+        nk.library().nk_hip_set_tile_config(0)
+    assert status == 0, nk.library().nk_hip_last_error()
+    return Route(*planned)
