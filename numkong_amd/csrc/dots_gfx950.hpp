@@ -2579,11 +2579,11 @@ hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream, PlannedTile *planne
                        strips_lds_bytes(BM, BATCH, g.k_chunks / kStageChunks), stream, g);
     return hipGetLastError();
 }
+/** Rows of a strip: 128 up to six stages, 64 beyond and for few rows. */
+inline uint32_t strip_rows(uint32_t m, uint32_t stages) { return m > 64 && strips_lds_bytes(128, 32, stages) <= kStripsLds ? 128 : 64; }
 template <class T>
 hipError_t launch_strips(GemmArgs &g, hipStream_t stream, PlannedTile *planned) {
-    uint32_t const stages = g.k_chunks / kStageChunks;
-    if (g.m > 64 && strips_lds_bytes(128, 32, stages) <= kStripsLds) return launch_strips_as<T, 4, 32>(g, stream, planned); // (up to six stages)
-    return launch_strips_as<T, 2, 16>(g, stream, planned);
+    return strip_rows(g.m, g.k_chunks / kStageChunks) == 128 ? launch_strips_as<T, 4, 32>(g, stream, planned) : launch_strips_as<T, 2, 16>(g, stream, planned);
 }
 
 template <class T>
@@ -2625,12 +2625,39 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         Choice(int config, uint32_t store_policy = 0) : config(config), store_policy(store_policy) {}
     };
     auto past = [](int config) { return Choice(config, 1); };
+    // Strips (see dots_strips_kernel) where C is large against the operands. What they save is the partial lines of rows off the lines
+    // and the staging of A with every tile; what they cost is the start and the end of every strip, with nothing beside it on the
+    // compute unit, and the columns of a row's last tile. So a row of C has to be more than eight tiles of 256 columns and a strip at
+    // least four: with fewer they took up to twice as long as the tiles below, now and before (us): i8 1,000,000 x 130 x 768 638
+    // and 447, angular 817 and 482; bf16 200,000 x 129 x 768 227 and 152; u8 714 x 25,854 x 198 (three to a strip) 31 and 26. On
+    // lines there are no partial ones to save, and a row has to be 32,768 long: i8 euclidean 349,434 x 448 x 64 279 and 151, 6718 x
+    // 20,000 x 448 172 and 150; two stages also take 512 MiB (u4 947 x 85,152 x 64 75 and 67).
+    // Two dot products of integers do not gain by whole lines: deep ones into rows on the memory's sectors, whose partial lines cost it
+    // little (i4 3276 x 27,600 x 1920 267 and 210), and those that take two strips of 64 rows where one tile of 128 holds all
+    // rows of A and reads the image once (u8 angular 109 x 242,980 x 1792 156 and 138).
+    auto strips_pay = [&](GemmArgs const &args, bool lines, uint64_t mib) -> bool {
+        if constexpr (T::kDeepOnly) return false;
+        uint32_t const stages = args.k_chunks / kStageChunks;
+        bool const norms = args.metric != 0;
+        if (!strips_possible<T>(args) || stages > 16 || args.n <= 2048) return false;
+        if (lines) {
+            if (args.m <= 64 || mib < (norms || stages > 2 ? 256 : 512) || args.n < 32768) return false;
+            if (T::kChunked ? !norms && stages > 8 : norms ? stages > 2 && stages <= 8 && (stages > 4 || mib < 512) : stages > 4) return false;
+        }
+        else {
+            if (mib < (stages <= 2 ? 64 : 96)) return false;
+            uintptr_t const rows_at = (uintptr_t)args.c | args.c_stride;
+            if (!T::kChunked && !norms && ((stages > 8 && (rows_at & 31) == 0) || (stages > 4 && (rows_at & 63) == 0))) return false;
+            if (!T::kChunked && args.m > 64 && args.m <= 128 && strip_rows(args.m, stages) == 64) return false;
+        }
+        return strip_plan(args.m, args.n, strip_rows(args.m, stages)).strip_tiles >= 4;
+    };
     // Where storing C is most of the work, what counts is how much of it there is, against the 256 MiB of the last-level
     // cache above all, and whether its rows start on lines. Drawn through 980 random shapes (33 to 8192 rows, depths of 1 to 64
     // stages, C of 4 to 2200 MiB, half of them with rows off the lines; whole calls that go round three sets of operands and
-    // results), every tile and the strips at each: 1.19 of the rules below in the mean; of the best at each shape 0.99; 27
-    // lose more than 3 per cent (0.90 at the least). Some of them (us, before and now): u8 euclidean 1000 x 500,009 x 301
-    // 1165 and 610 (strips), i8 1024 x 204,801 x 220 298 and 151 (strips), f16 8192 x 8191 x 1000 289 and 230 (strips); with rows on
+    // results), every tile and the strips at each, and again through 3000 with up to 2.5 million rows. Some of them (us, before and
+    // now): u8 euclidean 1000 x 500,009 x 301 1165 and 610 (strips), i8 1024 x 204,801 x 220 298 and 151 (strips), f16 8192 x 8191 x
+    // 1000 289 and 230 (strips); with rows on
     // lines bf16 208 x 60,160 x 485 71 and 43 (64 x 128), e5m2 150 x 136,704 x 320 84 and 63 (64 x 128), i8 angular 371 x
     // 34,739 x 1600 154 and 58 (64 x 128), bf16 527 x 400,384 x 192 384 and 259 (strips), bf16 3439 x 38,656 x 826 382 and 316
     // (128 x 128: two workgroups of it fit a compute unit, and the kernels for depths of no whole stage spill at 128 x 256).
@@ -2640,38 +2667,38 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         uint64_t const mib = ((uint64_t)args.m * args.n * 4) >> 20;
         bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0, norms = args.metric != 0;
         bool const whole = args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
-        bool strips = false;
-        if constexpr (!T::kDeepOnly) strips = strips_possible<T>(args) && stages <= 16;
-        // A strip has a start and an end to pay for: enough of C for many tiles to a strip, and what it saves (partial lines,
-        // the part of A staged with every tile) has to be a large part.
-        if (!lines && strips && mib >= (stages <= 2 ? 64 : 96)) return 7;
+        if (strips_pay(args, lines, mib)) return 7;
         if (args.m <= 64) return 0;
+        // Two tiles of 64 rows read the image twice, which is most of a deep product of few rows (u4 74 x 178,464 x 1664 89 us and 76
+        // through 128 x 128, i8 angular 79 x 269,824 x 2122 207 and 168).
+        if (!T::kChunked && args.m <= 128 && stages > (norms ? 16 : 4)) return 0;
         if (!lines) {
-            if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : 3;
-            if (norms) return stages > 16 && mib >= 96 ? 3 : 0;
+            // (Shallow products into so large a C belong to strips or, where those do not pay, to the rule at the end.)
+            if (stages <= 16 && mib >= (stages <= 2 ? 64 : 96)) return 0;
+            // Depths at which the MFMAs are most of the work again: the largest tiles, once there are enough of them (e2m3 euclidean
+            // 78,940 x 2733 x 12,009 5265 through 128 x 128 and 3664 through 256 x 256, f16 5825 x 48,330 x 5312 4360 and 4006).
+            if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : stages <= 32 || (stages <= 60 && mib < 256) ? 3 : 0;
+            if (norms) return stages > 16 && mib >= 96 && (stages <= 60 || mib < 300) ? 3 : 0;
             if (T::kChunked) return (stages > 4 && mib >= 32 && mib < 96) || (stages > 16 && mib >= 32 && mib < 256) ? 3 : 0;
             return stages <= 16 && mib < 96 ? 4 : 0;
         }
-        if (T::kChunked && norms) {
-            if (strips && mib >= 256 && args.n >= 32768) return 7;
-            return stages > 16 && stages < 32 && mib >= 64 ? 3 : 0;
-        }
+        // (two columns of tiles: A is read twice by the small ones; i8 216,199 x 256 x 384 94 and 62 through 256 x 256)
+        if (!T::kChunked && args.n <= 256 && mib >= 128) return 0;
+        if (T::kChunked && norms) return stages > 16 && stages < 32 && mib >= 64 ? 3 : 0;
         if (T::kChunked) {
             if (mib < 96) return stages > 2 && (stages <= 16 || (stages < 32 && !whole)) ? 4 : 0;
-            if (strips && mib >= 256 && stages <= 8) return 7;
-            if (stages <= 4) return stages > 2 ? 4 : 0;
-            return stages <= 16 || (stages < 32 && !whole) ? 3 : 0;
+            if (stages <= 4) return stages > 2 && mib < 256 ? 4 : 0;
+            return (stages <= 16 && (stages > 8 || mib < 256)) || (stages > 16 && stages < 32 && !whole) ? 3 : 0;
         }
         if (!norms) {
             if (stages > 16) return 0;
             if (mib < 96) return stages <= 8 || mib >= 32 ? 4 : 0; // (i8 2048^3 28.0 us through 128 x 128, 28.8 through 64 x 128)
-            if (stages <= 4) return strips && mib >= 256 ? 7 : stages > 2 ? 4 : 0;
+            if (stages <= 4) return stages > 2 && mib < 256 ? 4 : 0;
             return stages <= 8 && mib < 512 ? 3 : 0;
         }
         if (stages > 16) return stages < 32 && mib < 96 ? 4 : 0;
         if (mib < 256) return stages <= 8 || mib < 96 ? 4 : 3;
-        if (strips && (stages <= 2 || stages > 8 || (stages <= 4 && mib >= 512))) return 7;
-        return stages <= 4 ? 4 : 0;
+        return stages > 2 && stages <= 4 && mib < 512 ? 4 : 0;
     };
     // All pairs, once A comes out of the image: drawn through 110 random shapes (256 to 16,384 vectors of 64 to 8192 values),
     // every tile at each. Some of them (us, the largest tile that fills the device and the one taken): dots i8 8192 x 768 81 and 63

@@ -46,3 +46,33 @@ def test_planning_takes_no_time():
 
     tiles, strips = least((100, 300_001, 256), 4), least((100, 300_001, 256), STRIPS)
     assert strips < tiles + 1.0e-6, f"{(strips - tiles) * 1e6:.2f} us more than for a fixed tile"
+
+
+# Products for which strips were once chosen and took 1.1 to 2 times as long as the tiles that had them before: rows of C of a few
+# tiles, strips of three, long rows that start on lines anyway, deep products of integers into rows on the memory's sectors, two
+# strips of 64 rows where one tile holds all rows.
+@pytest.mark.parametrize("dtype, metric, m, n, k", [
+    ("i8", "dots", 1_000_000, 130, 768), ("i8", "angular", 1_000_000, 130, 768), ("bf16", "dots", 200_000, 129, 768), ("u8", "angular", 50_000, 600, 300),
+    ("e4m3", "angular", 40_000, 1001, 256), ("u8", "dots", 714, 25_854, 198), ("bf16", "dots", 3340, 6513, 64), ("i8", "euclidean", 349_434, 448, 64),
+    ("i8", "euclidean", 6718, 20_000, 448), ("u4", "dots", 947, 85_152, 64), ("i4", "dots", 3276, 27_600, 1920), ("u1", "dots", 25_065, 4016, 896),
+    ("u8", "angular", 109, 242_980, 1792)])
+def test_no_strips_where_they_do_not_pay(dtype, metric, m, n, k):
+    assert route_of(dtype, metric, m, n, k).shape != STRIPS
+
+
+# ... and those that they are for.
+@pytest.mark.parametrize("dtype, metric, m, n, k", [
+    ("u8", "euclidean", 1000, 500_009, 301), ("f16", "dots", 8192, 8191, 1000), ("i8", "dots", 1024, 204_801, 220), ("bf16", "dots", 527, 400_384, 192),
+    ("i8", "angular", 30_000, 2301, 128), ("bf16", "euclidean", 63_086, 5932, 128), ("u8", "angular", 1025, 279_648, 1500), ("e4m3", "dots", 407, 580_128, 340)])
+def test_strips_where_they_pay(dtype, metric, m, n, k):
+    route = route_of(dtype, metric, m, n, k)
+    assert route.shape == STRIPS and route.strip_tiles >= 4
+
+
+# Tiles chosen by the bytes of C that were slower than the larger ones in use before, by up to 1.4 times: deep distances into rows off
+# the lines through 128 x 128, and two tiles of 64 rows that read a large image twice.
+@pytest.mark.parametrize("dtype, metric, m, n, k, tile", [
+    ("e2m3", "euclidean", 78_940, 2733, 12_009, 2), ("i8", "euclidean", 1208, 245_611, 10_624, 2), ("f16", "euclidean", 5825, 48_330, 5312, 2),
+    ("u4", "euclidean", 90, 251_584, 3306, 3), ("i8", "angular", 79, 269_824, 2122, 3), ("u4", "dots", 74, 178_464, 1664, 3), ("i8", "dots", 216_199, 256, 384, 1)])
+def test_larger_tiles_where_the_operands_weigh_most(dtype, metric, m, n, k, tile):
+    assert route_of(dtype, metric, m, n, k).shape in (1, 2) if tile < 3 else route_of(dtype, metric, m, n, k).shape == tile
