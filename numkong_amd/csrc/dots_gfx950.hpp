@@ -2509,6 +2509,11 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
         *slots_only = resident;
         return hipSuccess;
     }
+    // Stores past the caches reach the memory as they are, and partial lines of two workgroups on a compute unit get in each other's way
+    // where they are most of the work: 128 x 128 of the two-accumulator types, one and two of them (us): bf16 99,543 x 1482 x 320 213 and
+    // 287, 1,000,000 x 130 x 768 598 and 716, e4m3 101,986 x 1059 x 512 179 and 211; the mean of fourteen such shapes 0.83. Of
+    // 17 to 31 stages two are faster again (seventeen shapes, 0.93).
+    if (T::kChunked && TM * TN == 4 && g.store_policy == 1 && stages <= 16 && compute_unit_count() > 0 && resident > compute_unit_count()) resident = compute_unit_count();
     uint32_t const blocks = (uint32_t)(tiles < (uint64_t)resident ? tiles : (uint64_t)resident);
     // Shallow products with several tiles per workgroup are bound by their stores: spread the starts over about the
     // time one round of tiles takes to store (the chip writes some 5.5 TB/s in this pattern; ticks of 10 ns).

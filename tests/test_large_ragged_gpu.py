@@ -55,3 +55,28 @@ def test_no_slower_than_the_tile_of_smaller_results(dtype, m, n, k, tile):
                 nk.library().nk_hip_set_tile_config(0)
             best[config] = min(best.get(config, 1e9), begin.elapsed_time(end) / 4)
     assert best[0] <= 1.12 * best[tile], f"{dtype} {m} x {n} x {k}: {best[0]:.3f} ms chosen, {best[tile]:.3f} ms through shape {tile}"
+
+
+# Partial lines of many rows past the caches: two workgroups on a compute unit took 1.2 and 1.15 times as long as one of the 128 x 256 tile
+# does (one of 128 x 128: 1.03 and 0.91). Results are new ones in turn: into one that the last-level cache holds all are alike.
+@pytest.mark.parametrize("dtype, m, n, k, tile", [("bf16", 1_000_000, 130, 768, 2), ("bf16", 1_536_789, 218, 382, 2)])
+def test_rows_past_the_caches(dtype, m, n, k, tile):
+    rng = np.random.default_rng(63)
+    a = values_of(dtype, 4099, k, rng).to(DEV).repeat(-(-m // 4099), 1)[:m].contiguous()
+    packed = nk.dots_pack(values_of(dtype, n, k, rng).to(DEV), dtype)
+    outs = [torch.empty((m, n), dtype=torch.float32, device=DEV) for _ in range(3)]
+    best = {}
+    for _ in range(5):
+        for config in (0, tile):
+            nk.library().nk_hip_set_tile_config(config)
+            try:
+                begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                begin.record()
+                for out in outs:
+                    nk.dots_packed(a, packed, out=out)
+                end.record()
+                end.synchronize()
+            finally:
+                nk.library().nk_hip_set_tile_config(0)
+            best[config] = min(best.get(config, 1e9), begin.elapsed_time(end) / 3)
+    assert best[0] <= 1.1 * best[tile], f"{dtype} {m} x {n} x {k}: {best[0]:.3f} ms chosen, {best[tile]:.3f} ms through shape {tile}"
