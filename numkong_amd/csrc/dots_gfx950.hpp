@@ -2681,10 +2681,11 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             // (Shallow products into so large a C belong to strips or, where those do not pay, to the rule at the end.)
             if (stages <= 16 && mib >= (stages <= 2 ? 64 : 96)) return 0;
             // Depths at which the MFMAs are most of the work again: the largest tiles, once there are enough of them (e2m3 euclidean
-            // 78,940 x 2733 x 12,009 5265 through 128 x 128 and 3664 through 256 x 256, f16 5825 x 48,330 x 5312 4360 and 4006).
+            // 78,940 x 2733 x 12,009 5265 through 128 x 128 and 3664 through 256 x 256, f16 5825 x 48,330 x 5312 4360 and 4006; dots
+            // e4m3 755 x 53,520 x 5376 458 and 425).
             if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : stages <= 32 || (stages <= 60 && mib < 256) ? 3 : 0;
             if (norms) return stages > 16 && mib >= 96 && (stages <= 60 || mib < 300) ? 3 : 0;
-            if (T::kChunked) return (stages > 4 && mib >= 32 && mib < 96) || (stages > 16 && mib >= 32 && mib < 256) ? 3 : 0;
+            if (T::kChunked) return mib >= 32 && ((stages > 4 && mib < 96) || (stages > 16 && mib < 256)) && stages <= 60 ? 3 : 0;
             return stages <= 16 && mib < 96 ? 4 : 0;
         }
         // (two columns of tiles: A is read twice by the small ones; i8 216,199 x 256 x 384 94 and 62 through 256 x 256)

@@ -72,7 +72,7 @@ def test_strips_where_they_pay(dtype, metric, m, n, k):
 # Tiles chosen by the bytes of C that were slower than the larger ones in use before, by up to 1.4 times: deep distances into rows off
 # the lines through 128 x 128, and two tiles of 64 rows that read a large image twice.
 @pytest.mark.parametrize("dtype, metric, m, n, k, tile", [
-    ("e2m3", "euclidean", 78_940, 2733, 12_009, 2), ("i8", "euclidean", 1208, 245_611, 10_624, 2), ("f16", "euclidean", 5825, 48_330, 5312, 2),
+    ("e2m3", "euclidean", 78_940, 2733, 12_009, 2), ("i8", "euclidean", 1208, 245_611, 10_624, 2), ("f16", "euclidean", 5825, 48_330, 5312, 2), ("e4m3", "dots", 755, 53_520, 5376, 2),
     ("u4", "euclidean", 90, 251_584, 3306, 3), ("i8", "angular", 79, 269_824, 2122, 3), ("u4", "dots", 74, 178_464, 1664, 3), ("i8", "dots", 216_199, 256, 384, 1)])
 def test_larger_tiles_where_the_operands_weigh_most(dtype, metric, m, n, k, tile):
     assert route_of(dtype, metric, m, n, k).shape in (1, 2) if tile < 3 else route_of(dtype, metric, m, n, k).shape == tile
