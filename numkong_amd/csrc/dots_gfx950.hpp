@@ -2182,8 +2182,9 @@ __global__ __launch_bounds__(64 * kStripWaves, 2) void dots_strips_kernel(GemmAr
         // are those of dots_packed_kernel, in the same order.
         meet(); // (the strip before is done with the LDS)
         {
-            uint32_t *const part_sums = stage_rows;           // (BM x 8 words)
-            norm_t *const part_norms = (norm_t *)carried;     // (BM x 8, at most 16 KiB: `carried` is as large)
+            uint32_t *const part_sums = stage_rows;       // (BM x 8 of them)
+            norm_t *const part_norms = (norm_t *)carried; // (and as many of these)
+            static_assert(BM * 8 <= BATCH * kStripColumns && BM * 8 * sizeof(norm_t) <= BM * 32 * sizeof(uint32_t), "partial sums: they fit where they wait");
             uint32_t const a_pos = tid & 7;
             for (uint32_t r = tid >> 3; r < (uint32_t)BM; r += NT / 8) {
                 bool const exists = row0 + r < g.m;

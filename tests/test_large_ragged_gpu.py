@@ -9,26 +9,48 @@ from tests.test_unaligned_gpu import DEV, same, values_of
 pytestmark = pytest.mark.gpu
 
 
-# One shape for each tile that the rule picks by depth (in stages of 128 bytes of operand), its rows not a multiple of any
-# tile, and the smallest C that the rule takes for large; 300 rows at six stages are an odd number of 128s, where the
-# integers leave the 256-row tile. (e2m3 takes its 128 x 512 tile for all of these: there are 256 of them each time. It is
-# here for that tile's masked stores into such rows.)
+def through(config, call):
+    nk.library().nk_hip_set_tile_config(config)
+    try:
+        return call()
+    finally:
+        nk.library().nk_hip_set_tile_config(0)
+
+
+def large(dtype, m, n, stages, rng):
+    values = {"bf16": 64, "f16": 64, "e4m3": 64, "i4": 64, "u1": 16}.get(dtype, 128)  # stored in a row of a stage
+    columns = stages * values - 8 * (values > 16)
+    a, b = values_of(dtype, m, columns, rng).to(DEV), values_of(dtype, 4099, columns, rng)
+    return a, nk.dots_pack(b.to(DEV).repeat(-(-n // 4099), 1)[:n].contiguous(), dtype), f"{dtype} {m} x {n} x {columns}"
+
+
+# What is chosen for them: strips up to ten stages, the fewest rows that leave one of 128 and of 64 a row or a few over; tiles at
+# 18 (of 256 x 256, of e2m3 128 x 512, of the two-accumulator types 128 x 128).
 @pytest.mark.parametrize("dtype", ["i8", "u8", "i4", "u1", "e2m3", "bf16", "f16", "e4m3"])
 def test_tiles_of_large_results(dtype):
     rng = np.random.default_rng(61)
-    values = {"bf16": 64, "f16": 64, "e4m3": 64, "i4": 64, "u1": 16}.get(dtype, 128)  # stored in a row of a stage
     for m, n, stages in ((133, 760_003, 2), (133, 760_003, 4), (129, 790_001, 6), (300, 340_003, 6), (257, 393_003, 10), (300, 120_001, 18)):
-        columns = stages * values - 8 * (values > 16)
-        a, b = values_of(dtype, m, columns, rng).to(DEV), values_of(dtype, 4099, columns, rng)
-        packed = nk.dots_pack(b.to(DEV).repeat(-(-n // 4099), 1)[:n].contiguous(), dtype)
+        a, packed, name = large(dtype, m, n, stages, rng)
         chosen = nk.dots_packed(a, packed)
-        nk.library().nk_hip_set_tile_config(4)
-        try:
-            expected = nk.dots_packed(a, packed)
-        finally:
-            nk.library().nk_hip_set_tile_config(0)
-        assert same(chosen, expected), f"{dtype} {m} x {n} x {columns}"
+        expected = through(4, lambda: nk.dots_packed(a, packed))
+        assert same(chosen, expected), name
         del packed, chosen, expected
+
+
+# Every larger tile into such rows, stored past the caches and through them (bits 28..29 of the hook): masked stores of rows that no
+# tile's height divides and of columns that no tile's width does, two-stage rows and pipelined ones.
+@pytest.mark.parametrize("dtype", ["i8", "u8", "i4", "u1", "e2m3", "bf16", "f16", "e4m3"])
+def test_every_tile_into_large_results(dtype):
+    rng = np.random.default_rng(64)
+    for m, n, stages in ((133, 300_003, 2), (300, 140_003, 6)):
+        a, packed, name = large(dtype, m, n, stages, rng)
+        expected = through(4, lambda: nk.dots_packed(a, packed))
+        for shape in (1, 2, 3) + ((5,) if dtype == "e2m3" else ()):
+            for policy in (1, 2):
+                got = torch.full_like(expected, 77)
+                through(shape | policy << 28, lambda: nk.dots_packed(a, packed, out=got))
+                assert same(got, expected), f"{name} shape {shape} store {policy}"
+        del packed, got, expected
 
 
 # Shapes that a rule for such results once made slower than the tile it replaced (by 1.22 to 1.44 times): whatever is chosen now

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import numkong_amd as nk
+from tests.support import DIMENSIONS_PER_VALUE, STRIPS, route_of
 from tests.test_unaligned_gpu import CALLS, DEV, same, values_of
 
 pytestmark = pytest.mark.gpu
@@ -50,9 +51,33 @@ def test_same_bits_as_tiles(dtype):
         for metric in ["dots"] if dtype == "u1" else list(CALLS):
             expected = through(4, lambda: CALLS[metric](a, packed))
             whole, window = framed(m, n, before, after, expected.dtype)
+            planned = route_of(dtype, metric, m, n, columns * DIMENSIONS_PER_VALUE.get(dtype, 1), STRIPS, 4 * (before + n + after))
+            assert planned.shape == STRIPS, f"{dtype} {metric} {m} x {n} x {columns}: not strips, which is what this test is for"
             through(7, lambda: CALLS[metric](a, packed, out=window))
             assert same(window.contiguous(), expected), f"{dtype} {metric} {m} x {n} x {columns}"
             assert untouched(whole, m, n, before), f"{dtype} {metric} {m} x {n} x {columns}: written outside C"
+
+
+# More pieces of work than there are compute units, so that a workgroup takes a second one (and a third) into the LDS that held the
+# first: its rows of A, their sums and norms, what its last lines had left over. (Rows per compute unit, columns, stages, how many
+# pieces a workgroup takes at the least): one tile to a piece and two, pieces of 128 rows and of 64, strips beside each other.
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("rows, n, stages, before, after, least", [(129, 129, 2, 3, 2, 2), (129, 300, 2, 0, 1, 2), (65, 300, 8, 5, 0, 2), (78, 1201, 16, 0, 0, 2), (257, 600, 3, 1, 0, 3)])
+def test_workgroups_of_several_pieces(dtype, rows, n, stages, before, after, least):
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    m = rows * units
+    rng = np.random.default_rng(84)
+    columns = stages * STAGE.get(dtype, 128) - 3
+    a = values_of(dtype, 4099, columns, rng).to(DEV).repeat(-(-m // 4099), 1)[:m].contiguous() # (4099: no two pieces have the same rows)
+    packed = nk.dots_pack(values_of(dtype, n, columns, rng).to(DEV), dtype)
+    for metric in ["dots"] if dtype == "u1" else list(CALLS):
+        planned = route_of(dtype, metric, m, n, columns * DIMENSIONS_PER_VALUE.get(dtype, 1), STRIPS, 4 * (before + n + after))
+        assert planned.shape == STRIPS and planned.units > (least - 1) * units, f"{planned.units} pieces for {units} workgroups"
+        expected = through(4, lambda: CALLS[metric](a, packed))
+        whole, window = framed(m, n, before, after, expected.dtype)
+        through(7, lambda: CALLS[metric](a, packed, out=window))
+        assert same(window.contiguous(), expected), f"{dtype} {metric} {m} x {n} x {columns}"
+        assert untouched(whole, m, n, before), f"{dtype} {metric} {m} x {n} x {columns}: written outside C"
 
 
 # NaN and infinities behind the ends of the rows of A (a row of 37 values in rows of 64) stay out of the sums.

@@ -31,8 +31,28 @@ def test_same_bits_as_both_sides_packed(dtype):
                 finally:
                     nk.library().nk_hip_set_tile_config(0)
                 assert torch.equal(torch.triu(got), full), f"{dtype} {metric} {count} x {columns} shape {config}"
-        if count > 64: # windows on a tile of the image and off it
-            whole = SYMMETRIC["dots"](vectors, dtype)
-            for start in (32, 45):
-                part = SYMMETRIC["dots"](vectors, dtype, start_row=start, end_row=count - 3)
-                assert torch.equal(torch.triu(part)[start:count - 3], torch.triu(whole)[start:count - 3]), f"{dtype} rows {start} on of {count} x {columns}"
+        if count > 64: # windows on a tile of the image (A out of it, its sums too) and off it (A and its sums from the vectors)
+            for metric in ["dots"] if dtype == "u1" else list(CALLS):
+                whole = SYMMETRIC[metric](vectors, dtype).view(torch.int32)
+                for start in (32, 45):
+                    part = SYMMETRIC[metric](vectors, dtype, start_row=start, end_row=count - 3).view(torch.int32)
+                    assert torch.equal(torch.triu(part)[start:count - 3], torch.triu(whole)[start:count - 3]), f"{dtype} {metric} rows {start} on of {count} x {columns}"
+
+
+# Values of many magnitudes, whose squares span more than f64 can add without rounding. The packing launch adds a row's squares in another
+# order than the loop does; the two are within 2^-42 of each other (600 additions in f64 each), so that rounded to f32 they can
+# differ for one row in 2^18 at the most. These rows do not.
+@pytest.mark.parametrize("dtype, spread", [("bf16", 9.0), ("f16", 3.0)])
+def test_row_sums_of_many_magnitudes(dtype, spread):
+    rng = np.random.default_rng(92)
+    count, columns = 700, 600
+    values = rng.standard_normal((count, columns)) * 10.0 ** rng.uniform(-spread, spread, (count, columns))
+    vectors = torch.from_numpy(values.astype(np.float32)).to(torch.bfloat16 if dtype == "bf16" else torch.float16).to(DEV)
+    assert not bool(torch.isinf(vectors).any())
+    packed = nk.dots_pack(vectors, dtype)
+    for metric in ("angular", "euclidean"):
+        full = torch.triu(CALLS[metric](vectors, packed).view(torch.int32), 1)
+        assert torch.equal(torch.triu(SYMMETRIC[metric](vectors, dtype).view(torch.int32)), full), f"{dtype} {metric}"
+        for start in (32, 45):
+            part = SYMMETRIC[metric](vectors, dtype, start_row=start, end_row=count).view(torch.int32)
+            assert torch.equal(torch.triu(part)[start:], full[start:]), f"{dtype} {metric} rows {start} on"
