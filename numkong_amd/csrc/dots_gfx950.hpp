@@ -2634,29 +2634,41 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // Strips (see dots_strips_kernel) where C is large against the operands. What they save is the partial lines of rows off the lines
     // and the staging of A with every tile; what they cost is the start and the end of every strip, with nothing beside it on the
     // compute unit, and the columns of a row's last tile. So a row of C has to be more than eight tiles of 256 columns and a strip at
-    // least four: with fewer they took up to twice as long as the tiles below, now and before (us): i8 1,000,000 x 130 x 768 638
+    // least four, or three where what the tiles do besides their columns is more (distances; e2m3, which widens: 2038 x 10,937 x 77 43 us
+    // and 113, u4 angular 436 x 39,391 x 122 55 and 90; of 240 such shapes two in a hundred were slower): with fewer they took up to twice as long as the tiles below, now and before (us): i8 1,000,000 x 130 x 768 638
     // and 447, angular 817 and 482; bf16 200,000 x 129 x 768 227 and 152; u8 714 x 25,854 x 198 (three to a strip) 31 and 26. On
     // lines there are no partial ones to save, and a row has to be 32,768 long: i8 euclidean 349,434 x 448 x 64 279 and 151, 6718 x
-    // 20,000 x 448 172 and 150; two stages also take 512 MiB (u4 947 x 85,152 x 64 75 and 67).
+    // 20,000 x 448 172 and 150; two stages also take 512 MiB (u4 947 x 85,152 x 64 75 and 67). Deep distances of the types whose tiles
+    // widen A or sum its bytes: 8192 (e2m3 angular 14,922 x 18,880 x 2041 715 and 1073, u4 angular 1.19 times as fast in the mean of
+    // 110 shapes; of i8 and of u8 euclidean half of the shapes would lose by it).
     // Two dot products of integers do not gain by whole lines: deep ones into rows on the memory's sectors, whose partial lines cost it
     // little (i4 3276 x 27,600 x 1920 267 and 210), and those that take two strips of 64 rows where one tile of 128 holds all
-    // rows of A and reads the image once (u8 angular 109 x 242,980 x 1792 156 and 138).
+    // rows of A and reads the image once (u8 angular 109 x 242,980 x 1792 156 and 138). Nor do those of little work, two stages into a C
+    // that the last-level cache takes in (u1 135 x 138,111 x 98 46 and 35, i4 5384 x 4087 x 212 48 and 38, bf16 5377 x 4053 x 29 47 and
+    // 39; of 900 such shapes up to 96 MiB, 112 of the narrow types, half were slower). The 4-bit types' tiles stage half of the bytes: not
+    // deep ones whose image no cache holds and every 64 rows would read again (u4 1239 x 188,257 x 1567 741 and 555), and on lines
+    // none below 512 MiB (u4 793 x 137,216 x 317 142 and 116) or of two stages (u4 161 x 1,191,936 x 75 265 and 238, u1 640 x 212,864 x 55 136
+    // and 130). The bytes' rows on 16 bytes, deep, with an image under 100 MiB: 0.95 of the time before as tiles in the mean of 34.
     auto strips_pay = [&](GemmArgs const &args, bool lines, uint64_t mib) -> bool {
         if constexpr (T::kDeepOnly) return false;
         uint32_t const stages = args.k_chunks / kStageChunks;
-        bool const norms = args.metric != 0;
+        bool const norms = args.metric != 0, nibbles = T::kDtype == kI4 || T::kDtype == kU4;
         if (!strips_possible<T>(args) || stages > 16 || args.n <= 2048) return false;
         if (lines) {
-            if (args.m <= 64 || mib < (norms || stages > 2 ? 256 : 512) || args.n < 32768) return false;
+            bool const wide_terms = norms && stages > 8 && (nibbles || T::kDtype == kE2M3 || (T::kDtype == kU8 && args.metric == 1));
+            if (args.m <= 64 || mib < (norms || (stages > 2 && !nibbles) ? 256 : 512) || args.n < (wide_terms ? 8192u : 32768u)) return false;
+            if (!norms && stages <= 2 && (nibbles || T::kDtype == kU1)) return false;
             if (T::kChunked ? !norms && stages > 8 : norms ? stages > 2 && stages <= 8 && (stages > 4 || mib < 512) : stages > 4) return false;
         }
         else {
-            if (mib < (stages <= 2 ? 64 : 96)) return false;
+            if (mib < (stages > 2 ? 96 : norms || T::kDtype == kE2M3 ? 64 : nibbles || T::kDtype == kU1 ? 112 : 96)) return false;
             uintptr_t const rows_at = (uintptr_t)args.c | args.c_stride;
-            if (!T::kChunked && !norms && ((stages > 8 && (rows_at & 31) == 0) || (stages > 4 && (rows_at & 63) == 0))) return false;
+            uint64_t const image_mib = ((uint64_t)args.n_tiles * args.k_chunks * kTileRows * T::kImageChunk) >> 20;
+            uintptr_t const sector = (T::kDtype == kI8 || T::kDtype == kU8) && image_mib < 100 ? 15 : 31;
+            if (!T::kChunked && !norms && ((stages > 8 && ((rows_at & sector) == 0 || (nibbles && image_mib >= 256))) || (stages > 4 && (rows_at & 63) == 0))) return false;
             if (!T::kChunked && args.m > 64 && args.m <= 128 && strip_rows(args.m, stages) == 64) return false;
         }
-        return strip_plan(args.m, args.n, strip_rows(args.m, stages)).strip_tiles >= 4;
+        return strip_plan(args.m, args.n, strip_rows(args.m, stages)).strip_tiles >= (norms || T::kDtype == kE2M3 ? 3 : 4);
     };
     // Where storing C is most of the work, what counts is how much of it there is, against the 256 MiB of the last-level
     // cache above all, and whether its rows start on lines. Drawn through 980 random shapes (33 to 8192 rows, depths of 1 to 64

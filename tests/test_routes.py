@@ -50,12 +50,15 @@ def test_planning_takes_no_time():
 
 # Products for which strips were once chosen and took 1.1 to 2 times as long as the tiles that had them before: rows of C of a few
 # tiles, strips of three, long rows that start on lines anyway, deep products of integers into rows on the memory's sectors, two
-# strips of 64 rows where one tile holds all rows.
+# strips of 64 rows where one tile holds all rows, two stages into a C that the last-level cache takes in, 4-bit types with an image
+# that it does not.
 @pytest.mark.parametrize("dtype, metric, m, n, k", [
     ("i8", "dots", 1_000_000, 130, 768), ("i8", "angular", 1_000_000, 130, 768), ("bf16", "dots", 200_000, 129, 768), ("u8", "angular", 50_000, 600, 300),
     ("e4m3", "angular", 40_000, 1001, 256), ("u8", "dots", 714, 25_854, 198), ("bf16", "dots", 3340, 6513, 64), ("i8", "euclidean", 349_434, 448, 64),
     ("i8", "euclidean", 6718, 20_000, 448), ("u4", "dots", 947, 85_152, 64), ("i4", "dots", 3276, 27_600, 1920), ("u1", "dots", 25_065, 4016, 896),
-    ("u8", "angular", 109, 242_980, 1792)])
+    ("u8", "angular", 109, 242_980, 1792), ("u1", "dots", 135, 138_111, 98), ("u1", "dots", 8733, 2341, 18), ("i4", "dots", 5384, 4087, 212), ("bf16", "dots", 5377, 4053, 29),
+    ("u4", "dots", 1239, 188_257, 1567), ("u4", "dots", 793, 137_216, 317), ("u4", "dots", 161, 1_191_936, 75), ("u1", "dots", 640, 212_864, 55),
+    ("i8", "dots", 2876, 15_004, 1500)])
 def test_no_strips_where_they_do_not_pay(dtype, metric, m, n, k):
     assert route_of(dtype, metric, m, n, k).shape != STRIPS
 
@@ -63,10 +66,19 @@ def test_no_strips_where_they_do_not_pay(dtype, metric, m, n, k):
 # ... and those that they are for.
 @pytest.mark.parametrize("dtype, metric, m, n, k", [
     ("u8", "euclidean", 1000, 500_009, 301), ("f16", "dots", 8192, 8191, 1000), ("i8", "dots", 1024, 204_801, 220), ("bf16", "dots", 527, 400_384, 192),
-    ("i8", "angular", 30_000, 2301, 128), ("bf16", "euclidean", 63_086, 5932, 128), ("u8", "angular", 1025, 279_648, 1500), ("e4m3", "dots", 407, 580_128, 340)])
+    ("i8", "angular", 30_000, 2301, 128), ("bf16", "euclidean", 63_086, 5932, 128), ("u8", "angular", 1025, 279_648, 1500), ("e4m3", "dots", 407, 580_128, 340), ("e2m3", "angular", 14_922, 18_880, 2041),
+    ("u4", "angular", 17_068, 14_720, 2000), ("u8", "angular", 14_922, 18_880, 2041)])
 def test_strips_where_they_pay(dtype, metric, m, n, k):
     route = route_of(dtype, metric, m, n, k)
     assert route.shape == STRIPS and route.strip_tiles >= 4
+
+
+# Strips of three tiles where a tile has more to do besides its columns; they were left out with the others for a while, at up to
+# 2.7 times the time.
+@pytest.mark.parametrize("dtype, metric, m, n, k", [("e2m3", "dots", 2038, 10_937, 77), ("i8", "angular", 1219, 13_997, 179), ("u4", "angular", 436, 39_391, 122), ("bf16", "euclidean", 500, 35_913, 91)])
+def test_short_strips(dtype, metric, m, n, k):
+    route = route_of(dtype, metric, m, n, k)
+    assert route.shape == STRIPS and route.strip_tiles == 3
 
 
 # Tiles chosen by the bytes of C that were slower than the larger ones in use before, by up to 1.4 times: deep distances into rows off
