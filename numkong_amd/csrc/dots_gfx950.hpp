@@ -2690,6 +2690,10 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // Two tiles of 64 rows read the image twice, which is most of a deep product of few rows (u4 74 x 178,464 x 1664 89 us and 76
         // through 128 x 128, i8 angular 79 x 269,824 x 2122 207 and 168).
         if (!T::kChunked && args.m <= 128 && stages > (norms ? 16 : 4)) return 0;
+        // Three tiles of 64 rows, but four of them in two of 128: 128 x 128 gains nothing by its second workgroup there (e5m2 angular 133 x
+        // 1,285,455 x 3780 4683 us and 3272 before it, bf16 euclidean 133 x 419,427 x 2376 1073 and 830, f16 angular 192 x 252,615 x 1731
+        // 481 and 461) but for deep rows into a middling C off the lines (1.1 times as fast).
+        if (T::kChunked && norms && args.m > 128 && args.m <= 192 && (lines || stages < 32 || mib >= 300 || args.m <= 144)) return 0;
         if (!lines) {
             // (Shallow products into so large a C belong to strips or, where those do not pay, to the rule at the end.)
             if (stages <= 16 && mib >= (stages <= 2 ? 64 : 96)) return 0;

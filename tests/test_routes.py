@@ -88,3 +88,9 @@ def test_short_strips(dtype, metric, m, n, k):
     ("u4", "euclidean", 90, 251_584, 3306, 3), ("i8", "angular", 79, 269_824, 2122, 3), ("u4", "dots", 74, 178_464, 1664, 3), ("i8", "dots", 216_199, 256, 384, 1)])
 def test_larger_tiles_where_the_operands_weigh_most(dtype, metric, m, n, k, tile):
     assert route_of(dtype, metric, m, n, k).shape in (1, 2) if tile < 3 else route_of(dtype, metric, m, n, k).shape == tile
+
+
+# Three tiles of 64 rows that were taken as four in two of 128, distances of the two-accumulator types (up to 1.4 times the time before).
+@pytest.mark.parametrize("dtype, metric, m, n, k", [("e5m2", "angular", 133, 1_285_455, 3780), ("bf16", "euclidean", 133, 419_427, 2376), ("f16", "angular", 192, 252_615, 1731), ("e3m2", "angular", 192, 342_208, 1408)])
+def test_rows_of_three_small_tiles(dtype, metric, m, n, k):
+    assert route_of(dtype, metric, m, n, k).shape != 3
