@@ -2684,7 +2684,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         uint32_t const stages = args.k_chunks / kStageChunks;
         uint64_t const mib = ((uint64_t)args.m * args.n * 4) >> 20;
         bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0, norms = args.metric != 0;
-        bool const whole = args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
+        bool const whole = args.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0, nibbles = T::kDtype == kI4 || T::kDtype == kU4;
         if (strips_pay(args, lines, mib)) return 7;
         if (args.m <= 64) return 0;
         // Two tiles of 64 rows read the image twice, which is most of a deep product of few rows (u4 74 x 178,464 x 1664 89 us and 76
@@ -2710,14 +2710,16 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         if (T::kChunked && norms) return stages > 16 && stages < 32 && mib >= 64 ? 3 : 0;
         if (T::kChunked) {
             if (mib < 96) return stages > 2 && (stages <= 16 || (stages < 32 && !whole)) ? 4 : 0;
-            if (stages <= 4) return stages > 2 && mib < 256 ? 4 : 0;
-            return (stages <= 16 && (stages > 8 || mib < 256)) || (stages > 16 && stages < 32 && !whole) ? 3 : 0;
+            if (stages <= 2) return 0;
+            if (stages <= 4 && mib < 256) return 4;
+            return stages <= 16 || (stages < 32 && !whole) ? 3 : 0; // (f16 4542 x 16,384 x 324 113 us, 167 through the largest tile)
         }
         if (!norms) {
             if (stages > 16) return 0;
             if (mib < 96) return stages <= 8 || mib >= 32 ? 4 : 0; // (i8 2048^3 28.0 us through 128 x 128, 28.8 through 64 x 128)
-            if (stages <= 4) return stages > 2 && mib < 256 ? 4 : 0;
-            return stages <= 8 && mib < 512 ? 3 : 0;
+            if (stages <= 4) return stages <= 2 ? 0 : mib < 256 || T::kDtype == kE2M3 ? 4 : 3;
+            // (e2m3's 128 x 512 tile, and 256 x 256 of the bytes, are as fast or faster: e2m3 409 x 197,504 x 960 221 us through 128 x 128, 207)
+            return stages <= 8 && mib < (nibbles || T::kDtype == kU1 ? 512 : T::kDtype == kE2M3 ? 130 : 200) ? 3 : 0;
         }
         if (stages > 16) return stages < 32 && mib < 96 ? 4 : 0;
         if (mib < 256) return stages <= 8 || mib < 96 ? 4 : 3;

@@ -94,3 +94,10 @@ def test_larger_tiles_where_the_operands_weigh_most(dtype, metric, m, n, k, tile
 @pytest.mark.parametrize("dtype, metric, m, n, k", [("e5m2", "angular", 133, 1_285_455, 3780), ("bf16", "euclidean", 133, 419_427, 2376), ("f16", "angular", 192, 252_615, 1731), ("e3m2", "angular", 192, 342_208, 1408)])
 def test_rows_of_three_small_tiles(dtype, metric, m, n, k):
     assert route_of(dtype, metric, m, n, k).shape != 3
+
+
+# Into large C on lines: dots of the two-accumulator types of 3 to 16 stages went through their largest tile, which is slower than it was
+# before it folded every two stages, by 1.1 times; 128 x 128 takes two thirds of its time. e2m3 keeps its 128 x 512 tile.
+@pytest.mark.parametrize("dtype, m, n, k, shape", [("f16", 4542, 16_384, 324, 3), ("e5m2", 3228, 25_856, 195, 3), ("bf16", 3503, 26_176, 232, 3), ("i4", 4911, 30_208, 288, 3), ("e2m3", 409, 197_504, 960, 5)])
+def test_tiles_into_large_results_on_lines(dtype, m, n, k, shape):
+    assert route_of(dtype, "dots", m, n, k).shape == shape
