@@ -2700,9 +2700,18 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             // Depths at which the MFMAs are most of the work again: the largest tiles, once there are enough of them (e2m3 euclidean
             // 78,940 x 2733 x 12,009 5265 through 128 x 128 and 3664 through 256 x 256, f16 5825 x 48,330 x 5312 4360 and 4006; dots
             // e4m3 755 x 53,520 x 5376 458 and 425).
-            if (norms && !T::kChunked) return stages <= 16 || mib < 32 ? 4 : stages <= 32 || (stages <= 60 && mib < 256) ? 3 : 0;
-            if (norms) return stages > 16 && mib >= 96 && (stages <= 60 || mib < 300) ? 3 : 0;
-            if (T::kChunked) return mib >= 32 && ((stages > 4 && mib < 96) || (stages > 16 && mib < 256)) && stages <= 60 ? 3 : 0;
+            // How deep those begin was timed at 2000 shapes, 128 x 128 against the largest tile: e2m3, whose largest is 128 x 512, 0.89
+            // of its time at 24 to 32 stages into 256 MiB and more, u4 1.18 and 1.05 up to 60; of the 8-bit floats into rows that
+            // start on odd words 1.05 to 1.16 up to 90 (into rows on halves of lines e4m3 755 x 53,520 x 5376 as above), bf16 0.95, dots 1.04 to 1.12.
+            bool const odd_rows = (((uintptr_t)args.c | args.c_stride) & 7) != 0;
+            if (norms && !T::kChunked) {
+                if (stages <= 16 || mib < 32) return 4;
+                uint32_t const deepest = T::kDtype == kE2M3 ? (mib < 256 ? 40 : 16) : mib < 256 || T::kDtype == kU4 ? 60 : 32;
+                return stages <= deepest ? 3 : 0;
+            }
+            uint32_t const deepest = odd_rows && (!norms || T::kDtype == kE4M3 || T::kDtype == kE5M2) ? 90 : 60;
+            if (norms) return stages > 16 && mib >= 96 && (stages <= deepest || mib < 300) ? 3 : 0;
+            if (T::kChunked) return mib >= 32 && ((stages > 4 && mib < 96) || (stages > 16 && mib < 256)) && stages <= deepest ? 3 : 0;
             return stages <= 16 && mib < 96 ? 4 : 0;
         }
         // (two columns of tiles: A is read twice by the small ones; i8 216,199 x 256 x 384 94 and 62 through 256 x 256)

@@ -101,3 +101,10 @@ def test_rows_of_three_small_tiles(dtype, metric, m, n, k):
 @pytest.mark.parametrize("dtype, m, n, k, shape", [("f16", 4542, 16_384, 324, 3), ("e5m2", 3228, 25_856, 195, 3), ("bf16", 3503, 26_176, 232, 3), ("i4", 4911, 30_208, 288, 3), ("e2m3", 409, 197_504, 960, 5)])
 def test_tiles_into_large_results_on_lines(dtype, m, n, k, shape):
     assert route_of(dtype, "dots", m, n, k).shape == shape
+
+
+# How deep 128 x 128 goes on into rows off the lines (see by_bytes_of_c).
+@pytest.mark.parametrize("dtype, metric, m, n, k, shape", [("e4m3", "euclidean", 6080, 40_457, 4682, 3), ("bf16", "dots", 667, 47_635, 5376, 3), ("f16", "euclidean", 5001, 49_001, 5312, 2), ("e2m3", "euclidean", 4000, 40_001, 3500, 1),
+                                                           ("u4", "euclidean", 4000, 40_001, 6400, 3)])
+def test_depth_of_the_middling_tile(dtype, metric, m, n, k, shape):
+    assert route_of(dtype, metric, m, n, k).shape == shape
