@@ -2642,7 +2642,8 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // widen A or sum its bytes: 8192 (e2m3 angular 14,922 x 18,880 x 2041 715 and 1073, u4 angular 1.19 times as fast in the mean of
     // 110 shapes; of i8 and of u8 euclidean half of the shapes would lose by it).
     // Two dot products of integers do not gain by whole lines: deep ones into rows on the memory's sectors, whose partial lines cost it
-    // little (i4 3276 x 27,600 x 1920 267 and 210), and those that take two strips of 64 rows where one tile of 128 holds all
+    // little (i4 3276 x 27,600 x 1920 267 and 210; not e2m3, whose tiles widen: 1.15 to 1.29 times as fast as strips in the mean of 700
+    // such shapes), and those that take two strips of 64 rows where one tile of 128 holds all
     // rows of A and reads the image once (u8 angular 109 x 242,980 x 1792 156 and 138). Nor do those of little work, two stages into a C
     // that the last-level cache takes in (u1 135 x 138,111 x 98 46 and 35, i4 5384 x 4087 x 212 48 and 38, bf16 5377 x 4053 x 29 47 and
     // 39; of 900 such shapes up to 96 MiB, 112 of the narrow types, half were slower). The 4-bit types' tiles stage half of the bytes: not
@@ -2665,7 +2666,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             uintptr_t const rows_at = (uintptr_t)args.c | args.c_stride;
             uint64_t const image_mib = ((uint64_t)args.n_tiles * args.k_chunks * kTileRows * T::kImageChunk) >> 20;
             uintptr_t const sector = (T::kDtype == kI8 || T::kDtype == kU8) && image_mib < 100 ? 15 : 31;
-            if (!T::kChunked && !norms && ((stages > 8 && ((rows_at & sector) == 0 || (nibbles && image_mib >= 256))) || (stages > 4 && (rows_at & 63) == 0))) return false;
+            if (!T::kChunked && T::kDtype != kE2M3 && !norms && ((stages > 8 && ((rows_at & sector) == 0 || (nibbles && image_mib >= 256))) || (stages > 4 && (rows_at & 63) == 0))) return false;
             if (!T::kChunked && args.m > 64 && args.m <= 128 && strip_rows(args.m, stages) == 64) return false;
         }
         return strip_plan(args.m, args.n, strip_rows(args.m, stages)).strip_tiles >= (norms || T::kDtype == kE2M3 ? 3 : 4);
