@@ -1153,8 +1153,12 @@ __device__ __forceinline__ void fetch_to_lds(__amdgpu_buffer_rsrc_t rsrc, lds_vo
  *  64 MFMAs. Whole calls, before and now (us): bf16 8192 x 8192 x 1024 184 and 172, 4096 x 4096 x 768 57 and 52, 1000 x 100,000 x
  *  300 263 and 235; e3m2 the same 224 and 193; all pairs of 8192 x 768 119 and 109; the same bits.
  */
-// (Workgroups per compute unit: 128 x 128 with two accumulator sets needs 232 to 256 registers, so two of them fit; left to one, the
-// compiler takes 300. bf16 angular 1024 x 262,144 x 768 768 us through 64 x 128, the best before, and 684.)
+// (Workgroups per compute unit: two of 128 x 128 also with two accumulator sets; left to one, the compiler takes 300 registers. The kernels of
+// dots on rows at dwords, four stages or more, and those of all pairs need 232 to 255 for that. The others spill: of the 16-bit floats
+// distances 6 to 11 registers, 21 on shifted rows, dots on those 2 to 5, two stages 17 and 28; of the 8-bit ones 3 to 8 for distances on
+// shifted rows or of two stages. Two are faster all the same: bf16 angular 1024 x 262,144 x 768 768 us through 64 x 128, the best before, and
+// 684; distances of 17 to 60 stages, 3000 shapes, 64 x 128 1.10 and 128 x 256 1.26 times the time in the mean, on shifted rows 1.07 to 1.12 and 1.18
+// to 1.52 by type.)
 template <class T, int TM, int TN, bool ACROSS, bool NORMS = false, bool WHOLE = false, bool DIRECT = false, bool SHIFTED = false, bool FOLDS = false, bool SELF = false>
 __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * TN <= 4 ? 2 : 1))) void dots_packed_kernel(GemmArgs g) {
     typedef typename T::acc_t acc_t;
@@ -2830,12 +2834,12 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         // to 16 stages 1.22 and 0.79, deeper 1.08 and 0.85; integers of 2 stages 1.09 and 0.80, of 3 and 4 1.22 and 0.96, of 5
         // to 8 1.32 and 0.90, deeper 1.15 and 0.80 (16 in 1000 of all shapes lose more than 3 per cent); of the best tile at
         // each, 0.96. Those launches wrote the same C over and over; going round three sets of operands and results, 8000 random
-        // shapes, the mean is 1.06 and 23 in 1000 lose more than 3 per cent. Some of them (us): i8 1000 x 500,009 x 304 1226 through 64 x 128 and 972 through
-        // 128 x 256, 1024 x 1,000,001 x 768 2855 and 1879 through 256 x 256 (300 x 524,289 x 768, which leaves a quarter of the
-        // tall tiles empty, 377 through them and 287 through 128 x 256); i8 1024 x 204,801 x 1500 (an image of 300 MiB) 692 past
-        // the caches, 566 through 256 x 256, but 1024 x 107,521 x 1500 (158 MiB) 288 and 306; bf16 2400 x 45,857 x 900 433
-        // through 64 x 128, 354 through 128 x 128 past the caches, 533 through 128 x 256, whose kernel for ragged depths of
-        // 16-bit floats and for shifted rows spills.
+        // shapes, the mean is 1.06 and 23 in 1000 lose more than 3 per cent. Most of those that it was drawn for go through strips now. What
+        // is left comes here (see strips_pay): rows of C of up to 2048 columns, more than 16 stages, rows 16 MiB or more apart, and
+        // the integers' rows on sectors. Some of them (us, 64 x 128 and what is taken): bf16 99,543 x 1482 x 320 387 and 236 (128 x 128 past
+        // the caches, 322 through them), 2400 x 45,857 x 1500 654 and 523 (the same; 611 through 128 x 256, whose kernel for ragged depths of
+        // 16-bit floats and for shifted rows spills), i8 2000 x 100,001 x 3000 1153 and 841 (256 x 256), 1,000,000 x 130 x 768 548 and 465 (128 x
+        // 128 past the caches). Of many rows of few columns it is not always the best: i8 200,003 x 1001 x 304 372, 319 through 128 x 256.
         uint32_t const limit = T::kChunked ? 16 : 8;
         if (unaligned_rows_of_c(args) && best < 4 && depth_stages <= 2 * limit) {
             bool const shallow = depth_stages <= limit, bits = T::kDtype == kU1;
