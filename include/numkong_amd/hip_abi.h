@@ -155,17 +155,21 @@ int nk_hip_fill_rows_async(void *c, size_t m, size_t n, size_t c_stride, uint32_
 
 /** TEST HOOK, not part of the product interface: forces the tile shape of the calling thread's launches (0 = the
  *  heuristic picks; 1..6 = 256x256, 128x256, 128x128, 64x128, 128x512 (e2m3 only), 32x128 (a triangle takes 64x128 in
- *  its place), 7 = strips (where they apply, else 64x128); bit 7: a forced shape may still split a triangle; bits 8..27: spread of the workgroups' start times in 10 ns ticks, plus one; bits 28..29: 1 = outputs
+ *  its place), 7 = strips, 8 and 9 = A in registers, one or two blocks of 32 rows per wavefront (where they apply, else 64x128); bit 7: a forced shape may still split a triangle; bits 8..27: spread of the workgroups' start times in 10 ns ticks, plus one; bits 28..29: 1 = outputs
  *  stored past the caches, 2 = through them, whatever the alignment of C; bit 30: A is staged through registers also
  *  where it would go straight into LDS). The tests use it to run every shape, both kinds of store and both kinds of
  *  staging over the same cases; thread-local, so it never reaches another thread's calls. */
 void nk_hip_set_tile_config(int config);
 
-/** TEST HOOK: what a packed product with these arguments would run as, without a GPU and without launching anything (`a` and `c` are
+/** TEST HOOK: what a packed product with these arguments would run as, unless A is kept in registers (below), without a GPU and without launching anything (`a` and `c` are
  *  addresses, nothing is read there): planned[0] the tile shape as above, [1] the kind of store, [2] tiles or, of strips, pieces of work
  *  for a workgroup, [3] of strips the tiles in one. A forced shape counts. Not for f32 and f64. 0, or non-zero for refused calls. */
 int nk_hip_planned_tile(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
                         uint32_t planned[4]);
+/** TEST HOOK, as the one above: whether the call keeps A in registers instead of taking that tile. planned[0] the rows of a wavefront (0:
+ *  it does not), [1] workgroups, [2] 32-column tiles that one walks. */
+int nk_hip_planned_resident(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                            uint32_t planned[3]);
 
 /** Thread-local text of the last failure in this layer ("" if none). */
 char const *nk_hip_last_error(void);

@@ -121,6 +121,8 @@ def library() -> ctypes.CDLL:
     lib.nk_hip_set_tile_config.restype = None
     lib.nk_hip_planned_tile.argtypes = [i32, i32, sz, sz, sz, vp, sz, vp, sz, ctypes.POINTER(ctypes.c_uint32)]
     lib.nk_hip_planned_tile.restype = i32
+    lib.nk_hip_planned_resident.argtypes = lib.nk_hip_planned_tile.argtypes
+    lib.nk_hip_planned_resident.restype = i32
     lib.nk_hip_device_count.restype = i32
     lib.nk_capabilities.restype = ctypes.c_uint64
     lib.nk_configure_thread.argtypes = [ctypes.c_uint64]

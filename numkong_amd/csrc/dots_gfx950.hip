@@ -726,14 +726,27 @@ void nk_hip_set_tile_config(int config) {
     t_forced_config = config & 0x7FFFFFFF; // (bits 0..6 the shape; bit 7: a forced shape may still hand the narrow end of a triangle to small tiles; bits 8..27: start spread in 10 ns ticks + 1; bits 28..29: kind of store; bit 30: no staging straight into LDS)
 }
 
-int nk_hip_planned_tile(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
-                        uint32_t planned[4]) {
+/** What a call would run as, into t_planned. */
+static int plan_only(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride) {
     if (!m || !n || !k || dtype == kF32 || dtype == kF64) return fail_msg("nk_hip_planned_tile: no tile to choose");
     int const forced = t_forced_config;
     t_forced_config = (int)((uint32_t)forced | 0x80000000u), t_planned = {};
     int const status = product_async(dtype, metric, a, (void const *)256, c, m, n, k, a_stride, c_stride, nullptr); // (launches nothing, reads nothing)
     t_forced_config = forced;
+    return status;
+}
+
+int nk_hip_planned_tile(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                        uint32_t planned[4]) {
+    int const status = plan_only(dtype, metric, m, n, k, a, a_stride, c, c_stride);
     planned[0] = t_planned.shape, planned[1] = t_planned.store_policy, planned[2] = t_planned.units, planned[3] = t_planned.strip_tiles;
+    return status;
+}
+
+int nk_hip_planned_resident(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                            uint32_t planned[3]) {
+    int const status = plan_only(dtype, metric, m, n, k, a, a_stride, c, c_stride);
+    planned[0] = t_planned.resident_rows, planned[1] = t_planned.resident_units, planned[2] = t_planned.resident_tiles;
     return status;
 }
 

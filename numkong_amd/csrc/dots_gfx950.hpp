@@ -72,7 +72,10 @@ struct GemmArgs {
     uint32_t tiles_m, tiles_n;
     int avec; // widest load the A pointer and stride allow (1, 2, 4, 8 or 16 bytes)
     int metric; // 0: dot products, 1: angular distances, 2: euclidean distances (kernels built with NORMS)
-    uint32_t chunk_stages; // chunked types: stages between folds of the accumulator (even, 2..16)
+    union {
+        uint32_t chunk_stages; // chunked types: stages between folds of the accumulator (even, 2..16)
+        uint32_t strip_waves;  // dots_resident_kernel, which folds every two: wavefronts of a workgroup that have rows
+    };
     // Symmetric products (C = A x A^T, upper triangle): only elements with col >= row + tri_shift are stored
     // (`tri_mask` all ones; 0 switches the test off), and the tiles to compute come as a list.
     uint32_t tri_shift, tri_mask;
@@ -145,6 +148,7 @@ int forced_tile_config();
  *  here and not launched. */
 struct PlannedTile {
     uint32_t shape, store_policy, units, strip_tiles;
+    uint32_t resident_rows, resident_units, resident_tiles; // A in registers instead (nk_hip_planned_resident; rows 0: not)
 };
 PlannedTile *planned_tile();
 /** Compute units of the current device, asked once per process. */
@@ -2385,11 +2389,354 @@ __global__ __launch_bounds__(64 * kStripWaves, 2) void dots_strips_kernel(GemmAr
     }
 }
 
+/**
+ *  Shallow products into a large C with A in registers. A workgroup of 8 wavefronts holds its rows of A (32*TM per wavefront, whole
+ *  depth) as the MFMA wants them and walks along the columns of C, one 32-column tile of the image at a time. The tile comes straight
+ *  from the image, which lies in the order of the fragments, into a ring of LDS tiles, kSlots - 1 ahead; every wavefront reads it there,
+ *  multiplies it with its own rows and stores 128 bytes of each. One barrier per tile, and nothing is staged.
+ *
+ *  Why: such products are bound by the memory, and what keeps a copy's rate from them is the reading. Writes of C in any of the shapes
+ *  below reach 5.2 TB/s, and reads of as many bytes as B has beside them take their own time more (1024 x 1,048,576 results and 768 bytes a
+ *  column, no arithmetic: 872 us written, 130 read, 1030 to 1040 both, as long as every byte is asked for once), but with every line of B
+ *  asked for by eight workgroups at about the same time, as tiles of 128 rows do, both take 1280, however far ahead they ask: what a
+ *  compute unit reads waits in one queue with what it writes. Here B is read once per 256 rows (TM 1) or 512.
+ *
+ *  Whole calls, before and now (us): i8 1024 x 1,048,576 x 768 1363 (256 x 256 tiles) and 1080, 1000 x 500,032 x 700 803 and 557, f16
+ *  8192 x 8191 x 500 149 (strips) and 104, 1000 x 300,009 x 600 650 and 481, i8 angular 1024 x 524,288 x 768 870 and 667; the same bits.
+ *
+ *  CARRY: rows of C that do not start on 128-byte lines. What is stored is whole lines all the same: the results of a row are
+ *  rotated by its distance from a line (ds_bpermute), and what belongs to its next line waits in registers for the next tile.
+ */
+constexpr int kResidentWaves = 8;
+template <class T, int TM, int STAGES, int METRIC, bool CARRY>
+__global__ __launch_bounds__(64 * kResidentWaves, 2) void dots_resident_kernel(GemmArgs g) {
+    typedef typename T::acc_t acc_t;
+    typedef typename T::norm_t norm_t;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) uint8_t global_u8_t;
+    typedef __attribute__((address_space(1))) uint32_t global_u32_t;
+    constexpr int BM = TM * 32, kSteps = STAGES * 4, kRows = kResidentWaves * BM;
+    constexpr int kStepBytes = 1024; // of a 32-column tile, what one MFMA step takes
+    static_assert(T::kImageChunk == 16, "the image holds the fragments");
+    constexpr int kTileBytes = kSteps * kStepBytes;
+    constexpr int kSlots = STAGES > 8 ? 3 : 4;
+    constexpr int kFetches = kTileBytes / 1024 / kResidentWaves; // per wavefront and tile
+    static_assert(kFetches * kResidentWaves * 1024 == kTileBytes, "every wavefront fetches as much: the waits count on it");
+    constexpr bool kChunked = T::kChunked;
+    __shared__ __attribute__((aligned(1024))) uint8_t ring0[kTileBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t ring1[kTileBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t ring2[kTileBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t ring3[kSlots > 3 ? kTileBytes : 16];
+    __shared__ __attribute__((aligned(16))) uint32_t row_terms[T::kUnsigned ? kRows : 4]; // as in dots_packed_kernel
+    __shared__ __attribute__((aligned(16))) uint32_t row_norms[METRIC != 0 ? kRows : 4];
+    __shared__ __attribute__((aligned(16))) float row_factors[METRIC == 1 ? kRows : 4];
+    uint32_t const tid = threadIdx.x, lane = tid & 63;
+    uint32_t const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t const half = lane >> 5, col_in_tile = lane & 31;
+
+    PackedHeader const *header = (PackedHeader const *)g.bp;
+    bool const image_ok = header->magic == kMagic && header->version == kVersion &&
+                          header->dtype == (uint32_t)T::kDtype && header->n == g.n && header->k == g.k &&
+                          header->k_chunks == g.k_chunks && header->n_tiles == g.n_tiles;
+    uint8_t const *data = g.bp + sizeof(PackedHeader);
+    uint32_t const *col_terms = (uint32_t const *)(data + (uint64_t)g.n_tiles * kTileBytes);
+    uint32_t const *col_norms = col_terms + (uint64_t)g.n_tiles * kTileRows;
+    uint32_t const waves = g.strip_waves, block_rows = waves * BM; // (the wavefronts that have rows)
+    uint32_t tile_m, strip;
+    tile_of_block(blockIdx.x, g, tile_m, strip);
+    uint32_t const first = strip * g.strip_tiles;
+    if (first >= g.n_tiles) return;
+    uint32_t const count = g.n_tiles - first < g.strip_tiles ? g.n_tiles - first : g.strip_tiles;
+    if (!image_ok) { // the image was not packed for this call: the reference's error convention, all bits set
+        for (uint32_t row = tile_m * block_rows; row < tile_m * block_rows + block_rows && row < g.m; ++row)
+            for (uint32_t col = first * 32 + tid; col < (first + count) * 32 && col < g.n; col += 64 * kResidentWaves)
+                *(global_u32_t *)((global_u8_t *)g.c + (uint64_t)row * g.c_stride + (uint64_t)col * 4) = 0xFFFFFFFFu;
+        return;
+    }
+    uint32_t const row0 = tile_m * block_rows + wave * BM;
+    bool const works = wave < waves && row0 < g.m; // (a wavefront without rows helps to fetch)
+
+    auto ring_of = [&](auto slot_tag) -> uint8_t * {
+        constexpr int slot = decltype(slot_tag)::value % kSlots;
+        return slot == 0 ? ring0 : (slot == 1 ? ring1 : (slot == 2 ? ring2 : ring3));
+    };
+    // Tile t of the strip on its way into LDS, 1 KiB per instruction (past the strip's end its last one again, which nobody reads).
+    auto fetch = [&](uint32_t t, auto slot_tag) __attribute__((always_inline)) {
+        uint32_t const tile = __builtin_amdgcn_readfirstlane(first + (t < count ? t : count - 1));
+        __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(data + (uint64_t)tile * kTileBytes), 0, kTileBytes, 0x00020000);
+#pragma unroll
+        for (int at = 0; at < kFetches * kResidentWaves; at += kResidentWaves)
+            fetch_to_lds(rsrc, (lds_void_t *)(ring_of(slot_tag) + (at + wave) * 1024), (at + wave) * 1024 + lane * 16, 0);
+    };
+    fetch(0, slot_c<0>()), fetch(1, slot_c<1>());
+    if constexpr (kSlots > 3) fetch(2, slot_c<2>());
+
+    // The wavefront's rows of A: lane l takes row l % 32 of each 32-row block and chunk 2q + l / 32. Rows may start on any byte:
+    // the aligned dwords that hold a chunk, one more than the chunk has, and a shift.
+    v4i a[kSteps][TM];
+    if (works) {
+        uint32_t const skew = (uint32_t)((uint64_t)g.a + (uint64_t)row0 * g.a_stride) & 3u;
+        uint8_t const *base = g.a + (uint64_t)row0 * g.a_stride - skew;
+        uint32_t const rows_here = g.m - row0 < (uint32_t)BM ? g.m - row0 : (uint32_t)BM;
+        uint32_t const bytes = (skew + (rows_here - 1) * (uint32_t)g.a_stride + (uint32_t)g.k_src_bytes + 3u) & ~3u;
+        __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00020000);
+        constexpr int kWords = (T::kSrcChunk + 3) / 4;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            uint32_t const at = skew + (i * 32 + col_in_tile) * (uint32_t)g.a_stride + half * T::kSrcChunk, shift = at & 3u;
+            uint32_t sum = 0;
+            norm_t squares[4] = {0, 0, 0, 0}; // (of the chunks at positions 2 * (q % 4) + half of their stages)
+#pragma unroll
+            for (int q = 0; q < kSteps; ++q) {
+                uint32_t const offset = (at & ~3u) + 2 * q * T::kSrcChunk;
+                uint32_t word[5] = {0, 0, 0, 0, 0};
+                if constexpr (T::kSrcChunk == 16) {
+                    v4i const wide = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, 0));
+                    word[0] = (uint32_t)wide[0], word[1] = (uint32_t)wide[1], word[2] = (uint32_t)wide[2], word[3] = (uint32_t)wide[3];
+                    word[4] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, offset + 16, 0, 0);
+                }
+                else {
+                    typedef unsigned v3u __attribute__((ext_vector_type(3)));
+                    v3u const narrow = __builtin_amdgcn_raw_buffer_load_b96(rsrc, offset, 0, 0);
+                    word[0] = narrow[0], word[1] = narrow[1], word[2] = narrow[2];
+                }
+                v4i v = {0, 0, 0, 0};
+#pragma unroll
+                for (int w = 0; w < kWords; ++w) v[w] = (int)__builtin_amdgcn_alignbyte(word[w + 1], word[w], shift);
+                // (the depth ends in the last two stages: what lies behind a row's end is cleared where the arithmetic cares)
+                uint32_t exists[kWords];
+#pragma unroll
+                for (int w = 0; w < kWords; ++w) {
+                    exists[w] = 0xFFFFFFFFu;
+                    if (tail_matters_for<T, METRIC != 0>() && q >= kSteps - 8) {
+                        int const over = (int)(uint32_t)g.k_src_bytes - (int)((2 * q + half) * T::kSrcChunk) - 4 * w, left = over < 0 ? 0 : (over > 4 ? 4 : over);
+                        exists[w] = left == 4 ? 0xFFFFFFFFu : ((1u << (8 * left)) - 1u);
+                        v[w] &= (int)exists[w];
+                    }
+                }
+                v4i const raw = v;
+                if constexpr (T::kUnsigned) {
+                    sum += sum_bytes_u8(v);
+#pragma unroll
+                    for (int w = 0; w < kWords; ++w) v[w] ^= (int)(exists[w] & 0x80808080u); // (the zeros behind a row's end stay zeros)
+                }
+                v4i const wide = T::widen(v);
+                if constexpr (METRIC != 0) squares[q % 4] += T::sumsq(raw, wide);
+                a[q][i] = wide;
+                if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            uint32_t const other = (lane ^ 32) * 4, row = wave * BM + i * 32 + col_in_tile;
+            if constexpr (T::kUnsigned) {
+                sum += (uint32_t)__builtin_amdgcn_ds_bpermute((int)other, (int)sum);
+                if (!half) row_terms[row] = sum * 128u;
+            }
+            if constexpr (METRIC != 0) {
+                norm_t total = 0;
+#pragma unroll
+                for (int position = 0; position < 8; ++position) { // (the order of dots_packed_kernel)
+                    norm_t theirs;
+                    norm_t const mine = squares[position / 2];
+                    if constexpr (sizeof(norm_t) == 8) {
+                        uint64_t const bits = __builtin_bit_cast(uint64_t, mine);
+                        uint64_t const low = (uint32_t)__builtin_amdgcn_ds_bpermute((int)other, (int)(uint32_t)bits);
+                        uint64_t const high = (uint32_t)__builtin_amdgcn_ds_bpermute((int)other, (int)(uint32_t)(bits >> 32));
+                        theirs = __builtin_bit_cast(norm_t, low | high << 32);
+                    }
+                    else theirs = (norm_t)__builtin_amdgcn_ds_bpermute((int)other, (int)mine);
+                    total += (position & 1) == (int)half ? mine : theirs;
+                }
+                uint32_t bits;
+                if constexpr (sizeof(norm_t) == 8) bits = __builtin_bit_cast(uint32_t, (float)total);
+                else bits = (uint32_t)total;
+                if (!half) {
+                    row_norms[row] = __builtin_bit_cast(uint32_t, norm_as_f32<T>(bits));
+                    if (METRIC == 1) row_factors[row] = refined_rsqrt(norm_as_f32<T>(bits));
+                }
+            }
+        }
+    }
+    auto column_of = [&](uint32_t t) { return (first + (t < count ? t : count - 1)) * kTileRows + col_in_tile; };
+    uint32_t col_term = 0, col_norm = 0;
+    if (T::kUnsigned) col_term = col_terms[column_of(0)];
+    if (METRIC != 0) col_norm = col_norms[column_of(0)];
+
+    acc_t acc[TM], total[kChunked ? TM : 1];
+    // Own fetches of the tile first (all but the `later` youngest vector memory operations have to be done), then everybody's. No
+    // fence: that would wait for the later tiles as well.
+    auto arrived = [&](auto later_tag) __attribute__((always_inline)) {
+        constexpr int later = decltype(later_tag)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070 | (later & 15) | (later >> 4) << 14); // (and this wavefront's LDS reads are done)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t carried[CARRY ? TM : 1][CARRY ? 16 : 1];
+    uint32_t const step4 = CARRY ? (uint32_t)g.c_stride & 127u : 0u; // how much further from a line the next row starts, in bytes
+    uint32_t const skew4 = CARRY ? ((uint32_t)(uint64_t)g.c + (row0 + 4 * half) * (uint32_t)g.c_stride) & 127u : 0u;
+    // A tile issues TM * 16 stores at least whatever of it exists (what does not is stored nowhere: past the end of the descriptor), so
+    // that this many operations at least are younger than its fetches when a tile is waited for.
+    constexpr int kLater = (kSlots - 1) * TM * 16 + (kSlots - 2) * kFetches;
+    auto tile = [&](uint32_t t, auto slot_tag) __attribute__((always_inline)) {
+        arrived(slot_c<(kLater < 62 ? kLater : 62)>());
+        fetch(t + kSlots - 1, slot_c<decltype(slot_tag)::value + kSlots - 1>());
+        uint8_t const *src = ring_of(slot_tag) + lane * 16;
+        constexpr int kAhead = TM == 2 && STAGES == 6 ? 2 : 3; // (fragments read ahead: registers are short there)
+        v4i b[4];
+        auto read_b = [&](int q) __attribute__((always_inline)) {
+            b[q & 3] = *(v4i const *)(src + q * kStepBytes);
+        };
+        read_b(0), read_b(1);
+        if constexpr (kAhead > 2) read_b(2);
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+            if (q + kAhead < kSteps) read_b(q + kAhead);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (kChunked && q % 8 == 0) { // (two-accumulator types: the sums go into the totals every two stages)
+                    if (q == 0) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) total[i][v] = 0;
+                    }
+                    else total[i] += acc[i];
+                }
+                if (q == 0 || (kChunked && q % 8 == 0)) T::mma_fresh(acc[i], a[q][i], b[q & 3]);
+                else T::mma(acc[i], a[q][i], b[q & 3]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        uint32_t const my_term = col_term, my_norm = col_norm;
+        if (T::kUnsigned) col_term = col_terms[column_of(t + 1)]; // (asked for in front of the stores)
+        if (METRIC != 0) col_norm = col_norms[column_of(t + 1)];
+        uint32_t const col0 = (first + t) * 32;
+        typedef __attribute__((address_space(4))) GemmArgs const late_args_t;
+        late_args_t *late = (late_args_t *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(late));
+        constexpr uint32_t kNowhere = 0x80000000u; // (the host checks that a wavefront's rows end below it)
+        uint32_t const row_step = (uint32_t)late->c_stride, n = late->n;
+        // (CARRY: from a line further left, so that offsets of lines that start in front of the tile are not negative)
+        uint8_t *const c_tile = late->c + (uint64_t)row0 * late->c_stride + (uint64_t)col0 * 4 - (CARRY ? 128 : 0);
+        uint64_t const left = (uint64_t)(late->m - row0 - 1) * late->c_stride + ((uint64_t)n - col0) * 4 + (CARRY ? 128 : 0);
+        __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)c_tile, 0, (int)(left < kNowhere ? (uint32_t)left : kNowhere), 0x00020000);
+        int const cols_left = (int)(n - col0); // of columns from this tile's first on
+        float const col_value = METRIC != 0 ? norm_as_f32<T>(my_norm) : 0.0f;
+        float const col_factor = METRIC == 1 ? refined_rsqrt(col_value) : 0.0f;
+        constexpr int kGroup = CARRY ? 8 : 16;
+        auto store_all = [&](auto edge_tag) __attribute__((always_inline)) {
+            constexpr bool edge = decltype(edge_tag)::value != 0; // (CARRY) the strip's first tile or its last
+            uint32_t offset = 4 * half * row_step + col_in_tile * 4;
+            if (CARRY) offset += 128;
+            else offset = (int)col_in_tile < cols_left ? offset : kNowhere;
+            // (the empty asm keeps these two from being worked out for every row once and held in registers)
+            uint32_t moved = skew4, lane4 = col_in_tile * 4;
+            if (CARRY) asm volatile("" : "+v"(moved), "+v"(lane4));
+            uint32_t moved_again = moved;
+            v4i row_term4 = {0, 0, 0, 0}, row_norm4 = {0, 0, 0, 0};
+            v4f row_factor4 = {0, 0, 0, 0};
+#pragma unroll
+            for (int group = 0; group < TM * 16 / kGroup; ++group) {
+                int const i = group * kGroup / 16, v0 = group * kGroup % 16;
+                uint32_t finished[kGroup];
+#pragma unroll
+                for (int v = v0; v < v0 + kGroup; ++v) {
+                    uint32_t const rows_at = wave * BM + i * 32 + 8 * (v / 4) + 4 * half;
+                    auto element = acc[i][v];
+                    if constexpr (kChunked) element += total[i][v];
+                    uint32_t bits = finished_dot<T>(__builtin_bit_cast(uint32_t, element));
+                    if (T::kUnsigned) {
+                        if (v % 4 == 0) row_term4 = *(v4i const *)&row_terms[rows_at];
+                        bits += (uint32_t)row_term4[v % 4] + my_term;
+                    }
+                    if (METRIC == 1) {
+                        if (v % 4 == 0) row_factor4 = *(v4f const *)&row_factors[rows_at];
+                        bool cheap;
+                        float const quick = angular_from_factors<T>(bits, row_factor4[v % 4], col_factor, &cheap);
+                        uint32_t result = __builtin_bit_cast(uint32_t, quick);
+                        if (__builtin_amdgcn_ballot_w64(!cheap) != 0) {
+                            int const row_bits = *(int const *)&row_norms[rows_at + v % 4];
+                            uint32_t const full = distance_from_dot<T, 1>(bits, __builtin_bit_cast(float, row_bits), col_value);
+                            result = cheap ? result : full;
+                        }
+                        bits = result;
+                    }
+                    else if (METRIC == 2) {
+                        if (v % 4 == 0) row_norm4 = *(v4i const *)&row_norms[rows_at];
+                        int const row_bits = row_norm4[v % 4];
+                        bits = distance_from_dot<T, 2>(bits, __builtin_bit_cast(float, row_bits), col_value);
+                    }
+                    finished[v - v0] = bits;
+                    if constexpr (CARRY) { // Lane p of a row that starts `moved` bytes past a line takes column p - moved / 4 of the tile.
+                        uint32_t const from = (lane4 - moved) & 124u;
+                        finished[v - v0] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(from | half * 128), (int)bits);
+                        moved = (moved + (v % 4 == 3 ? 5 : 1) * step4) & 127u;
+                    }
+                    if ((T::kUnsigned || METRIC != 0) && v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int v = v0; v < v0 + kGroup; ++v) {
+                    uint32_t bits = finished[v - v0], at = offset;
+                    if constexpr (CARRY) { // What belongs to the row's line before, this tile's first lanes, was left by the tile before.
+                        bool const before = lane4 < moved_again;
+                        bits = before ? carried[i][v] : finished[v - v0];
+                        carried[i][v] = finished[v - v0];
+                        at = offset - moved_again;
+                        if (edge) {
+                            int const column4 = (int)(lane4 - moved_again);
+                            if (t + 1 == count) // the end of the strip: what the last line of every row still lacks
+                                __builtin_amdgcn_raw_buffer_store_b32(finished[v - v0], rsrc, before && column4 + 128 < 4 * cols_left ? at + 128 : kNowhere, 0, 2);
+                            at = (t != 0 || !before) && column4 < 4 * cols_left ? at : kNowhere;
+                        }
+                        moved_again = (moved_again + (v % 4 == 3 ? 5 : 1) * step4) & 127u;
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b32(bits, rsrc, at, 0, 2); // (2: `nt`)
+                    offset += (v % 4 == 3 ? 5 : 1) * row_step;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if (!CARRY || (t != 0 && t + 1 != count)) store_all(slot_c<0>());
+        else store_all(slot_c<1>());
+    };
+    __builtin_amdgcn_s_waitcnt(0x0F70); // (all that was fetched so far is there: from here on the waits count)
+    if (!works) { // fetches only
+        auto help = [&](uint32_t t, auto slot_tag) __attribute__((always_inline)) {
+            arrived(slot_c<(kSlots - 2) * kFetches>());
+            fetch(t + kSlots - 1, slot_c<decltype(slot_tag)::value + kSlots - 1>());
+        };
+        for (uint32_t t = 0; t < count; t += kSlots) {
+            help(t, slot_c<0>());
+            if (t + 1 >= count) break;
+            help(t + 1, slot_c<1>());
+            if (t + 2 >= count) break;
+            help(t + 2, slot_c<2>());
+            if constexpr (kSlots > 3) {
+                if (t + 3 >= count) break;
+                help(t + 3, slot_c<3>());
+            }
+        }
+    }
+    else
+        for (uint32_t t = 0; t < count; t += kSlots) {
+            tile(t, slot_c<0>());
+            if (t + 1 >= count) break;
+            tile(t + 1, slot_c<1>());
+            if (t + 2 >= count) break;
+            tile(t + 2, slot_c<2>());
+            if constexpr (kSlots > 3) {
+                if (t + 3 >= count) break;
+                tile(t + 3, slot_c<3>());
+            }
+        }
+    __builtin_amdgcn_s_waitcnt(0x0F70); // (no fetch may outlive the workgroup's LDS)
+}
+
 struct TileConfig {
     int tm, tn;
 };
-// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only; 6: full grids only; 7: strips, dots_strips_kernel).
-constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}, {1, 1}, {4, 2}};
+// Index 0 is "choose for me"; 1.. are explicit (5: e2m3 only; 6: full grids only; 7: strips, dots_strips_kernel; 8 and 9: A in
+// registers, dots_resident_kernel with one and two blocks of rows).
+constexpr TileConfig kConfigs[] = {{0, 0}, {8, 2}, {4, 2}, {4, 1}, {2, 1}, {4, 4}, {1, 1}, {4, 2}, {4, 2}, {4, 2}};
 constexpr int kConfigCount = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kTriangleConfigs = 6; // the shapes below this index serve triangular grids
 
@@ -2580,7 +2927,7 @@ hipError_t launch_strips_as(GemmArgs &g, hipStream_t stream, PlannedTile *planne
     uint64_t const units = (uint64_t)g.tiles_m * g.tiles_n;
     if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
     if (planned) {
-        *planned = {7, 0, (uint32_t)units, g.strip_tiles};
+        planned->shape = 7, planned->units = (uint32_t)units, planned->strip_tiles = g.strip_tiles;
         return hipSuccess;
     }
     g.tile_count = (uint32_t)units, g.tile_list = nullptr;
@@ -2594,6 +2941,78 @@ inline uint32_t strip_rows(uint32_t m, uint32_t stages) { return m > 64 && strip
 template <class T>
 hipError_t launch_strips(GemmArgs &g, hipStream_t stream, PlannedTile *planned) {
     return strip_rows(g.m, g.k_chunks / kStageChunks) == 128 ? launch_strips_as<T, 4, 32>(g, stream, planned) : launch_strips_as<T, 2, 16>(g, stream, planned);
+}
+
+/** Which of these kernels there are. Left out are those whose registers do not fit (two-accumulator types of 12 stages; of 10 with
+ *  the angular finaliser; two blocks of rows beside anything but a plain store) or that were slower than strips: rows off the lines of up to four stages (i8
+ *  1000 x 500,009 x 301 550 and 571) and the angular finaliser there (two-accumulator types only at 8 stages, integers from 8 on), or on lines
+ *  with an integer loop of two stages. */
+template <class T, int TM, int STAGES, int METRIC, bool CARRY>
+constexpr bool resident_built() {
+    if (T::kImageChunk != 16 || T::kDeepOnly || (METRIC != 0 && !T::kDistances) || STAGES % 2 != 0 || STAGES > (T::kChunked ? 10 : 12)) return false;
+    if (TM == 2) return METRIC == 0 && !CARRY && STAGES <= (T::kChunked ? 4 : 6);
+    if (METRIC == 1 && (T::kChunked ? STAGES > 8 : STAGES < 4)) return false;
+    return !CARRY || (STAGES >= (METRIC == 1 ? 8 : 6) && STAGES <= 10);
+}
+typedef void (*resident_kernel_t)(GemmArgs);
+template <class T, int TM, int METRIC, bool CARRY, int STAGES = 2>
+resident_kernel_t resident_kernel_of(uint32_t stages) {
+    if constexpr (STAGES > 12) return nullptr;
+    else {
+        if (stages != STAGES) return resident_kernel_of<T, TM, METRIC, CARRY, STAGES + 2>(stages);
+        if constexpr (resident_built<T, TM, STAGES, METRIC, CARRY>()) return dots_resident_kernel<T, TM, STAGES, METRIC, CARRY>;
+        else return nullptr;
+    }
+}
+/** The kernel for these arguments with `tm` blocks of 32 rows per wavefront (1 or 2); NULL: there is none. */
+template <class T>
+resident_kernel_t resident_kernel(GemmArgs const &g, int tm) {
+    uint32_t const stages = g.k_chunks / kStageChunks;
+    bool const lines = (((uintptr_t)g.c | g.c_stride) & 127) == 0;
+    // (a wavefront's rows of A and of C lie within 31 bits; the two-accumulator types' sums go into their totals every two stages)
+    if (g.c_stride < 4 * (uint64_t)g.n || g.c_stride >= (1u << 24) || g.a_stride >= (1u << 24) - 1 || (T::kChunked && g.chunk_stages != 2)) return nullptr;
+    if (tm == 2) return lines && g.metric == 0 ? resident_kernel_of<T, 2, 0, false>(stages) : nullptr;
+    switch (g.metric) {
+    case 0: return lines ? resident_kernel_of<T, 1, 0, false>(stages) : resident_kernel_of<T, 1, 0, true>(stages);
+    case 1: return lines ? resident_kernel_of<T, 1, 1, false>(stages) : resident_kernel_of<T, 1, 1, true>(stages);
+    default: return lines ? resident_kernel_of<T, 1, 2, false>(stages) : resident_kernel_of<T, 1, 2, true>(stages);
+    }
+}
+/** Rows are shared out evenly over as few workgroups as hold them, and the columns are cut into strips so that whole rounds of
+ *  workgroups (one per compute unit) walk the fewest tiles, four to each strip for its start: as strip_plan. */
+struct ResidentPlan {
+    uint32_t blocks, waves, strips, strip_tiles;
+};
+inline ResidentPlan resident_plan(uint32_t m, uint32_t n_tiles, uint32_t bm) {
+    uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256, rows = kResidentWaves * (uint64_t)bm;
+    uint64_t const least = (m + rows - 1) / rows, waves = ((m + least - 1) / least + bm - 1) / bm, blocks = (m + waves * bm - 1) / (waves * bm);
+    uint64_t best = ~0ull, length = n_tiles, strips = 1;
+    for (int candidate = 0; candidate < 8; ++candidate) {
+        uint64_t const rounds = (blocks * strips + resident - 1) / resident;
+        strips = rounds * resident / blocks;
+        uint64_t const here = strips < n_tiles ? (n_tiles + strips - 1) / strips : 1;
+        if (rounds * (here + 4) < best) best = rounds * (here + 4), length = here;
+        if (here == 1) break;
+        ++strips;
+    }
+    return {(uint32_t)blocks, (uint32_t)waves, (uint32_t)((n_tiles + length - 1) / length), (uint32_t)length};
+}
+/** `planned`: nothing is launched. */
+template <class T>
+hipError_t launch_resident(GemmArgs &g, hipStream_t stream, int tm, PlannedTile *planned) {
+    resident_kernel_t const kernel = resident_kernel<T>(g, tm);
+    if (!kernel) return hipErrorInvalidValue;
+    ResidentPlan const plan = resident_plan(g.m, g.n_tiles, 32 * tm);
+    uint64_t const units = (uint64_t)plan.blocks * plan.strips;
+    if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    if (planned) {
+        planned->resident_rows = 32 * tm, planned->resident_units = (uint32_t)units, planned->resident_tiles = plan.strip_tiles;
+        return hipSuccess;
+    }
+    g.tiles_m = plan.blocks, g.tiles_n = plan.strips, g.strip_tiles = plan.strip_tiles, g.strip_waves = plan.waves;
+    g.tile_count = (uint32_t)units, g.tile_list = nullptr;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)units), dim3(64 * kResidentWaves), 0, stream, g);
+    return hipGetLastError();
 }
 
 template <class T>
@@ -2877,6 +3296,30 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         }
         return best;
     };
+    // A in registers (see dots_resident_kernel) wherever there is such a kernel, C is most of the traffic and a strip is long enough for
+    // what its start costs. Against the choice without it, rounds of three sets of operands and results: at 2800 random shapes of all types
+    // that it takes, 65 to 300,000 rows, the time is 0.81 of that before in the mean (dots 0.81, euclidean 0.81, angular 0.80), and 2 in 100
+    // of the dots and the euclidean are slower by more than 3 per cent. At 4400 more, where the lines lie: C under 64 MiB 0.98 to 1.05, strips of fewer than 12 tiles 0.98
+    // to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16 69 x 2,664,123 x 602 1.55, u4
+    // 318 x 137,089 x 1072 1.29; of workgroups with six and more of them 1 in 20 is slower).
+    // Two blocks of rows where the image does not stay in the last-level cache and reading it half as often counts (i8 1024 x 1,048,576 x
+    // 768 1195 us and 1080; 4096 x 65,536 x 500, whose image does, 256 and 266).
+    auto resident_blocks = [&](GemmArgs const &args) -> int {
+        if (triangle || args.m <= 64 || (uint64_t)args.m * args.n * 4 < (64ull << 20) || !resident_kernel<T>(args, 1)) return 0;
+        ResidentPlan const plan = resident_plan(args.m, args.n_tiles, 32);
+        if (plan.strip_tiles < 16 || (args.metric == 1 && plan.waves < 6)) return 0;
+        uint64_t const image = (uint64_t)args.n_tiles * args.k_chunks * kTileChunkBytes;
+        return args.m > 256 && image >= (128ull << 20) && resident_kernel<T>(args, 2) ? 2 : 1;
+    };
+    if (config == 8 || config == 9) {
+        if (!triangle && resident_kernel<T>(g, config - 7)) return launch_resident<T>(g, stream, config - 7, planned);
+        config = 4;
+    }
+    if (chosen_here)
+        if (int const blocks = resident_blocks(g)) {
+            hipError_t const status = launch_resident<T>(g, stream, blocks, planned);
+            if (!planned) return status;
+        }
     Choice const chosen = chosen_here ? choose(g, 1) : Choice(config);
     config = chosen.config, g.store_policy = chosen.store_policy;
     if (config == 7) {
@@ -2942,7 +3385,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         return hipSuccess;
     }
     if (planned) {
-        *planned = {(uint32_t)config, g.store_policy, (uint32_t)tiles_of(g, config), 0};
+        planned->shape = (uint32_t)config, planned->store_policy = g.store_policy, planned->units = (uint32_t)tiles_of(g, config);
         return hipSuccess;
     }
     return launch_config<T>(g, stream, triangle, config);
