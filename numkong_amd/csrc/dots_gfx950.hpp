@@ -1054,10 +1054,17 @@ struct Totals<acc_t, TM, TN, false> {
  *  with a private L2, so ids are first regrouped into 8 contiguous ranges (one per XCD) and each range
  *  walks the tile grid in column-major bands of 8 tile rows: tiles resident on one XCD at the same time
  *  share A row blocks and B column tiles in that XCD's L2.
+ *  A single row of tiles shares nothing but A. All XCDs walk it side by side, from the image's end to its start: of an image that was
+ *  packed a moment ago the end is what the last-level cache still holds (us: packed and multiplied by 16 rows, i8 1,048,576 x 768,
+ *  504.6 and 493.7; the product alone 180 and 175, angular bf16 32 x 262,144 x 768 95.3 and 93.9).
  */
 __device__ __forceinline__ void tile_of_block(uint32_t pid, GemmArgs const &g, uint32_t &tm, uint32_t &tn) {
     uint32_t const tiles_m = g.tiles_m, tiles_n = g.tiles_n;
     uint32_t const total = g.tile_count;
+    if (tiles_m == 1 && !g.tile_list) {
+        tm = 0, tn = total - 1 - pid;
+        return;
+    }
     uint32_t const per_xcd = total / 8;
     uint32_t lid = pid;
     if (pid < per_xcd * 8) lid = (pid % 8) * per_xcd + pid / 8;
