@@ -320,6 +320,7 @@ __global__ __launch_bounds__(256) void dots_f64_compensated_kernel(WideArgs g) {
     }
 }
 
+constexpr uint32_t kWideBand = 16; // tile rows per band of the walk over the tiles
 constexpr int kMatrixRows = 128, kMatrixCols = 64; // rows (at most) and columns of C per workgroup of the f32 matrix kernel
 constexpr int kMatrixDepth = 32;                     // k per step: two groups of four MFMA depths for each of the four sums
 // A row of staged A is 128 bytes of f32, eight 16-byte units; unit u of row r sits at position u ^ (r % 8), so that the
@@ -342,6 +343,13 @@ constexpr int kMatrixDepth = 32;                     // k per step: two groups o
  *  group, and widened where it is multiplied; B comes from the k-major f64 image into [k][column]. A step is 32 depths =
  *  8 IB JB MFMAs per wavefront; loads from memory are asked for a whole step before the stash that takes them, and the
  *  stash, the barrier and the reads of LDS sit between groups of MFMAs.
+ *
+ *  Which tile a workgroup takes: consecutive workgroups go to the 8 XCDs in turn, so each XCD is given a contiguous part of a walk
+ *  down bands of 16 tile rows, column by column. A column of tiles is then read by an XCD whose L2 holds it already; row by row over
+ *  the whole width, the image (51 MB for 20,001 x 300, eight bytes a value) came from behind the L2 once per row of tiles.
+ *  Whole calls, row by row and this way (us): angular 1000 x 20,001 x 300 276.5 and 273.0, dots 246.2 and 242.5, 1 x 100,000 x 1024 167.0 and
+ *  154.8, 256 x 8000 x 300 40.1 and 39.6. Not for two rows of tiles (33 x 200,000 x 200 129.9 and 131.1) nor for a triangle, whose parts
+ *  would be of unequal work.
  */
 template <bool NORMS, int IB, int JB, int WR, int WC>
 __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_matrix_kernel(WideArgs g) {
@@ -361,7 +369,14 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
     double *row_norms = &b_lds[1][0][0];
     static_assert(sizeof(double) * ROWS * 8 <= sizeof(b_lds) / 2, "the partial sums fit one stage of B");
     uint32_t const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint32_t const row0 = blockIdx.y * ROWS, col0 = blockIdx.x * kMatrixCols;
+    uint32_t tile_m = blockIdx.y, tile_n = blockIdx.x;
+    if (!g.tri_mask && gridDim.y != 2) {
+        uint32_t const across = gridDim.x, down = gridDim.y, pid = tile_m * across + tile_n, part = across * down / 8;
+        uint32_t const at = pid < part * 8 ? pid % 8 * part + pid / 8 : pid;
+        uint32_t const first = at / (kWideBand * across) * kWideBand, rows = down - first < kWideBand ? down - first : kWideBand, in_band = at % (kWideBand * across);
+        tile_m = first + in_band % rows, tile_n = in_band / rows;
+    }
+    uint32_t const row0 = tile_m * ROWS, col0 = tile_n * kMatrixCols;
     // symmetric form: a tile wholly left of the diagonal has nothing to store
     if (((row0 + g.tri_shift) & g.tri_mask) > col0 + (kMatrixCols - 1)) return;
     PackedHeader const *header = (PackedHeader const *)((uint8_t const *)g.b - sizeof(PackedHeader));
