@@ -2814,14 +2814,14 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     // trips of four stages, and for the two-accumulator types folds that fall between trips (measured at 8192^3,
     // alternating in one session: i8 0.438 -> 0.419 ms, bf16 0.930 -> 0.902, f16 0.997 -> 0.968; with a fold after every
     // second stage of the trip instead, the compiler ran out of registers in the folds and bf16 took 1.10 ms). Of 128 x 128 the
-    // integers, from 16 stages and more than two rows of tiles on (680 shapes of i8, 0.97 of the time in the mean and none slower; 2048^3 27.9
-    // and 27.1 us, 2048 x 2048 x 8192 51.4 and 49.3; shallower ones were up to 1.07 times as slow).
+    // integers, from 24 stages and more than two rows of tiles on (486 shapes of i8, 0.965 of the time in the mean; going round twelve sets of
+    // operands 2048 x 2048 x 4096 37.0 and 35.9 us, x 3072 33.1 and 32.7, but x 2560 31.0 and 31.0 and x 2048 28.7 and 29.1).
     bool direct = false;
     if constexpr (kDirectStaging && !T::kUnsigned && !T::kPrewiden && T::kSrcChunk == 16 && T::kImageChunk == 16 &&
                   ((TM == 8 && TN == 2) || (TM == 4 && TN == 1 && !T::kChunked) || (TM == 4 && TN == 2 && T::kChunked))) {
         direct = across && !norms && stages % 4 == 0 && stages >= 8 && (whole || !tail_matters_for<T, false>()) &&
                  (!T::kChunked || g.chunk_stages % 4 == 0) &&
-                 (TN == 2 || (stages >= 16 && g.m > 256)) && (g.avec >= 16) && !(forced_tile_config() & 0x40000000);
+                 (TN == 2 || (stages >= 24 && g.m > 256)) && (g.avec >= 16) && !(forced_tile_config() & 0x40000000);
         if (direct) kernel = dots_packed_kernel<T, TM, TN, true, false, tail_matters_for<T, false>(), true>;
     }
     if constexpr (T::kDistances) {
