@@ -1054,14 +1054,17 @@ struct Totals<acc_t, TM, TN, false> {
  *  with a private L2, so ids are first regrouped into 8 contiguous ranges (one per XCD) and each range
  *  walks the tile grid in column-major bands of 8 tile rows: tiles resident on one XCD at the same time
  *  share A row blocks and B column tiles in that XCD's L2.
- *  A single row of tiles shares nothing but A. All XCDs walk it side by side, from the image's end to its start: of an image that was
- *  packed a moment ago the end is what the last-level cache still holds (us: packed and multiplied by 16 rows, i8 1,048,576 x 768,
- *  504.6 and 493.7; the product alone 180 and 175, angular bf16 32 x 262,144 x 768 95.3 and 93.9).
+ *  FEW_ROWS: tiles of 32 rows, which are hardly ever more than one row of tiles and then share nothing but A. All XCDs walk that side by
+ *  side, from the image's end to its start: of an image that was packed a moment ago the end is what the last-level cache still holds (us: packed and
+ *  multiplied by 16 rows, i8 1,048,576 x 768, 504.6 and 493.7; the product alone 180 and 175, angular bf16 32 x 262,144 x 768 95.3
+ *  and 93.9). Not the taller tiles, where the choice costs registers (e2m3 of two stages a workgroup per compute unit: all pairs of 8192 x 219
+ *  53.3 and 56.3).
  */
+template <bool FEW_ROWS = false>
 __device__ __forceinline__ void tile_of_block(uint32_t pid, GemmArgs const &g, uint32_t &tm, uint32_t &tn) {
     uint32_t const tiles_m = g.tiles_m, tiles_n = g.tiles_n;
     uint32_t const total = g.tile_count;
-    if (tiles_m == 1 && !g.tile_list) {
+    if (FEW_ROWS && tiles_m == 1) {
         tm = 0, tn = total - 1 - pid;
         return;
     }
@@ -1255,7 +1258,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     auto view_of = [&](uint32_t tile) {
         TileView view;
         uint32_t tile_m, tile_n;
-        tile_of_block(tile, g, tile_m, tile_n);
+        tile_of_block<TM * TN == 1>(tile, g, tile_m, tile_n);
         view.row0 = tile_m * BM;
         view.col0 = tile_n * (128 * TN) + wave * (32 * TN);
         uint32_t const rows_here = g.m - view.row0 < (uint32_t)BM ? g.m - view.row0 : (uint32_t)BM;
@@ -1319,7 +1322,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
     if (!image_ok) { // the image was not packed for this call: the reference's error convention, all bits set
         for (uint32_t tile = blockIdx.x; tile < g.tile_count; tile += gridDim.x) {
             uint32_t tile_m, tile_n;
-            tile_of_block(tile, g, tile_m, tile_n);
+            tile_of_block<TM * TN == 1>(tile, g, tile_m, tile_n);
             for (uint32_t at = tid; at < (uint32_t)BM * 128 * TN; at += NT) {
                 uint32_t const row = tile_m * BM + at / (128 * TN), col = tile_n * (128 * TN) + at % (128 * TN);
                 if (row < g.m && col < g.n && ((row + g.tri_shift) & g.tri_mask) <= col) *(global_u32_t *)((global_u8_t *)g.c + (uint64_t)row * g.c_stride + (uint64_t)col * 4) = 0xFFFFFFFFu;
