@@ -2433,6 +2433,10 @@ __global__ __launch_bounds__(64 * kResidentWaves, 2) void dots_resident_kernel(G
     constexpr int kFetches = kTileBytes / 1024 / kResidentWaves; // per wavefront and tile
     static_assert(kFetches * kResidentWaves * 1024 == kTileBytes, "every wavefront fetches as much: the waits count on it");
     constexpr bool kChunked = T::kChunked;
+    // (three kernels whose registers fit only with two fragments read ahead: with three they reloaded 8 (u8, e2m3) and 16 (u4) of them in
+    // front of every tile's MFMAs, behind the stores. Means over 444 to 513 shapes each, against the tiles or strips they replace: u8 0.93
+    // and 0.82 of the time, u4 1.01 and 0.79, e2m3 0.93 and 0.82)
+    constexpr bool kTight = CARRY && STAGES == 10 && METRIC == 1 && (T::kDtype == kU8 || T::kDtype == kU4 || T::kDtype == kE2M3);
     __shared__ __attribute__((aligned(1024))) uint8_t ring0[kTileBytes];
     __shared__ __attribute__((aligned(1024))) uint8_t ring1[kTileBytes];
     __shared__ __attribute__((aligned(1024))) uint8_t ring2[kTileBytes];
@@ -2592,7 +2596,7 @@ __global__ __launch_bounds__(64 * kResidentWaves, 2) void dots_resident_kernel(G
         arrived(slot_c<(kLater < 62 ? kLater : 62)>());
         fetch(t + kSlots - 1, slot_c<decltype(slot_tag)::value + kSlots - 1>());
         uint8_t const *src = ring_of(slot_tag) + lane * 16;
-        constexpr int kAhead = TM == 2 && STAGES == 6 ? 2 : 3; // (fragments read ahead: registers are short there)
+        constexpr int kAhead = (TM == 2 && STAGES == 6) || kTight ? 2 : 3; // (fragments read ahead: registers are short there)
         v4i b[4];
         auto read_b = [&](int q) __attribute__((always_inline)) {
             b[q & 3] = *(v4i const *)(src + q * kStepBytes);
@@ -2632,7 +2636,9 @@ __global__ __launch_bounds__(64 * kResidentWaves, 2) void dots_resident_kernel(G
         int const cols_left = (int)(n - col0); // of columns from this tile's first on
         float const col_value = METRIC != 0 ? norm_as_f32<T>(my_norm) : 0.0f;
         float const col_factor = METRIC == 1 ? refined_rsqrt(col_value) : 0.0f;
-        constexpr int kGroup = CARRY ? 8 : 16;
+        // (Results finished before any is stored. u8 euclidean of twelve stages: 25 registers were reloaded with every tile with 16 of them;
+        // 599 shapes 0.97 and 0.75 of the time of what it replaces)
+        constexpr int kGroup = CARRY || (T::kDtype == kU8 && STAGES == 12 && METRIC == 2) ? 8 : 16;
         auto store_all = [&](auto edge_tag) __attribute__((always_inline)) {
             constexpr bool edge = decltype(edge_tag)::value != 0; // (CARRY) the strip's first tile or its last
             uint32_t offset = 4 * half * row_step + col_in_tile * 4;
@@ -2956,7 +2962,9 @@ hipError_t launch_strips(GemmArgs &g, hipStream_t stream, PlannedTile *planned) 
 }
 
 /** Which of these kernels there are. Left out are those whose registers do not fit (two-accumulator types of 12 stages; of 10 with
- *  the angular finaliser; two blocks of rows beside anything but a plain store) or that were slower than strips: rows off the lines of up to four stages (i8
+ *  the angular finaliser; two blocks of rows beside anything but a plain store): a reload in the loop would wait for the stores in front
+ *  of it. None is left that has any there (u8 dots of 10 stages off the lines and u8 angular of 12 save one register around the loading
+ *  of A). Or those that were slower than strips: rows off the lines of up to four stages (i8
  *  1000 x 500,009 x 301 550 and 571) and the angular finaliser there (two-accumulator types only at 8 stages, integers from 8 on), or on lines
  *  with an integer loop of two stages. */
 template <class T, int TM, int STAGES, int METRIC, bool CARRY>
