@@ -348,8 +348,12 @@ constexpr int kMatrixDepth = 32;                     // k per step: two groups o
  *  down bands of 16 tile rows, column by column. A column of tiles is then read by an XCD whose L2 holds it already; row by row over
  *  the whole width, the image (51 MB for 20,001 x 300, eight bytes a value) came from behind the L2 once per row of tiles.
  *  Whole calls, row by row and this way (us): angular 1000 x 20,001 x 300 276.5 and 273.0, dots 246.2 and 242.5, 1 x 100,000 x 1024 167.0 and
- *  154.8, 256 x 8000 x 300 40.1 and 39.6. Not for two rows of tiles (33 x 200,000 x 200 129.9 and 131.1) nor for a triangle, whose parts
- *  would be of unequal work.
+ *  154.8, 256 x 8000 x 300 40.1 and 39.6. Shallow products are bound by writing C instead, which row by row goes to neighbouring addresses and
+ *  this way to as many rows at once as a band has: up to 64 values deep only where there are three rows of tiles at most, up to 96
+ *  eight. Timed both ways at 3603 random shapes (1 to 5000 rows, 2000 to 300,000 columns, 32 to 2048 values): down to 64 values, the time of this
+ *  walk over the other is 1.12 at 17 and more rows of tiles (1528 x 15,837 x 41 80.0 and 109.7), 1.06 at 9 to 16, 1.00 at 4 to 8, 0.96 at up to
+ *  three; of 65 to 96 values 1.02, 1.00, 0.98 and 0.96; deeper 0.99, 0.99, 0.98 and 0.97 (two rows of tiles 0.98). Not for a triangle,
+ *  whose parts would be of unequal work.
  */
 template <bool NORMS, int IB, int JB, int WR, int WC>
 __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_matrix_kernel(WideArgs g) {
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(64 * WR * WC, IB * JB == 1 ? 4 : 2) void dots_f32_m
     static_assert(sizeof(double) * ROWS * 8 <= sizeof(b_lds) / 2, "the partial sums fit one stage of B");
     uint32_t const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t tile_m = blockIdx.y, tile_n = blockIdx.x;
-    if (!g.tri_mask && gridDim.y != 2) {
+    if (!g.tri_mask && (g.k_padded > 96 || gridDim.y <= (g.k_padded > 64 ? 8 : 3))) {
         uint32_t const across = gridDim.x, down = gridDim.y, pid = tile_m * across + tile_n, part = across * down / 8;
         uint32_t const at = pid < part * 8 ? pid % 8 * part + pid / 8 : pid;
         uint32_t const first = at / (kWideBand * across) * kWideBand, rows = down - first < kWideBand ? down - first : kWideBand, in_band = at % (kWideBand * across);

@@ -157,3 +157,20 @@ def test_f32_distances_of_extreme_vectors(metric):
     # (roundings of a few units of 2^-53: of one for the angular distance, of the result for the other)
     scale = torch.ones_like(expected) if metric == "angular" else expected.abs()
     assert bool(((got - expected).abs()[finite] <= 16 * 2.0**-53 * scale[finite]).all())
+
+
+# Both orders of walking over the tiles of a product, on both sides of where the depth and the rows of tiles switch between them (64 and
+# 96 values; three and eight rows of tiles of 64), a last band of one row of tiles and of all sixteen: the rows of a product are those of
+# the products of 64 of them, which are one row of tiles.
+@pytest.mark.parametrize("depth", [64, 65, 96, 97])
+def test_f32_walks(depth):
+    rng = np.random.default_rng(98)
+    a = torch.from_numpy(rng.standard_normal((2112, depth)).astype(np.float32)).to(DEV)
+    packed = nk.dots_pack(torch.from_numpy(rng.standard_normal((5003, depth)).astype(np.float32)).to(DEV), "f32")
+    for call in CALLS:
+        single = torch.cat([call(a[first:first + 64], packed) for first in range(0, 2112, 64)])
+        for rows in (65, 192, 193, 512, 513, 1024, 1025, 2048, 2112):
+            out = torch.full((rows + 1, 5003), -7.0, dtype=torch.float64, device=DEV)
+            call(a[:rows], packed, out=out[:rows])
+            assert same(out[:rows], single[:rows]), f"{call.__name__} {rows} rows"
+            assert bool((out[rows] == -7.0).all())
