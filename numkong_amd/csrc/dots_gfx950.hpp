@@ -2999,11 +2999,17 @@ resident_kernel_t resident_kernel(GemmArgs const &g, int tm) {
     }
 }
 /** Rows are shared out evenly over as few workgroups as hold them, and the columns are cut into strips so that whole rounds of
- *  workgroups (one per compute unit) walk the fewest tiles, four to each strip for its start: as strip_plan. */
+ *  workgroups (one per compute unit) walk the fewest tiles, four to each strip for its start: as strip_plan.
+ *
+ *  `in_step`: where rows of C are a multiple of 4 KiB apart and strips too (32 tiles of 32 columns), all workgroups, which go at about the same
+ *  pace, write to addresses that agree in their lower twelve bits all the time, and those share few of the memory's channels (i8 4982 x
+ *  12,288 x 256 72.5 us, 50.7 through tiles). Up to 24 workgroups of rows a strip has one tile more then: 0.94 of the time in the mean
+ *  of 1160 such shapes; with more of them the rows are too many for that to help (0.98 to 1.02). */
 struct ResidentPlan {
     uint32_t blocks, waves, strips, strip_tiles;
+    bool in_step;
 };
-inline ResidentPlan resident_plan(uint32_t m, uint32_t n_tiles, uint32_t bm) {
+inline ResidentPlan resident_plan(uint32_t m, uint32_t n_tiles, uint32_t bm, uint64_t c_stride) {
     uint64_t const resident = compute_unit_count() > 0 ? compute_unit_count() : 256, rows = kResidentWaves * (uint64_t)bm;
     uint64_t const least = (m + rows - 1) / rows, waves = ((m + least - 1) / least + bm - 1) / bm, blocks = (m + waves * bm - 1) / (waves * bm);
     uint64_t best = ~0ull, length = n_tiles, strips = 1;
@@ -3015,14 +3021,16 @@ inline ResidentPlan resident_plan(uint32_t m, uint32_t n_tiles, uint32_t bm) {
         if (here == 1) break;
         ++strips;
     }
-    return {(uint32_t)blocks, (uint32_t)waves, (uint32_t)((n_tiles + length - 1) / length), (uint32_t)length};
+    bool const in_step = c_stride % 4096 == 0 && length % 32 == 0;
+    if (in_step && blocks <= 24 && length < n_tiles) ++length;
+    return {(uint32_t)blocks, (uint32_t)waves, (uint32_t)((n_tiles + length - 1) / length), (uint32_t)length, in_step};
 }
 /** `planned`: nothing is launched. */
 template <class T>
 hipError_t launch_resident(GemmArgs &g, hipStream_t stream, int tm, PlannedTile *planned) {
     resident_kernel_t const kernel = resident_kernel<T>(g, tm);
     if (!kernel) return hipErrorInvalidValue;
-    ResidentPlan const plan = resident_plan(g.m, g.n_tiles, 32 * tm);
+    ResidentPlan const plan = resident_plan(g.m, g.n_tiles, 32 * tm, g.c_stride);
     uint64_t const units = (uint64_t)plan.blocks * plan.strips;
     if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
     if (planned) {
@@ -3322,14 +3330,18 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // of the dots and the euclidean are slower by more than 3 per cent. At 4400 more, where the lines lie: C under 64 MiB 0.98 to 1.05, strips of fewer than 12 tiles 0.98
     // to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16 69 x 2,664,123 x 602 1.55, u4
     // 318 x 137,089 x 1072 1.29; of workgroups with six and more of them 1 in 20 is slower).
+    // Left out: short dots whose strips write in step (see ResidentPlan) with more than eight workgroups of rows, 1.09 to 1.18 of the time
+    // (i8 31,126 x 2048 x 256 77 us, 52 through tiles).
     // Two blocks of rows where the image does not stay in the last-level cache and reading it half as often counts (i8 1024 x 1,048,576 x
     // 768 1195 us and 1080; 4096 x 65,536 x 500, whose image does, 256 and 266).
     auto resident_blocks = [&](GemmArgs const &args) -> int {
         if (triangle || args.m <= 64 || (uint64_t)args.m * args.n * 4 < (64ull << 20) || !resident_kernel<T>(args, 1)) return 0;
-        ResidentPlan const plan = resident_plan(args.m, args.n_tiles, 32);
+        ResidentPlan const plan = resident_plan(args.m, args.n_tiles, 32, args.c_stride);
         if (plan.strip_tiles < 16 || (args.metric == 1 && plan.waves < 6)) return 0;
         uint64_t const image = (uint64_t)args.n_tiles * args.k_chunks * kTileChunkBytes;
-        return args.m > 256 && image >= (128ull << 20) && resident_kernel<T>(args, 2) ? 2 : 1;
+        bool const two = args.m > 256 && image >= (128ull << 20) && resident_kernel<T>(args, 2);
+        if (args.metric == 0 && args.k_chunks <= 4 * kStageChunks && plan.in_step && plan.blocks > 8 && !two) return 0;
+        return two ? 2 : 1;
     };
     if (config == 8 || config == 9) {
         if (!triangle && resident_kernel<T>(g, config - 7)) return launch_resident<T>(g, stream, config - 7, planned);
