@@ -3325,22 +3325,29 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         return best;
     };
     // A in registers (see dots_resident_kernel) wherever there is such a kernel, C is most of the traffic and a strip is long enough for
-    // what its start costs. Against the choice without it, rounds of three sets of operands and results: at 2800 random shapes of all types
-    // that it takes, 65 to 300,000 rows, the time is 0.81 of that before in the mean (dots 0.81, euclidean 0.81, angular 0.80), and 2 in 100
-    // of the dots and the euclidean are slower by more than 3 per cent. At 4400 more, where the lines lie: C under 64 MiB 0.98 to 1.05, strips of fewer than 12 tiles 0.98
-    // to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16 69 x 2,664,123 x 602 1.55, u4
-    // 318 x 137,089 x 1072 1.29; of workgroups with six and more of them 1 in 20 is slower).
+    // what its start costs. Against the choice without it, rounds of three sets of operands and results, at 13,700 random shapes of all types
+    // that it takes, 65 to 300,000 rows, C of 64 MiB to 2.4 GiB, the time is in the mean 0.81 (dots), 0.80 (euclidean) and 0.80 (angular), and more by 3 per
+    // cent at 24, 22 and 47 in 1000. Half of the slower angular ones are floats of 4 and 6 stages on lines with images of 64 MiB and more
+    // and 257 to 2048 rows, whose mean is 1.0 one way and 0.9 another time. At 4400 more shapes, where the lines lie: C under 64 MiB 0.98 to 1.05, strips
+    // of fewer than 12 tiles 0.98 to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16
+    // 69 x 2,664,123 x 602 1.55, u4 318 x 137,089 x 1072 1.29).
+    // Two blocks of rows, which ask half as often for the image, where that does not stay in the last-level cache beside C, and of more
+    // rows the deeper the product (7400 shapes, each both ways): of 2 stages 1.03 of the time with one up to 8 MiB of image, 1.02 to 32, 1.01 to 64, then 0.93,
+    // 0.87 from 80 to 256 MiB; of 4 stages 1.02 to 64 MiB, then 0.91, 0.88 to 112; of 6 stages 1.05 to 64 MiB, 1.02 to 80, then 0.90. From there on
+    // by workgroups of 256 rows: two 0.90 (2 stages), 1.01 (4) and 1.05 (6), three 0.87, 0.94 and 1.01, four 0.85, 0.86 and 0.99, five 0.88, 0.80 and 0.91. (i8
+    // 1024 x 1,048,576 x 768 1195 us and 1080.)
     // Left out: short dots whose strips write in step (see ResidentPlan) with more than eight workgroups of rows, 1.09 to 1.18 of the time
-    // (i8 31,126 x 2048 x 256 77 us, 52 through tiles).
-    // Two blocks of rows where the image does not stay in the last-level cache and reading it half as often counts (i8 1024 x 1,048,576 x
-    // 768 1195 us and 1080; 4096 x 65,536 x 500, whose image does, 256 and 266).
+    // (i8 31,126 x 2048 x 256 77 us, 52 through tiles), and floats of 8 stages off the lines with up to 128 rows, 1.04 (190 shapes).
     auto resident_blocks = [&](GemmArgs const &args) -> int {
         if (triangle || args.m <= 64 || (uint64_t)args.m * args.n * 4 < (64ull << 20) || !resident_kernel<T>(args, 1)) return 0;
         ResidentPlan const plan = resident_plan(args.m, args.n_tiles, 32, args.c_stride);
+        uint32_t const stages = args.k_chunks / kStageChunks;
+        bool const lines = (((uintptr_t)args.c | args.c_stride) & 127) == 0;
+        uint64_t const image_mib = ((uint64_t)args.n_tiles * args.k_chunks * kTileChunkBytes) >> 20;
         if (plan.strip_tiles < 16 || (args.metric == 1 && plan.waves < 6)) return 0;
-        uint64_t const image = (uint64_t)args.n_tiles * args.k_chunks * kTileChunkBytes;
-        bool const two = args.m > 256 && image >= (128ull << 20) && resident_kernel<T>(args, 2);
-        if (args.metric == 0 && args.k_chunks <= 4 * kStageChunks && plan.in_step && plan.blocks > 8 && !two) return 0;
+        bool const two = image_mib >= (stages <= 4 ? 64 : 80) && args.m > (stages <= 2 ? 256 : stages <= 4 ? 512 : 768) && resident_kernel<T>(args, 2);
+        if (args.metric == 0 && stages <= 4 && plan.in_step && plan.blocks > 8 && !two) return 0;
+        if (args.metric == 0 && T::kChunked && stages == 8 && args.m <= 128 && !lines) return 0;
         return two ? 2 : 1;
     };
     if (config == 8 || config == 9) {

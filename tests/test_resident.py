@@ -160,6 +160,20 @@ def test_registers_hold_a(tmp_path):
     assert kernels > 150 and not spilled
 
 
+# Both sides of the lines of the rule: rows, bytes of C, tiles of a strip, wavefronts with rows (angular), floats of eight stages off the lines
+# with few rows, two blocks of rows by image and rows.
+@pytest.mark.parametrize("dtype, metric, m, n, k, rows", [
+    ("i8", "dots", 64, 1_048_576, 512, 0), ("i8", "dots", 65, 1_048_576, 512, 32), ("i8", "dots", 128, 131_040, 512, 0), ("i8", "dots", 128, 131_072, 512, 32),
+    ("i8", "dots", 255, 122_880, 512, 0), ("i8", "dots", 255, 122_912, 512, 32), ("i8", "angular", 160, 500_000, 768, 0), ("i8", "angular", 161, 500_000, 768, 32),
+    ("f16", "dots", 128, 500_000, 500, 32), ("f16", "dots", 129, 500_001, 500, 32), ("f16", "dots", 128, 500_001, 500, 0), ("f16", "dots", 128, 500_001, 600, 32), ("i8", "dots", 128, 500_001, 1000, 32),
+    ("i8", "dots", 1000, 300_001, 700, 32),
+    ("i8", "dots", 512, 262_112, 256, 32), ("i8", "dots", 512, 262_144, 256, 64), ("i8", "dots", 256, 500_000, 256, 32), ("i8", "dots", 257, 500_000, 256, 64),
+    ("bf16", "dots", 512, 500_000, 256, 32), ("bf16", "dots", 513, 500_000, 256, 64), ("u8", "dots", 768, 500_000, 768, 32), ("u8", "dots", 769, 500_000, 768, 64),
+    ("u8", "dots", 1024, 109_216, 768, 32), ("u8", "dots", 1024, 109_248, 768, 64), ("u8", "dots", 1024, 500_001, 768, 32), ("f16", "dots", 1024, 500_000, 350, 32)])
+def test_where_a_is_kept(dtype, metric, m, n, k, rows):
+    assert resident_of(dtype, metric, m, n, k)[0] == rows
+
+
 # Rows of C a multiple of 4 KiB apart: strips of 33 tiles in the place of 32, or the tiles where too many rows share them.
 @pytest.mark.parametrize("dtype, metric, m, n, k, tiles", [
     ("i8", "dots", 2048, 32_768, 512, 33), ("i8", "dots", 2048, 32_736, 512, 32), ("i8", "euclidean", 4982, 12_288, 256, 33), ("i8", "dots", 4982, 12_288, 768, 33),
