@@ -1645,12 +1645,17 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         fetch_a(view, s, ring_tag, slot_c<0>()), fetch_a(view, s, ring_tag, slot_c<1>());
         fetch_a(view, s, ring_tag, slot_c<2>()), fetch_a(view, s, ring_tag, slot_c<3>());
     };
-    // Every wavefront waits for its own fetches into a stage (the compiler puts that wait in front of any read of the
-    // stage's array: one word is read for the purpose), then all meet: after that the stage is whole for everybody.
+    // Every wavefront waits for its own fetches into a stage, then all meet: after that the stage is whole for everybody. `younger`:
+    // the fetches and loads that a wavefront has issued behind those, at the least (stores of a tile come on top); memory answers in
+    // order. The compiler puts the same wait in front of the word read below, of its own accord, but it has once left such waits out, and
+    // then results were wrong now and then: written here, the wait does not depend on it.
     // No fence: a fence would wait for the fetches of the later stages as well. The waits for the fragment reads
     // that are still in flight come with the word read (LDS answers in order).
-    auto stage_arrived = [&](auto ring_tag) __attribute__((always_inline)) {
+    auto stage_arrived = [&](auto ring_tag, auto younger_tag) __attribute__((always_inline)) {
+        constexpr int younger = decltype(younger_tag)::value;
+        static_assert(younger < 64, "what a wait can count to");
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (younger & 15) | (younger >> 4) << 14);
         typedef __attribute__((address_space(3))) uint32_t const lds_u32_t;
         uint32_t const word = *(lds_u32_t *)(ring_of(ring_tag) + lane * 4);
         asm volatile("" ::"v"(word) : "memory");
@@ -1705,7 +1710,8 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         multiply(slot_c<P>(), slot_c<2>());
         load_b(b2, s2, slot_c<P>(), slot_c<2>()), fetch_a(a3, s3, slot_c<R + 3>(), slot_c<2>());
         schedule_direct_k_step();
-        stage_arrived(slot_c<R + 1>());
+        // (behind the fetches of stage s + 1: B and A of the stage before this one, and three quarters of both of this one)
+        stage_arrived(slot_c<R + 1>(), slot_c<7 * TN + kLoads + kLoads * 3 / 4>());
         read_frags(slot_c<R + 1>(), slot_c<0>(), slot_c<0>());
         multiply(slot_c<P>(), slot_c<3>());
         load_b(b2, s2, slot_c<P>(), slot_c<3>()), fetch_a(a3, s3, slot_c<R + 3>(), slot_c<3>());
@@ -1720,7 +1726,7 @@ __global__ __launch_bounds__(256, (TM * TN == 1 ? 4 : TM * TN <= 2 ? 3 : (TM * T
         load_b(cur, 1, slot_c<1>(), slot_c<0>()), load_b(cur, 1, slot_c<1>(), slot_c<1>());
         load_b(cur, 1, slot_c<1>(), slot_c<2>()), load_b(cur, 1, slot_c<1>(), slot_c<3>());
         fetch_a_all(cur, 2, slot_c<2>());
-        stage_arrived(slot_c<0>());
+        stage_arrived(slot_c<0>(), slot_c<8 * TN + 2 * kLoads>());
         read_frags(slot_c<0>(), slot_c<0>(), slot_c<0>());
     };
 
