@@ -171,6 +171,10 @@ int nk_hip_planned_tile(int dtype, int metric, size_t m, size_t n, size_t k, voi
 int nk_hip_planned_resident(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
                             uint32_t planned[3]);
 
+/** TEST HOOK, as the two above: planned[0] is 1 where the tile's A goes straight into LDS, not through registers. */
+int nk_hip_planned_direct(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                          uint32_t planned[1]);
+
 /** Thread-local text of the last failure in this layer ("" if none). */
 char const *nk_hip_last_error(void);
 

@@ -123,6 +123,8 @@ def library() -> ctypes.CDLL:
     lib.nk_hip_planned_tile.restype = i32
     lib.nk_hip_planned_resident.argtypes = lib.nk_hip_planned_tile.argtypes
     lib.nk_hip_planned_resident.restype = i32
+    lib.nk_hip_planned_direct.argtypes = lib.nk_hip_planned_tile.argtypes
+    lib.nk_hip_planned_direct.restype = i32
     lib.nk_hip_device_count.restype = i32
     lib.nk_capabilities.restype = ctypes.c_uint64
     lib.nk_configure_thread.argtypes = [ctypes.c_uint64]

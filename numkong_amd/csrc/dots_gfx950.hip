@@ -750,6 +750,13 @@ int nk_hip_planned_resident(int dtype, int metric, size_t m, size_t n, size_t k,
     return status;
 }
 
+int nk_hip_planned_direct(int dtype, int metric, size_t m, size_t n, size_t k, void const *a, size_t a_stride, void *c, size_t c_stride,
+                          uint32_t planned[1]) {
+    int const status = plan_only(dtype, metric, m, n, k, a, a_stride, c, c_stride);
+    planned[0] = t_planned.direct;
+    return status;
+}
+
 char const *nk_hip_last_error(void) { return g_last_error; }
 
 } // extern "C"

@@ -149,6 +149,7 @@ int forced_tile_config();
 struct PlannedTile {
     uint32_t shape, store_policy, units, strip_tiles;
     uint32_t resident_rows, resident_units, resident_tiles; // A in registers instead (nk_hip_planned_resident; rows 0: not)
+    uint32_t direct;                                        // A straight into LDS (nk_hip_planned_direct)
 };
 PlannedTile *planned_tile();
 /** Compute units of the current device, asked once per process. */
@@ -2784,6 +2785,27 @@ inline bool needs_shift(GemmArgs const &g) {
     return g.avec < (T::kSrcChunk < 4 ? T::kSrcChunk : 4) && g.k_chunks / kStageChunks >= 4;
 }
 
+/** A straight into LDS (see the kernel): the largest tile of the types that reach LDS as they are, depths of whole
+ *  trips of four stages, and for the two-accumulator types folds that fall between trips (measured at 8192^3,
+ *  alternating in one session: i8 0.438 -> 0.419 ms, bf16 0.930 -> 0.902, f16 0.997 -> 0.968; with a fold after every
+ *  second stage of the trip instead, the compiler ran out of registers in the folds and bf16 took 1.10 ms). Of 128 x 128 the
+ *  integers, from 24 stages and more than two rows of tiles on (486 shapes of i8, 0.965 of the time in the mean; going round twelve sets of
+ *  operands 2048 x 2048 x 4096 37.0 and 35.9 us, x 3072 33.1 and 32.7, but x 2560 31.0 and 31.0 and x 2048 28.7 and 29.1). */
+template <class T, int TM, int TN>
+constexpr bool direct_built() {
+    return kDirectStaging && !T::kUnsigned && !T::kPrewiden && T::kSrcChunk == 16 && T::kImageChunk == 16 &&
+           ((TM == 8 && TN == 2) || (TM == 4 && TN == 1 && !T::kChunked) || (TM == 4 && TN == 2 && T::kChunked));
+}
+template <class T, int TM, int TN>
+bool goes_direct(GemmArgs const &g) {
+    if constexpr (!direct_built<T, TM, TN>()) return false;
+    uint32_t const stages = g.k_chunks / kStageChunks;
+    bool const whole = g.k_src_bytes % (2 * kStageChunks * T::kSrcChunk) == 0;
+    return !needs_shift<T>(g) && g.metric == 0 && stages % 4 == 0 && stages >= 8 && (whole || !tail_matters_for<T, false>()) &&
+           (!T::kChunked || g.chunk_stages % 4 == 0) && (TN == 2 || (stages >= 24 && g.m > 256)) && g.avec >= 16 &&
+           !(forced_tile_config() & 0x40000000);
+}
+
 /** `slots_only`: do not launch, only report how many workgroups of the kernel this call would use are resident on
  *  the device at once. */
 template <class T, int TM, int TN>
@@ -2825,18 +2847,9 @@ hipError_t launch_one(GemmArgs &g, hipStream_t stream, TriangleScratch const *tr
     if constexpr (tail_matters_for<T, false>()) {
         if (whole) kernel = dots_packed_kernel<T, TM, TN, true, false, true>;
     }
-    // A straight into LDS (see the kernel): the largest tile of the types that reach LDS as they are, depths of whole
-    // trips of four stages, and for the two-accumulator types folds that fall between trips (measured at 8192^3,
-    // alternating in one session: i8 0.438 -> 0.419 ms, bf16 0.930 -> 0.902, f16 0.997 -> 0.968; with a fold after every
-    // second stage of the trip instead, the compiler ran out of registers in the folds and bf16 took 1.10 ms). Of 128 x 128 the
-    // integers, from 24 stages and more than two rows of tiles on (486 shapes of i8, 0.965 of the time in the mean; going round twelve sets of
-    // operands 2048 x 2048 x 4096 37.0 and 35.9 us, x 3072 33.1 and 32.7, but x 2560 31.0 and 31.0 and x 2048 28.7 and 29.1).
     bool direct = false;
-    if constexpr (kDirectStaging && !T::kUnsigned && !T::kPrewiden && T::kSrcChunk == 16 && T::kImageChunk == 16 &&
-                  ((TM == 8 && TN == 2) || (TM == 4 && TN == 1 && !T::kChunked) || (TM == 4 && TN == 2 && T::kChunked))) {
-        direct = across && !norms && stages % 4 == 0 && stages >= 8 && (whole || !tail_matters_for<T, false>()) &&
-                 (!T::kChunked || g.chunk_stages % 4 == 0) &&
-                 (TN == 2 || (stages >= 24 && g.m > 256)) && (g.avec >= 16) && !(forced_tile_config() & 0x40000000);
+    if constexpr (direct_built<T, TM, TN>()) {
+        direct = goes_direct<T, TM, TN>(g);
         if (direct) kernel = dots_packed_kernel<T, TM, TN, true, false, tail_matters_for<T, false>(), true>;
     }
     if constexpr (T::kDistances) {
@@ -3431,6 +3444,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     }
     if (planned) {
         planned->shape = (uint32_t)config, planned->store_policy = g.store_policy, planned->units = (uint32_t)tiles_of(g, config);
+        planned->direct = config == 1 ? goes_direct<T, 8, 2>(g) : config == 2 ? goes_direct<T, 4, 2>(g) : config == 3 && goes_direct<T, 4, 1>(g);
         return hipSuccess;
     }
     return launch_config<T>(g, stream, triangle, config);

@@ -30,3 +30,20 @@ def _again(m, k):
     rng = np.random.default_rng(95)
     values_of("i8", m, (k + 15) // 16 * 16, rng)
     return rng
+
+
+# Windows of all pairs whose first row is not one of the image's tiles take A from the vectors: the same tile, along a triangle's list.
+@pytest.mark.parametrize("start, count, k", [(33, 1000, 3072), (1, 700, 3584), (95, 1300, 4096)])
+def test_windows_of_all_pairs(start, count, k):
+    rng = np.random.default_rng(99)
+    vectors = values_of("i8", count, k, rng).to(DEV)
+
+    def window(config):
+        out = torch.full((count, count), 77, dtype=torch.int32, device=DEV)
+        return through(config, lambda: nk.dots_symmetric(vectors, "i8", out=out, start_row=start, end_row=count))
+
+    straight = window(3)
+    assert torch.equal(straight, window(3 | 1 << 30))
+    expected = (vectors.cpu().double() @ vectors.cpu().double().T).to(torch.int32)  # (exact: whole numbers below 2^53)
+    row, column = torch.arange(count)[:, None], torch.arange(count)[None, :]
+    assert torch.equal(straight.cpu(), torch.where((row >= start) & (column >= row), expected, 77))

@@ -1,10 +1,13 @@
 """What a call runs as, asked of the library's own choice without a GPU (nk_hip_planned_tile)."""
+import ctypes
 import random
 import time
 
+import numpy as np
 import pytest
 
-from tests.support import STRIPS, route_of
+import numkong_amd as nk
+from tests.support import CODES, DIMENSIONS_PER_VALUE, METRICS, STORAGE, STRIPS, route_of
 
 COMPUTE_UNITS = 256  # what the library takes where it cannot ask a device
 
@@ -108,3 +111,24 @@ def test_tiles_into_large_results_on_lines(dtype, m, n, k, shape):
                                                            ("u4", "euclidean", 4000, 40_001, 6400, 3)])
 def test_depth_of_the_middling_tile(dtype, metric, m, n, k, shape):
     assert route_of(dtype, metric, m, n, k).shape == shape
+
+
+def _planned(hook, dtype, metric, m, n, k, config=0):
+    planned = (ctypes.c_uint32 * 4)()
+    nk.library().nk_hip_set_tile_config(config)
+    try:
+        row = -(-k // DIMENSIONS_PER_VALUE.get(dtype, 1)) * np.dtype(STORAGE[dtype]).itemsize
+        assert getattr(nk.library(), hook)(CODES[dtype], {"dots": 0, **METRICS}[metric], m, n, k, 1 << 30, row, 1 << 40, 4 * n, planned) == 0
+    finally:
+        nk.library().nk_hip_set_tile_config(0)
+    return planned[0]
+
+
+# A straight into the LDS of 128 x 128 tiles, on both sides of 257 rows and of 24 stages (of 128 values); not where bit 30 forbids it, nor
+# for rows off 16 bytes, u8 (whose bytes are summed on the way), distances.
+@pytest.mark.parametrize("dtype, metric, m, k, config, straight", [
+    ("i8", "dots", 257, 3072, 3, 1), ("i8", "dots", 256, 3072, 3, 0), ("i8", "dots", 257, 2560, 3, 0), ("i8", "dots", 257, 3200, 3, 0), ("i8", "dots", 257, 3584, 3, 1),
+    ("i8", "dots", 4097, 3072, 3 | 1 << 30, 0), ("i8", "dots", 4097, 3500, 3, 0), ("u8", "dots", 4097, 3072, 3, 0), ("i8", "angular", 4097, 3072, 3, 0),
+    ("i8", "dots", 2048, 4096, 0, 1), ("i8", "dots", 2048, 2048, 0, 0), ("i8", "dots", 8192, 8192, 0, 1), ("bf16", "dots", 8192, 8192, 0, 1)])
+def test_straight_into_lds(dtype, metric, m, k, config, straight):
+    assert _planned("nk_hip_planned_direct", dtype, metric, m, max(m, 2048), k, config) == straight
