@@ -11,7 +11,7 @@ import torch
 import numkong_amd as nk
 from tests.support import CODES, DIMENSIONS_PER_VALUE, METRICS, STORAGE
 from tests.test_strips_gpu import STAGE, framed, through, untouched
-from tests.test_unaligned_gpu import CALLS, DEV, same, values_of
+from tests.test_unaligned_gpu import CALLS, DEV, aligned, placed, same, values_of
 
 TYPES = ["i8", "u8", "bf16", "f16", "e4m3", "e5m2", "e2m3", "e3m2", "i4", "u4"]
 FLOATS = ["bf16", "f16", "e4m3", "e5m2", "e3m2"]
@@ -158,6 +158,49 @@ def test_registers_hold_a(tmp_path):
                 if int(line.split()[-1]) > 1:
                     spilled[name] = int(line.split()[-1])
     assert kernels > 150 and not spilled
+
+
+# The deeper kernels on lines, whose rings of LDS differ (four tiles at eight stages, three at ten and twelve): more rows than a workgroup
+# has, several strips, each longer than the ring, a strip that ends nine columns into a tile; depths whole, short by one, by eight values
+# and by more than a stage.
+@pytest.mark.gpu
+@pytest.mark.parametrize("stages", [8, 10, 12])
+@pytest.mark.parametrize("dtype", TYPES)
+def test_deeper_on_lines(dtype, stages):
+    rng = np.random.default_rng(96)
+    m, ran = 777, 0
+    for n, after, short in ((20_000, 0, 0), (19_977, 23, 1), (20_000, 32, 8), (19_977, 23, STAGE.get(dtype, 128) + 3)):
+        columns = stages * STAGE.get(dtype, 128) - short
+        a = values_of(dtype, m, columns, rng).to(DEV)
+        packed = nk.dots_pack(values_of(dtype, 4099, columns, rng).to(DEV).repeat(5, 1)[:n].contiguous(), dtype)
+        for metric in CALLS:
+            if not built(dtype, metric, stages, 1, True):
+                continue
+            rows, units, tiles = resident_of(dtype, metric, m, n, columns * DIMENSIONS_PER_VALUE.get(dtype, 1), 8, 4 * (n + after))
+            assert rows == 32 and units >= 40 and tiles > 4, f"{units} pieces of {tiles} tiles"
+            expected = through(4, lambda: CALLS[metric](a, packed))
+            whole, window = framed(m, n, 0, after, expected.dtype)
+            through(8, lambda: CALLS[metric](a, packed, out=window))
+            assert same(window.contiguous(), expected), f"{dtype} {metric} {m} x {n} x {columns}"
+            assert untouched(whole, m, n, 0), f"{dtype} {metric} {m} x {n} x {columns}: written outside C"
+            ran += 1
+    assert ran >= 4 or (dtype in FLOATS and stages == 12)
+
+
+# NaN around the rows of A for the types whose chunks are 8 bytes as well, rows that start on odd addresses, an image of which almost two
+# stages are empty: seven hold values, the seventh a single one.
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "e4m3", "e5m2"])
+@pytest.mark.parametrize("metric", list(CALLS))
+@pytest.mark.parametrize("n", [1024, 1111])
+def test_nan_around_the_rows_of_a(dtype, metric, n):
+    rng = np.random.default_rng(97)
+    a, b = values_of(dtype, 300, 385, rng), values_of(dtype, n, 385, rng)
+    packed = nk.dots_pack(aligned(b), dtype)
+    expected = through(4, lambda: CALLS[metric](aligned(a), packed))
+    assert resident_of(dtype, metric, 300, n, 385, 8)[0] == 32
+    for pad, offset in ((131, 0), (130, 1), (128, 3), (64, 1)):
+        assert same(through(8, lambda: CALLS[metric](placed(a, pad, offset), packed)), expected), f"{pad} values behind, {offset} in front"
 
 
 # Both sides of the lines of the rule: rows, bytes of C, tiles of a strip, wavefronts with rows (angular), floats of eight stages off the lines
