@@ -2413,7 +2413,7 @@ __global__ __launch_bounds__(64 * kStripWaves, 2) void dots_strips_kernel(GemmAr
  *  multiplies it with its own rows and stores 128 bytes of each. One barrier per tile, and nothing is staged.
  *
  *  Why: such products are bound by the memory, and what keeps a copy's rate from them is the reading. Writes of C in any of the shapes
- *  below reach 5.2 TB/s, and reads of as many bytes as B has beside them take their own time more (1024 x 1,048,576 results and 768 bytes a
+ *  below reach 4.9 TB/s, and reads of as many bytes as B has beside them take their own time more (1024 x 1,048,576 results and 768 bytes a
  *  column, no arithmetic: 872 us written, 130 read, 1030 to 1040 both, as long as every byte is asked for once), but with every line of B
  *  asked for by eight workgroups at about the same time, as tiles of 128 rows do, both take 1280, however far ahead they ask: what a
  *  compute unit reads waits in one queue with what it writes. Here B is read once per 256 rows (TM 1) or 512.
@@ -3022,8 +3022,9 @@ resident_kernel_t resident_kernel(GemmArgs const &g, int tm) {
  *
  *  `in_step`: where rows of C are a multiple of 4 KiB apart and strips too (32 tiles of 32 columns), all workgroups, which go at about the same
  *  pace, write to addresses that agree in their lower twelve bits all the time, and those share few of the memory's channels (i8 4982 x
- *  12,288 x 256 72.5 us, 50.7 through tiles). Up to 24 workgroups of rows a strip has one tile more then: 0.94 of the time in the mean
- *  of 1160 such shapes; with more of them the rows are too many for that to help (0.98 to 1.02). */
+ *  12,288 x 256 72.5 us, 50.7 through tiles). Up to 24 workgroups of rows a strip of 32 to 128 tiles has one more then: the time of 32 is 0.93
+ *  in the mean of 770 dots, 0.94 of 414 euclidean and 0.98 of 274 angular, of 128 0.95, 0.94 and 0.97. With more rows that does not help (0.98
+ *  to 1.02), nor do longer strips gain (0.97 to 1.0, 1.0 and 1.0 to 1.02; 1024 x 1,048,576 x 768 1082 us and 1086). */
 struct ResidentPlan {
     uint32_t blocks, waves, strips, strip_tiles;
     bool in_step;
@@ -3041,7 +3042,7 @@ inline ResidentPlan resident_plan(uint32_t m, uint32_t n_tiles, uint32_t bm, uin
         ++strips;
     }
     bool const in_step = c_stride % 4096 == 0 && length % 32 == 0;
-    if (in_step && blocks <= 24 && length < n_tiles) ++length;
+    if (in_step && blocks <= 24 && length <= 128 && length < n_tiles) ++length;
     return {(uint32_t)blocks, (uint32_t)waves, (uint32_t)((n_tiles + length - 1) / length), (uint32_t)length, in_step};
 }
 /** `planned`: nothing is launched. */
@@ -3103,7 +3104,9 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     auto past = [](int config) { return Choice(config, 1); };
     // Strips (see dots_strips_kernel) where C is large against the operands. What they save is the partial lines of rows off the lines
     // and the staging of A with every tile; what they cost is the start and the end of every strip, with nothing beside it on the
-    // compute unit, and the columns of a row's last tile. So a row of C has to be more than eight tiles of 256 columns and a strip at
+    // compute unit, and the columns of a row's last tile. (Calls that keep A in registers, resident_blocks, do not ask here. Of dots on lines that
+    // leaves u1, short ones whose strips would write in step, and rows of A 16 MiB apart; times of other dots on lines in this comment and the next are of what they
+    // would take without it, and the choice is that too.) So a row of C has to be more than eight tiles of 256 columns and a strip at
     // least four, or three where what the tiles do besides their columns is more (distances; e2m3, which widens: 2038 x 10,937 x 77 43 us
     // and 113, u4 angular 436 x 39,391 x 122 55 and 90; of 240 such shapes two in a hundred were slower): with fewer they took up to twice as long as the tiles below, now and before (us): i8 1,000,000 x 130 x 768 638
     // and 447, angular 817 and 482; bf16 200,000 x 129 x 768 227 and 152; u8 714 x 25,854 x 198 (three to a strip) 31 and 26. On
@@ -3148,7 +3151,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // now): u8 euclidean 1000 x 500,009 x 301 1165 and 610 (strips), i8 1024 x 204,801 x 220 298 and 151 (strips), f16 8192 x 8191 x
     // 1000 289 and 230 (strips); with rows on
     // lines bf16 208 x 60,160 x 485 71 and 43 (64 x 128), e5m2 150 x 136,704 x 320 84 and 63 (64 x 128), i8 angular 371 x
-    // 34,739 x 1600 154 and 58 (64 x 128), bf16 527 x 400,384 x 192 384 and 259 (strips), bf16 3439 x 38,656 x 826 382 and 316
+    // 34,739 x 1600 154 and 58 (64 x 128), bf16 527 x 400,384 x 192 384 and 259 (strips; 228 with A in registers), bf16 3439 x 38,656 x 826 382 and 316
     // (128 x 128: two workgroups of it fit a compute unit, and the kernels for depths of no whole stage spill at 128 x 256).
     // 0: nothing here applies.
     auto by_bytes_of_c = [&](GemmArgs const &args) -> int {
@@ -3192,7 +3195,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
             if (mib < 96) return stages > 2 && (stages <= 16 || (stages < 32 && !whole)) ? 4 : 0;
             if (stages <= 2) return 0;
             if (stages <= 4 && mib < 256) return 4;
-            return stages <= 16 || (stages < 32 && !whole) ? 3 : 0; // (f16 4542 x 16,384 x 324 113 us, 167 through the largest tile)
+            return stages <= 16 || (stages < 32 && !whole) ? 3 : 0; // (f16 4542 x 16,384 x 324, which keeps A in registers now, 113 us, 167 through the largest tile)
         }
         if (!norms) {
             if (stages > 16) return 0;
@@ -3344,10 +3347,10 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         return best;
     };
     // A in registers (see dots_resident_kernel) wherever there is such a kernel, C is most of the traffic and a strip is long enough for
-    // what its start costs. Against the choice without it, rounds of three sets of operands and results, at 13,700 random shapes of all types
-    // that it takes, 65 to 300,000 rows, C of 64 MiB to 2.4 GiB, the time is in the mean 0.81 (dots), 0.80 (euclidean) and 0.80 (angular), and more by 3 per
-    // cent at 24, 22 and 47 in 1000. Half of the slower angular ones are floats of 4 and 6 stages on lines with images of 64 MiB and more
-    // and 257 to 2048 rows, whose mean is 1.0 one way and 0.9 another time. At 4400 more shapes, where the lines lie: C under 64 MiB 0.98 to 1.05, strips
+    // what its start costs. Against the choice without it, rounds of three sets of operands and results, at 13,000 random shapes of all types
+    // that it takes, 65 to 300,000 rows, C of 64 MiB to 2.4 GiB, the time is in the mean 0.80 (dots), 0.80 (euclidean) and 0.79 (angular), and more by 3 per
+    // cent at 26, 29 and 36 in 1000, by 10 per cent at 6. Of the slower angular ones a quarter are floats of 4 and 6 stages on lines with images of 64 MiB
+    // and more and 257 to 2048 rows (0.93 in the mean of 96). At 4400 more shapes, where the lines lie: C under 64 MiB 0.98 to 1.05, strips
     // of fewer than 12 tiles 0.98 to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16
     // 69 x 2,664,123 x 602 1.55, u4 318 x 137,089 x 1072 1.29).
     // Two blocks of rows, which ask half as often for the image, where that does not stay in the last-level cache beside C, and of more
