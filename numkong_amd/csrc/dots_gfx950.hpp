@@ -3358,8 +3358,9 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
     // 0.87 from 80 to 256 MiB; of 4 stages 1.02 to 64 MiB, then 0.91, 0.88 to 112; of 6 stages 1.05 to 64 MiB, 1.02 to 80, then 0.90. From there on
     // by workgroups of 256 rows: two 0.90 (2 stages), 1.01 (4) and 1.05 (6), three 0.87, 0.94 and 1.01, four 0.85, 0.86 and 0.99, five 0.88, 0.80 and 0.91. (i8
     // 1024 x 1,048,576 x 768 1195 us and 1080.)
-    // Left out: short dots whose strips write in step (see ResidentPlan) with more than eight workgroups of rows, 1.09 to 1.18 of the time
-    // (i8 31,126 x 2048 x 256 77 us, 52 through tiles), and floats of 8 stages off the lines with up to 128 rows, 1.04 (190 shapes).
+    // Left out: short dots whose strips write in step (see ResidentPlan) with more than eight workgroups of rows (i8 31,126 x 2048 x 256 77 us, 52
+    // through tiles; without A in registers 0.87 of the time in the mean of 471 calls of two stages, 0.92 of 381 of four, but of e2m3 and
+    // u8, whose tiles widen or sum A, 1.13 and 1.07 at four), and floats of 8 stages off the lines with up to 128 rows (0.97 of 415).
     auto resident_blocks = [&](GemmArgs const &args) -> int {
         if (triangle || args.m <= 64 || (uint64_t)args.m * args.n * 4 < (64ull << 20) || !resident_kernel<T>(args, 1)) return 0;
         ResidentPlan const plan = resident_plan(args.m, args.n_tiles, 32, args.c_stride);
@@ -3368,7 +3369,7 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         uint64_t const image_mib = ((uint64_t)args.n_tiles * args.k_chunks * kTileChunkBytes) >> 20;
         if (plan.strip_tiles < 16 || (args.metric == 1 && plan.waves < 6)) return 0;
         bool const two = image_mib >= (stages <= 4 ? 64 : 80) && args.m > (stages <= 2 ? 256 : stages <= 4 ? 512 : 768) && resident_kernel<T>(args, 2);
-        if (args.metric == 0 && stages <= 4 && plan.in_step && plan.blocks > 8 && !two) return 0;
+        if (args.metric == 0 && stages <= (T::kDtype == kE2M3 || T::kUnsigned ? 2 : 4) && plan.in_step && plan.blocks > 8 && !two) return 0;
         if (args.metric == 0 && T::kChunked && stages == 8 && args.m <= 128 && !lines) return 0;
         return two ? 2 : 1;
     };

@@ -220,7 +220,7 @@ def test_where_a_is_kept(dtype, metric, m, n, k, rows):
 # Rows of C a multiple of 4 KiB apart: strips of 33 tiles in the place of 32, up to 129; tiles where too many rows share them.
 @pytest.mark.parametrize("dtype, metric, m, n, k, tiles", [
     ("i8", "dots", 2048, 32_768, 512, 33), ("i8", "dots", 2048, 32_736, 512, 32), ("i8", "euclidean", 4982, 12_288, 256, 33), ("i8", "dots", 4982, 12_288, 768, 33),
-    ("i8", "dots", 4982, 12_288, 256, 0), ("i8", "dots", 4982, 12_256, 256, 32), ("i8", "euclidean", 8192, 16_384, 256, 64), ("bf16", "dots", 60_000, 1024, 256, 0), ("bf16", "dots", 60_000, 1024, 600, 32),
+    ("i8", "dots", 4982, 12_288, 256, 0), ("i8", "dots", 4982, 12_288, 512, 0), ("e2m3", "dots", 4982, 12_288, 512, 33), ("u8", "dots", 4982, 12_288, 512, 33), ("u8", "dots", 4982, 12_288, 256, 0), ("i8", "dots", 4982, 12_256, 256, 32), ("i8", "euclidean", 8192, 16_384, 256, 64), ("bf16", "dots", 60_000, 1024, 256, 0), ("bf16", "dots", 60_000, 1024, 600, 32),
     ("i8", "angular", 2048, 131_072, 768, 129), ("i8", "angular", 2048, 163_840, 768, 160), ("i8", "dots", 1024, 1_048_576, 768, 256)])
 def test_strips_out_of_step(dtype, metric, m, n, k, tiles):
     assert resident_of(dtype, metric, m, n, k)[2] == tiles
