@@ -3347,10 +3347,10 @@ hipError_t launch_typed(GemmArgs &g, hipStream_t stream, TriangleScratch const *
         return best;
     };
     // A in registers (see dots_resident_kernel) wherever there is such a kernel, C is most of the traffic and a strip is long enough for
-    // what its start costs. Against the choice without it, rounds of three sets of operands and results, at 13,000 random shapes of all types
-    // that it takes, 65 to 300,000 rows, C of 64 MiB to 2.4 GiB, the time is in the mean 0.80 (dots), 0.80 (euclidean) and 0.79 (angular), and more by 3 per
-    // cent at 26, 29 and 36 in 1000, by 10 per cent at 6. Of the slower angular ones a quarter are floats of 4 and 6 stages on lines with images of 64 MiB
-    // and more and 257 to 2048 rows (0.93 in the mean of 96). At 4400 more shapes, where the lines lie: C under 64 MiB 0.98 to 1.05, strips
+    // what its start costs. Against the choice without it, rounds of three sets of operands and results, at 14,000 random shapes of all types
+    // that it takes, 65 to 300,000 rows, C of 64 MiB to 2.4 GiB, the time is 0.81 in the mean (dots, euclidean and angular alike), and more by 3 per
+    // cent at 35, 38 and 61 in 1000, by 10 per cent at 8 (on another machine 26, 29, 36 and 6). Of the slower angular ones a fifth are floats of 4 and 6 stages on
+    // lines with images of 64 MiB and more and 257 to 2048 rows (0.96 in the mean of 109). At 4400 more shapes, where the lines lie: C under 64 MiB 0.98 to 1.05, strips
     // of fewer than 12 tiles 0.98 to 1.1 (of 12 to 15 up to 1.16), up to 64 rows 1.0. The angular finaliser is too much for few wavefronts (f16
     // 69 x 2,664,123 x 602 1.55, u4 318 x 137,089 x 1072 1.29).
     // Two blocks of rows, which ask half as often for the image, where that does not stay in the last-level cache beside C, and of more
